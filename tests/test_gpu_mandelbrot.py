@@ -50,3 +50,22 @@ def test_config3_full_grid(hip, oracle):
     # and conjugate symmetry: row r has ci = -1.5 + r*d, and rows r and n - r
     # carry opposite ci exactly (both are k*d from the centre)
     assert np.array_equal(C[1:n // 2], C[n - 1:n // 2:-1])
+
+
+# Windows whose orbits settle on cycles of period 1, 2, 3 and many, around the
+# iteration counts at which the compared state is taken (16, 24, 36, ...), with
+# max_iter on both sides of a block of 8; and windows that hold NaN and infinity.
+@pytest.mark.parametrize("it", [0, 1, 7, 8, 15, 16, 17, 24, 31, 41, 1000, 3001])
+@pytest.mark.parametrize("x0,y0,span", [(-0.3, -0.2, 0.4), (-1.1, -0.1, 0.2), (-0.16, 0.70, 0.1),
+                                        (-0.9, -0.05, 0.3), (-1.41, -0.01, 0.02), (-1e20, 0.0, 2e20)])
+def test_cycling_orbits_bit_exact(hip, oracle, x0, y0, span, it):
+    w, h = 67, 43
+    d = np.float32(span / w)
+    got = hip.escape_counts(w, h, x0, y0, d, d, it).numpy()
+    assert np.array_equal(got, oracle.mandelbrot(w, h, x0, y0, d, d, it, threads=8))
+
+
+def test_nan_and_infinite_coordinates(hip, oracle):
+    for x0, y0 in ((np.nan, 0.0), (0.0, np.nan), (np.inf, 0.0), (0.0, -np.inf)):
+        got = hip.escape_counts(9, 5, x0, y0, 0.0, 0.0, 100).numpy()
+        assert np.array_equal(got, oracle.mandelbrot(9, 5, x0, y0, 0.0, 0.0, 100)), (x0, y0)
