@@ -6,17 +6,23 @@
 // broadcast form out[i][j] = a[i][j] + b[j]; its reverse rule is db[j] = sum_i g[i][j],
 // the cotangent summed over the broadcast dimension.
 //
-// Both are HBM-bound.  Threads own one 16-byte column chunk and walk a group of rows,
-// so every wave reads and writes whole 1 KiB row segments; the bias chunk (or the
-// column accumulator) stays in registers.  The column sums add each row group in
-// ascending row order, then the group partials in ascending group order: a fixed
-// order, so results are deterministic for a given shape.
+// Both are HBM-bound.  Threads own one 16-byte column chunk (or one element, where
+// rows are not whole chunks) and walk a group of rows; the bias chunk (or the column
+// accumulator) stays in registers.  The column sums add in an order that the shape
+// alone fixes, so results are deterministic for a given shape.
+#include <cmath>
+
 #include "common.hpp"
+#include "last_block.hpp"
 
 namespace {
 
 constexpr int kThreads = 256;
 constexpr int kRowUnroll = 4;
+
+// Past the 256 MiB MALL a matrix read once streams with non-temporal loads; a
+// smaller one is often still there from the kernel that wrote it.
+constexpr int64_t kStreamBytes = 256LL << 20;
 
 // A 16-byte column chunk: 4 floats or 2 doubles.
 template <class T>
@@ -54,17 +60,6 @@ Tiling tiling_rows(int64_t rows, int64_t cols, int64_t rows_per_group, int per_c
 // one-shot map) keep the most bytes in flight: 8 rows per block measured
 // 6.6 TB/s at 65536 x 4096 against 4.8 TB/s for 128.
 Tiling tiling_bias(int64_t rows, int64_t cols, int per_chunk) { return tiling_rows(rows, cols, 8, per_chunk); }
-// The column sums write one partial row per group, which the second stage
-// reads back; about four blocks per CU in the first stage measured best
-// (6.75 TB/s at 65536 x 4096, 256 groups).
-Tiling tiling_sum(int64_t rows, int64_t cols, int per_chunk) {
-    const int64_t nseg = (cols / per_chunk + kThreads - 1) / kThreads;
-    int64_t groups = 4LL * ch::num_cus() / nseg;
-    if (groups < 1) groups = 1;
-    if (groups > rows) groups = rows;
-    return tiling_rows(rows, cols, (rows + groups - 1) / groups, per_chunk);
-}
-
 template <class T>
 __global__ __launch_bounds__(kThreads) void add_row_bias_kernel(const T* __restrict__ a, const T* __restrict__ bias,
                                                                 T* __restrict__ out, int64_t rows, int64_t cols,
@@ -87,87 +82,122 @@ __global__ __launch_bounds__(kThreads) void add_row_bias_kernel(const T* __restr
     for (; r < r1; ++r) stnt(out + r * cols + c, ldnt(a + r * cols + c) + b);
 }
 
-template <class T>
-__global__ __launch_bounds__(kThreads) void sum_rows_stage1(const T* __restrict__ g, T* __restrict__ part,
-                                                            int64_t rows, int64_t cols, int64_t nseg, int64_t rpg) {
-    typedef typename Chunk<T>::type V;
-    const int64_t seg = blockIdx.x % nseg, group = blockIdx.x / nseg;
-    const int64_t c = (seg * kThreads + threadIdx.x) * Chunk<T>::kN;
-    if (c >= cols) return;
-    const int64_t r0 = group * rpg;
-    const int64_t r1 = r0 + rpg < rows ? r0 + rpg : rows;
-    V acc = ldnt(g + r0 * cols + c);
-    int64_t r = r0 + 1;
-    for (; r + kRowUnroll <= r1; r += kRowUnroll) {
-        V v[kRowUnroll];
-#pragma unroll
-        for (int u = 0; u < kRowUnroll; ++u) v[u] = ldnt(g + (r + u) * cols + c);
-#pragma unroll
-        for (int u = 0; u < kRowUnroll; ++u) acc = acc + v[u];
-    }
-    for (; r < r1; ++r) acc = acc + ldnt(g + r * cols + c);
-    *reinterpret_cast<V*>(part + group * cols + c) = acc;
+// Column sums, out[j] = sum_i g[i][j], in one launch for any width.
+//
+// A row is `units` loads of one unit: a 16-byte chunk, or one element where a row
+// is not whole chunks or g is not aligned.  A workgroup takes `width` neighbouring
+// units of a group of rows; its threads are `lanes` = 256 / width rows deep, so a
+// narrow matrix (the 10 columns of a classifier's bias) still reads whole lines
+// with nearly every thread.  Thread (lane, unit) adds the group's rows lane,
+// lane + lanes, ... in order, the lanes meet in a fixed tree in LDS, and the
+// workgroup that arrives last at its segment's counter folds the groups the same
+// way.  One group writes its result straight out.
+struct ColSums {
+    int64_t units, nseg, groups, rows_per_group;
+    int width, lanes;
+};
+constexpr int kColCounters = 2048;
+static __device__ uint32_t g_col_counters[kColCounters];  // one per segment, 0 between launches
+
+// Segments of at most 64 chunks (a wave per 1 KiB row piece) or 128 elements, and
+// sqrt(rows) / 4 groups: the last workgroup's serial fold grows with the groups, a
+// workgroup's serial rows with their inverse.  Measured (us, f32) at sqrt(rows) times
+// 0.15 / 0.25 / 0.5 / 1: 20000 x 1000 20.6 / 19.5 / 23.8 / 24.1, 65536 x 4096 175 /
+// 167 / 195 / 188, 4096 x 256 7.5 / 7.0 / 7.0 / 7.7, 65536 x 10 6.0 / 6.1 / 6.7 / 7.6;
+// segments of 128 chunks 25 us at 20000 x 1000, of 64 or 256 elements 27 and 31 at
+// 20000 x 1001 against 22.  Before, with a launch for the fold: 24.5, 166, 12.2, and
+// with one thread per column where rows are not whole chunks: 7154 us at 65536 x 10,
+// 4724 at 20000 x 1001.
+// From kColCounters segments (2 MiB of a row) the segments alone fill the chip and
+// one group takes all rows.
+ColSums col_sums_plan(int64_t rows, int64_t units, bool chunks) {
+    ColSums p{};
+    p.units = units;
+    const int64_t widest = chunks ? 64 : 128;
+    p.nseg = (units + widest - 1) / widest;
+    p.width = (int)((units + p.nseg - 1) / p.nseg);
+    p.nseg = (units + p.width - 1) / p.width;
+    p.lanes = kThreads / p.width;
+    int64_t groups = p.nseg >= kColCounters ? 1 : (int64_t)(std::sqrt((double)rows) / 4.0);
+    const int64_t most = rows / ((int64_t)p.lanes * 4);  // at least four rows a thread
+    if (groups > most) groups = most;
+    if (groups < 1) groups = 1;
+    p.rows_per_group = (rows + groups - 1) / groups;
+    p.groups = (rows + p.rows_per_group - 1) / p.rows_per_group;
+    return p;
 }
 
-// out[j] = the sum of part[0..groups)[j].  Eight threads share a column:
-// thread s left-folds groups [s*G/8, (s+1)*G/8) with eight loads in flight,
-// then thread 0 folds the eight partials in order s = 0..7, so the result is
-// deterministic.  A block covers 32 columns; the 32 threads of a half-wave
-// that share s read 128 contiguous bytes of a partial row.  At 65536 x 4096
-// this stage takes 5.4 us (sixteen threads per column: the same); one thread
-// per column, folding all 256 groups itself, left 16 blocks and took 12.4 us.
-constexpr int kGroupUnroll = 8;
-constexpr int kStage2Split = 8, kStage2Cols = kThreads / kStage2Split;
-template <class T>
-__global__ __launch_bounds__(kThreads) void sum_rows_stage2(const T* __restrict__ part, T* __restrict__ out,
-                                                            int64_t groups, int64_t cols) {
-    __shared__ T red[kStage2Split][kStage2Cols];
-    const int jj = threadIdx.x % kStage2Cols, s = threadIdx.x / kStage2Cols;
-    const int64_t j = (int64_t)blockIdx.x * kStage2Cols + jj;
-    const int64_t q0 = groups * s / kStage2Split, q1 = groups * (s + 1) / kStage2Split;
-    T acc = T(0);
-    if (j < cols && q0 < q1) {
-        acc = part[q0 * cols + j];
-        int64_t q = q0 + 1;
-        for (; q + kGroupUnroll <= q1; q += kGroupUnroll) {
-            T v[kGroupUnroll];
+// The sum of rows first, first + step, ... < n at p (row pitch `pitch` units), in
+// that order, 8 loads in flight, or 16 of the uncached ones; first < n.
+enum class Read { kCached, kStream, kFetch };
+template <class U, Read RD>
+__device__ __forceinline__ U add_rows(const U* p, int64_t first, int64_t n, int step, int64_t pitch) {
+    auto ld = [&](int64_t r) {
+        if constexpr (RD == Read::kStream) return __builtin_nontemporal_load(p + r * pitch);
+        else if constexpr (RD == Read::kFetch) return ch::fetch(p + r * pitch);
+        else return p[r * pitch];
+    };
+    constexpr int kColUnroll = RD == Read::kFetch ? 16 : 8;
+    U acc = ld(first);
+    int64_t r = first + step;
+    for (; r + (int64_t)(kColUnroll - 1) * step < n; r += (int64_t)kColUnroll * step) {
+        U v[kColUnroll];
 #pragma unroll
-            for (int u = 0; u < kGroupUnroll; ++u) v[u] = part[(q + u) * cols + j];
+        for (int u = 0; u < kColUnroll; ++u) v[u] = ld(r + (int64_t)u * step);
 #pragma unroll
-            for (int u = 0; u < kGroupUnroll; ++u) acc = acc + v[u];
-        }
-        for (; q < q1; ++q) acc = acc + part[q * cols + j];
+        for (int u = 0; u < kColUnroll; ++u) acc = acc + v[u];
     }
-    red[s][jj] = acc;
+    for (; r < n; r += step) acc = acc + ld(r);
+    return acc;
+}
+
+// Folds the `nv` lanes' values of each unit into lane 0's, in a fixed tree.
+template <class U>
+__device__ __forceinline__ U fold_lanes(U acc, int lane, int nv, int width, U* red) {
+    if (nv <= 1) return acc;
     __syncthreads();
-    if (s == 0 && j < cols) {
-        // fold the non-empty chunks in order (a chunk is empty only when
-        // groups < 8; the last one never is)
-        int t = 0;
-        while (groups * (t + 1) / kStage2Split == groups * t / kStage2Split) ++t;
-        T r = red[t][jj];
-        for (++t; t < kStage2Split; ++t)
-            if (groups * (t + 1) / kStage2Split > groups * t / kStage2Split) r = r + red[t][jj];
-        out[j] = r;
+    red[threadIdx.x] = acc;
+    int half = 1;
+    while (half * 2 < nv) half *= 2;
+    for (; half >= 1; half /= 2) {
+        __syncthreads();
+        if (lane < half && lane + half < nv) red[threadIdx.x] = red[threadIdx.x] + red[threadIdx.x + half * width];
     }
+    return red[threadIdx.x];
 }
 
-// Scalar forms for widths that are not a multiple of 4 or unaligned pointers.
+// U: a unit's type (a chunk of T, or T).
+template <class U, Read RD>
+__global__ __launch_bounds__(kThreads) void col_sums_kernel(const U* __restrict__ g, U* part,
+                                                            U* __restrict__ out, int64_t rows, ColSums p) {
+    __shared__ U red[kThreads];
+    const int64_t seg = blockIdx.x % p.nseg, group = blockIdx.x / p.nseg;
+    const int lane = threadIdx.x / p.width;
+    const int64_t c = seg * p.width + threadIdx.x % p.width;
+    const bool mine = lane < p.lanes && c < p.units;
+    const int64_t r0 = group * p.rows_per_group;
+    const int64_t n = min(p.rows_per_group, rows - r0);
+    U acc = U(0);
+    if (mine && lane < n) acc = add_rows<U, RD>(g + r0 * p.units + c, lane, n, p.lanes, p.units);
+    acc = fold_lanes(acc, lane, (int)min((int64_t)p.lanes, n), p.width, red);
+    if (p.groups == 1) {
+        if (mine && lane == 0) out[c] = acc;
+        return;
+    }
+    if (mine && lane == 0) ch::publish(part + group * p.units + c, acc);
+    if (!ch::last_block(&g_col_counters[seg], (uint32_t)p.groups)) return;
+    if (mine && lane < p.groups) acc = add_rows<U, Read::kFetch>(part + c, lane, p.groups, p.lanes, p.units);
+    acc = fold_lanes(acc, lane, (int)min((int64_t)p.lanes, p.groups), p.width, red);
+    if (mine && lane == 0) out[c] = acc;
+}
+
+// Scalar form for widths that are not a multiple of 4 or unaligned pointers.
 template <class T>
 __global__ void add_row_bias_scalar(const T* a, const T* bias, T* out, int64_t rows, int64_t cols) {
     const int64_t n = rows * cols;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
         out[i] = a[i] + bias[i % cols];
 }
-template <class T>
-__global__ void sum_rows_scalar(const T* g, T* out, int64_t rows, int64_t cols) {
-    for (int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; j < cols; j += (int64_t)gridDim.x * blockDim.x) {
-        T acc = g[j];
-        for (int64_t r = 1; r < rows; ++r) acc = acc + g[r * cols + j];
-        out[j] = acc;
-    }
-}
-
 bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 unsigned blocks_for(int64_t n) {
@@ -201,6 +231,24 @@ int32_t run_add_row_bias(const char* fn, const T* a, int64_t alen, const T* bias
     return CLEAVE_HIP_OK;
 }
 
+template <class T, class U>
+int32_t launch_col_sums(const char* fn, const T* g, T* out, int64_t rows, int64_t units) {
+    const ColSums p = col_sums_plan(rows, units, sizeof(U) > sizeof(T));
+    U* part = nullptr;
+    if (p.groups > 1) {
+        part = (U*)ch::scratch(5, sizeof(U) * (size_t)(p.groups * units));
+        if (!part)
+            return ch::fail(CLEAVE_HIP_ERR_OOM, "%s: scratch of %lld elements", fn, (long long)(p.groups * units));
+    }
+    const unsigned grid = (unsigned)(p.nseg * p.groups);
+    if (rows * units * (int64_t)sizeof(U) > kStreamBytes)
+        col_sums_kernel<U, Read::kStream><<<grid, kThreads, 0, ch::stream()>>>((const U*)g, part, (U*)out, rows, p);
+    else
+        col_sums_kernel<U, Read::kCached><<<grid, kThreads, 0, ch::stream()>>>((const U*)g, part, (U*)out, rows, p);
+    CH_LAUNCHED(fn);
+    return CLEAVE_HIP_OK;
+}
+
 template <class T>
 int32_t run_sum_rows(const char* fn, const T* g, int64_t glen, T* out, int64_t outlen, int32_t rows, int32_t cols) {
     constexpr int V = Chunk<T>::kN;
@@ -213,20 +261,9 @@ int32_t run_sum_rows(const char* fn, const T* g, int64_t glen, T* out, int64_t o
     CH_INIT_OR_RETURN();
     CH_DEVICE(fn, g, glen * sizeof(T));
     CH_DEVICE(fn, out, outlen * sizeof(T));
-    if (cols % V == 0 && aligned16(g)) {
-        const Tiling t = tiling_sum(rows, cols, V);
-        T* part = (T*)ch::scratch(5, sizeof(T) * (size_t)(t.groups * cols));
-        if (!part) return ch::fail(CLEAVE_HIP_ERR_OOM, "%s: scratch of %lld elements", fn, (long long)(t.groups * cols));
-        sum_rows_stage1<T><<<(unsigned)(t.nseg * t.groups), kThreads, 0, ch::stream()>>>(g, part, rows, cols, t.nseg,
-                                                                                          t.rows_per_group);
-        CH_LAUNCHED(fn);
-        sum_rows_stage2<T><<<(unsigned)((cols + kStage2Cols - 1) / kStage2Cols), kThreads, 0, ch::stream()>>>(
-            part, out, t.groups, cols);
-    } else {
-        sum_rows_scalar<T><<<blocks_for(cols), kThreads, 0, ch::stream()>>>(g, out, rows, cols);
-    }
-    CH_LAUNCHED(fn);
-    return CLEAVE_HIP_OK;
+    if (cols % V == 0 && aligned16(g) && aligned16(out))
+        return launch_col_sums<T, typename Chunk<T>::type>(fn, g, out, rows, cols / V);
+    return launch_col_sums<T, T>(fn, g, out, rows, cols);
 }
 
 // ---- Broadcasting maps and their reverse rule ----------------------------

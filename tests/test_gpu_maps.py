@@ -174,3 +174,33 @@ def test_sum_rows_is_deterministic_and_at_full_size(hip):
     x = hip.fill_normal(hip.empty((8192, 1024)), seed=6)
     a, b = hip.sum_rows(x).numpy(), hip.sum_rows(x).numpy()
     assert np.array_equal(a, b)
+
+
+# Both units (16-byte chunks; single elements where the width or the pointer asks for
+# them), widths around a segment, rows around a lane count and the first second group.
+@pytest.mark.parametrize("dtype", ["f32", "f64"])
+@pytest.mark.parametrize("rows", [1, 2, 7, 63, 64, 65, 1023, 4099])
+@pytest.mark.parametrize("cols", [1, 2, 3, 10, 64, 127, 128, 129, 255, 256, 257, 260, 1000])
+def test_sum_rows_edges(hip, rows, cols, dtype):
+    g = np.random.default_rng(rows * 1009 + cols)
+    np_t = np.float32 if dtype == "f32" else np.float64
+    G = g.integers(-8, 9, (rows, cols)).astype(np_t)  # whole numbers: every order gives the exact sum
+    assert np.array_equal(hip.sum_rows(hip.from_numpy(G)).numpy(), G.sum(axis=0))
+    # a view one element in: rows are read element by element
+    flat = hip.from_numpy(np.concatenate([np.zeros(1, np_t), G.reshape(-1)]))
+    assert np.array_equal(hip.sum_rows(flat.sub(1, (rows, cols))).numpy(), G.sum(axis=0))
+
+
+@pytest.mark.parametrize("cols", [2048 * 128, 2048 * 256])  # one group takes all rows: no fold
+def test_sum_rows_wide(hip, cols):
+    G = np.random.default_rng(cols).integers(-8, 9, (300, cols)).astype(np.float32)
+    assert np.array_equal(hip.sum_rows(hip.from_numpy(G)).numpy(), G.sum(axis=0))
+
+
+def test_sum_rows_keeps_nan_inf_and_negative_zero(hip, oracle):
+    G = np.ones((4096, 10), np.float32)
+    G[17, 1], G[4095, 2], G[0, 3], G[5, 4], G[6, 4] = np.nan, np.inf, -np.inf, np.inf, -np.inf
+    G[:, 5] = -0.0
+    got, want = hip.sum_rows(hip.from_numpy(G)).numpy(), oracle.sum_rows(G)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[~np.isnan(got)], want[~np.isnan(want)]) and np.signbit(got[5])
