@@ -9,25 +9,34 @@
 // gfx950: unlike the f32 16x16x4 form, whose lane holds four consecutive
 // rows, the f64 form interleaves them).  On MI355X one such
 // instruction keeps a SIMD's matrix core busy 64 cycles (FP64 matrix peak
-// 78.6 TFLOP/s = 128 FLOP per CU-clock), so the kernel is matrix-core bound
-// with little memory traffic per instruction: it needs enough independent
-// accumulators per wave to issue back to back, not an elaborate copy
-// pipeline.
+// 78.6 TFLOP/s = 128 FLOP per CU-clock).
 //
-// Tiles: a 256-thread workgroup computes a 128 x 128 block of C as 2 x 2 waves
-// of 64 x 64 (4 x 4 MFMA tiles, 64 accumulator doubles per lane).  K advances
-// 16 at a time through two LDS stages (2 x 32 KiB): the next tile's global
-// loads are issued before the current tile's MFMAs and written to the other
-// stage after them, one barrier per tile.  Both operands sit in LDS k-major
-// ([k][m] and [k][n], rows padded to 144 doubles so the two 16-lane row
-// groups of a half-wave read opposite bank halves, columns swizzled per k-row
-// pair, lds_col).  Global loads are 16-byte
-// vectors along whichever index is contiguous in memory when that extent is
-// even, single doubles otherwise; out-of-range elements load as zero, so any
-// M, N, K (K = 0 included: C = 0, the zero-filled accumulator of
-// matrix.cleave:59) takes the same path.
+// With so much time per operand pair there is no LDS staging: a wave computes
+// a (16 FM) x (16 FN) tile of C from register fragments that it loads from the
+// caches, 16 of K at a time (FM FN x 256 cycles of MFMA a step), and the other
+// waves of its SIMD cover the loads.  The register-staged LDS tiles of 128 x
+// 128 that this replaced were slower at every size: 4096^3 A.B 2206 -> 2124 us,
+// A.B^T 2428 -> 2178, 4095^3 A.B^T (rows not 16-byte aligned) 3412 -> 1885,
+// and with few tiles 1000^3 167 -> 43, 256^3 45 -> 5, 64^2 x 10000 1586 -> 14,
+// 8192 x 10 x 4096 660 -> 46.  The same LDS scheme on 64 x 64 tiles took 69-73
+// us at 1000^3.
+//
+// WK = 4: the workgroup's four waves take quarters of K, added in LDS in wave
+// order.  WK = 1: they take a 2 x 2 block of tiles, sharing their fragments'
+// lines in L1.  Past that K is cut into `slices` workgroups per tile; each
+// publishes its partial tile and the last to arrive adds them in slice order
+// (last_block.hpp).  The order of every sum depends on the shape alone.
+//
+// k order: over an 8-deep block, lane group h = lane / 16 takes k = 2h + s at
+// step s for A and B alike, so a k-contiguous operand is one 16-byte load per
+// lane, fragment and block (V2; two 8-byte loads where its rows or base are
+// not 16-byte aligned).  Rows and columns past the product are read from its
+// last row or column and feed only entries that are not stored; k past K
+// enters as zero on both sides.  Any M, N, K takes the same path (K = 0
+// included: C = 0, the zero-filled accumulator of matrix.cleave:59).
 #include "common.hpp"
 #include "gemm_common.hpp"
+#include "last_block.hpp"
 
 namespace {
 
@@ -35,174 +44,328 @@ typedef double d4 __attribute__((ext_vector_type(4)));
 typedef double d2 __attribute__((ext_vector_type(2)));
 
 constexpr int kThreads = 256;
-constexpr int BM = 128, BN = 128, BK = 16;
-constexpr int kPitch = 144;  // LDS row pitch in doubles: 1152 B, 128 B mod 256
+constexpr int kStep = 16;        // K per step of a wave
+constexpr int kCounters = 4096;  // tiles that may be cut along K
+static __device__ uint32_t g_counters[kCounters];  // 0 between launches
 
-// LDS column of output index r in k-row k.  A k-contiguous operand is stored
-// transposed: the 64 lanes of one store instruction cover 8 k-rows (8 lanes
-// each) at 8 columns, and with a 144-double pitch every even k-row starts on
-// the same bank, an 8-way conflict.  XOR-ing the column with 8 * ((k / 2) % 8)
-// spreads those lanes over all 32 double slots of a 256-byte bank cycle (2
-// passes for 512 bytes).  The XOR only moves 8-double groups, so the 16 lanes
-// of an MFMA operand read still see one aligned 128-byte block per k-row, and
-// k-rows 2j and 2j + 1 (one half-wave) share the XOR and stay 128 bytes apart
-// modulo 256.  A 16-byte pair (r, r + 1), r even, stays adjacent.
-__device__ __forceinline__ int lds_col(int k, int r) { return r ^ (((k >> 1) & 7) << 3); }
+// One operand of a wave: F fragments of 16 rows (of A, or columns of B) by 16
+// doubles of K.  KC: k-contiguous in memory.
+template <int F, bool KC, bool V2>
+struct Frags {
+    const double* p[F];
+    int64_t ld;
 
-// Global -> register staging of one operand tile (R rows of the output
-// dimension by BK along k).  KC: the operand is k-contiguous in memory (A
-// stored M x K, B stored N x K); otherwise it is m/n-contiguous (A stored
-// K x M, B stored K x N).  V doubles per load.
-template <bool KC, int V>
-struct TileLoad {
-    static constexpr int kPer = (BM * BK) / (kThreads * V);  // loads per thread
-    double v[kPer * V];
-
-    // rows: extent of the output dimension (M or N); ld: row pitch in memory.
-    __device__ __forceinline__ void load(const double* __restrict__ p, int64_t ld, int r0, int rows, int k0, int K) {
+    // r0: the wave's first row; rows: the operand's.
+    __device__ __forceinline__ void init(const double* base, int64_t pitch, int r0, int rows, int lane) {
+        ld = pitch;
+        const int h = lane >> 4;
 #pragma unroll
-        for (int i = 0; i < kPer; ++i) {
-            const int c = threadIdx.x + kThreads * i;
-            int r, k;
-            if constexpr (KC) {
-                r = c / (BK / V);
-                k = (c % (BK / V)) * V;
-            } else {
-                k = c / (BM / V);
-                r = (c % (BM / V)) * V;
-            }
-            const bool ok = (r0 + r < rows) && (k0 + k < K);
-            const int64_t off = KC ? (int64_t)(r0 + r) * ld + (k0 + k) : (int64_t)(k0 + k) * ld + (r0 + r);
-            if constexpr (V == 2) {
-                const d2 x = ok ? *reinterpret_cast<const d2*>(p + off) : d2{0.0, 0.0};
-                v[2 * i] = x[0];
-                v[2 * i + 1] = x[1];
-            } else {
-                v[i] = ok ? p[off] : 0.0;
+        for (int f = 0; f < F; ++f) {
+            const int r = min(r0 + 16 * f + (lane & 15), rows - 1);
+            p[f] = base + (KC ? (int64_t)r * pitch + 2 * h : (int64_t)(2 * h) * pitch + r);
+        }
+    }
+    __device__ __forceinline__ void load(int64_t k, double (&v)[F][4]) const {
+#pragma unroll
+        for (int f = 0; f < F; ++f) {
+            const double* q = p[f] + (KC ? k : k * ld);
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                if constexpr (KC && V2) {
+                    const d2 x = *reinterpret_cast<const d2*>(q + 8 * b);
+                    v[f][2 * b] = x[0];
+                    v[f][2 * b + 1] = x[1];
+                } else {
+#pragma unroll
+                    for (int s = 0; s < 2; ++s) v[f][2 * b + s] = KC ? q[8 * b + s] : q[(int64_t)(8 * b + s) * ld];
+                }
             }
         }
     }
-
-    // Into the k-major LDS stage s[BK][kPitch].
-    __device__ __forceinline__ void store(double* s) const {
+    // The step at k of a range that ends at k1 < k + 16.
+    __device__ __forceinline__ void load_tail(int64_t k, int64_t k1, int lane, double (&v)[F][4]) const {
+        const int h = lane >> 4;
 #pragma unroll
-        for (int i = 0; i < kPer; ++i) {
-            const int c = threadIdx.x + kThreads * i;
-            if constexpr (KC) {
-                const int r = c / (BK / V), k = (c % (BK / V)) * V;
+        for (int f = 0; f < F; ++f) {
+            const double* q = p[f] + (KC ? k : k * ld);
 #pragma unroll
-                for (int e = 0; e < V; ++e) s[(k + e) * kPitch + lds_col(k + e, r)] = v[V * i + e];
-            } else {
-                const int k = c / (BM / V), r = (c % (BM / V)) * V;
-                if constexpr (V == 2)
-                    *reinterpret_cast<d2*>(s + k * kPitch + lds_col(k, r)) = d2{v[2 * i], v[2 * i + 1]};
-                else
-                    s[k * kPitch + lds_col(k, r)] = v[i];
-            }
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    const bool in = k + 8 * b + 2 * h + s < k1;
+                    v[f][2 * b + s] = in ? (KC ? q[8 * b + s] : q[(int64_t)(8 * b + s) * ld]) : 0.0;
+                }
         }
     }
 };
 
-// C[b] = op(A[b]) op(B[b]) for b < batch; a 1-D grid of tiles_m * tiles_n *
-// batch workgroups in the XCD-aware order of block_coords.
-template <bool TA, bool TB, int VA, int VB>
-__global__ __launch_bounds__(kThreads) void gemm_f64_kernel(const double* __restrict__ A, const double* __restrict__ B,
-                                                           double* __restrict__ C, int M, int N, int K, int batch,
-                                                           int64_t sa, int64_t sb, int64_t sc) {
-    __shared__ double As[2][BK * kPitch];
-    __shared__ double Bs[2][BK * kPitch];
+// `part`: tiles x slices partial tiles, unused with slices == 1.  A 1-D grid of
+// tiles_m * tiles_n * batch * slices workgroups.
+template <bool KCA, bool KCB, bool V2A, bool V2B, int FM, int FN, int WK, int PF>
+__global__ __launch_bounds__(kThreads) void gemm_f64_kernel(
+    const double* __restrict__ A, const double* __restrict__ B, double* __restrict__ C, int M, int N, int K,
+    int64_t lda, int64_t ldb, int64_t sa, int64_t sb, int64_t sc, int tiles_m, int tiles_n, int batch, int slices,
+    int64_t kslice, double* part) {
+    static_assert(WK == 1 || WK == 4, "waves along K");
+    constexpr int NF = FM * FN;
+    __shared__ double red[WK > 1 ? (WK - 1) * NF * 4 * 64 : 1];
 
-    const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-    int b, tm, tn;
-    ch::block_coords(blockIdx.x, tiles_m, tiles_n, batch, b, tm, tn);
-    A += (int64_t)b * sa;
-    B += (int64_t)b * sb;
-    C += (int64_t)b * sc;
-    const int m0 = tm * BM, n0 = tn * BN;
-    // A is k-contiguous unless stored K x M (trans_a); B is k-contiguous when stored N x K (trans_b).
-    const int64_t lda = TA ? M : K, ldb = TB ? K : N;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int b, tm, tn;  // b: batch entry and slice
+    ch::block_coords(blockIdx.x, tiles_m, tiles_n, batch * slices, b, tm, tn);
+    const int entry = b / slices, z = b - entry * slices;
+    A += (int64_t)entry * sa;
+    B += (int64_t)entry * sb;
+    C += (int64_t)entry * sc;
+    const int m0 = WK == 1 ? (tm * 2 + (wave >> 1)) * 16 * FM : tm * 16 * FM;
+    const int n0 = WK == 1 ? (tn * 2 + (wave & 1)) * 16 * FN : tn * 16 * FN;
 
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
-    const int lr = lane & 15, lk = lane >> 4;
-
-    d4 acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
-
-    TileLoad<!TA, VA> la;
-    TileLoad<TB, VB> lb;
-    const int tiles_k = (K + BK - 1) / BK;
-    if (tiles_k > 0) {
-        la.load(A, lda, m0, M, 0, K);
-        lb.load(B, ldb, n0, N, 0, K);
-        la.store(As[0]);
-        lb.store(Bs[0]);
+    int64_t k0 = z * kslice, k1 = min((int64_t)K, k0 + kslice);
+    if constexpr (WK > 1) {
+        const int64_t steps = (k1 - k0 + kStep - 1) / kStep, each = (steps + WK - 1) / WK * kStep;
+        k0 += wave * each;
+        k1 = min(k1, k0 + each);
     }
-    __syncthreads();
-    for (int t = 0; t < tiles_k; ++t) {
-        const int s = t & 1;
-        const bool more = t + 1 < tiles_k;
-        if (more) {
-            la.load(A, lda, m0, M, (t + 1) * BK, K);
-            lb.load(B, ldb, n0, N, (t + 1) * BK, K);
+
+    d4 acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
+    auto mfma = [&](const double (&a)[FM][4], const double (&bb)[FN][4]) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int j = 0; j < FN; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i][t], bb[j][t], acc[i][j], 0, 0, 0);
+    };
+
+    Frags<FM, KCA, V2A> fa;
+    Frags<FN, KCB, V2B> fb;
+    if (k0 < k1) {
+        fa.init(A, lda, m0, M, lane);
+        fb.init(B, ldb, n0, N, lane);
+        const int whole = (int)((k1 - k0) / kStep);
+        double a[PF][FM][4], bb[PF][FN][4];
+#pragma unroll
+        for (int u = 0; u < PF; ++u)
+            if (u < whole) {
+                fa.load(k0 + u * kStep, a[u]);
+                fb.load(k0 + u * kStep, bb[u]);
+            }
+        for (int t = 0; t < whole; t += PF) {
+#pragma unroll
+            for (int u = 0; u < PF; ++u)
+                if (t + u < whole) {
+                    mfma(a[u], bb[u]);
+                    if (t + u + PF < whole) {
+                        fa.load(k0 + (int64_t)(t + u + PF) * kStep, a[u]);
+                        fb.load(k0 + (int64_t)(t + u + PF) * kStep, bb[u]);
+                    }
+                }
         }
-        const double* as = As[s];
-        const double* bs = Bs[s];
-#pragma unroll
-        for (int ks = 0; ks < BK; ks += 4) {
-            double a[4], bv[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = as[(ks + lk) * kPitch + lds_col(ks + lk, wm + 16 * i + lr)];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) bv[j] = bs[(ks + lk) * kPitch + lds_col(ks + lk, wn + 16 * j + lr)];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], bv[j], acc[i][j], 0, 0, 0);
+        k0 += (int64_t)whole * kStep;
+        if (k0 < k1) {
+            fa.load_tail(k0, k1, lane, a[0]);
+            fb.load_tail(k0, k1, lane, bb[0]);
+            mfma(a[0], bb[0]);
         }
-        if (more) {
-            la.store(As[s ^ 1]);
-            lb.store(Bs[s ^ 1]);
+    }
+
+    if constexpr (WK > 1) {
+        if (wave > 0) {
+#pragma unroll
+            for (int f = 0; f < NF; ++f)
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    red[(((wave - 1) * NF + f) * 4 + v) * 64 + lane] = acc[f / FN][f % FN][v];
         }
         __syncthreads();
+        if (wave == 0) {
+#pragma unroll
+            for (int w = 0; w < WK - 1; ++w)
+#pragma unroll
+                for (int f = 0; f < NF; ++f)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        acc[f / FN][f % FN][v] += red[((w * NF + f) * 4 + v) * 64 + lane];
+        }
     }
 
-    // acc[i][j][v] is C[m0 + wm + 16 i + lane / 16 + 4 v][n0 + wn + 16 j + lane % 16].
+    // acc[i][j][v] is C[m0 + 16 i + lane / 16 + 4 v][n0 + 16 j + lane % 16].
+    auto put = [&](int f, int v, double x) {
+        const int m = m0 + 16 * (f / FN) + (lane >> 4) + 4 * v, n = n0 + 16 * (f % FN) + (lane & 15);
+        if (m < M && n < N) C[(int64_t)m * N + n] = x;
+    };
+    if (slices == 1) {
+        if (WK > 1 && wave != 0) return;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+        for (int f = 0; f < NF; ++f)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int m = m0 + wm + 16 * i + lk + 4 * v;
-            if (m >= M) continue;
+            for (int v = 0; v < 4; ++v) put(f, v, acc[f / FN][f % FN][v]);
+        return;
+    }
+    if constexpr (WK > 1) {
+        const int64_t tile = ((int64_t)entry * tiles_m + tm) * tiles_n + tn;
+        double* mine = part + tile * slices * (NF * 256);
+        if (wave == 0) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int n = n0 + wn + 16 * j + lr;
-                if (n < N) C[(int64_t)m * N + n] = acc[i][j][v];
-            }
+            for (int f = 0; f < NF; ++f)
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    ch::publish(mine + ((int64_t)z * NF + f) * 256 + v * 64 + lane, acc[f / FN][f % FN][v]);
         }
+        if (!ch::last_block(&g_counters[tile], (uint32_t)slices)) return;
+        constexpr int kFoldLoads = 4;  // slices in flight
+        for (int f = wave; f < NF; f += 4) {
+            double s[4];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) s[v] = ch::fetch(mine + (int64_t)f * 256 + v * 64 + lane);
+            for (int q0 = 1; q0 < slices; q0 += kFoldLoads) {
+                double x[kFoldLoads][4];
+#pragma unroll
+                for (int u = 0; u < kFoldLoads; ++u) {
+                    const int q = min(q0 + u, slices - 1);
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) x[u][v] = ch::fetch(mine + ((int64_t)q * NF + f) * 256 + v * 64 + lane);
+                }
+#pragma unroll
+                for (int u = 0; u < kFoldLoads; ++u)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        if (q0 + u < slices) s[v] += x[u][v];
+            }
+#pragma unroll
+            for (int v = 0; v < 4; ++v) put(f, v, s[v]);
+        }
+    }
 }
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
-template <bool TA, bool TB>
-void launch_layout(const double* a, const double* b, double* c, int M, int N, int K, int batch, int64_t sa,
-                   int64_t sb, int64_t sc, unsigned grid) {
-    // 16-byte loads need every row of the contiguous index to start 16-byte aligned.
-    const int contig_a = TA ? M : K, contig_b = TB ? K : N;
-    const bool va = contig_a % 2 == 0 && aligned16(a) && sa % 2 == 0;
-    const bool vb = contig_b % 2 == 0 && aligned16(b) && sb % 2 == 0;
-    if (va && vb)
-        gemm_f64_kernel<TA, TB, 2, 2><<<grid, kThreads, 0, ch::stream()>>>(a, b, c, M, N, K, batch, sa, sb, sc);
-    else if (va)
-        gemm_f64_kernel<TA, TB, 2, 1><<<grid, kThreads, 0, ch::stream()>>>(a, b, c, M, N, K, batch, sa, sb, sc);
-    else if (vb)
-        gemm_f64_kernel<TA, TB, 1, 2><<<grid, kThreads, 0, ch::stream()>>>(a, b, c, M, N, K, batch, sa, sb, sc);
-    else
-        gemm_f64_kernel<TA, TB, 1, 1><<<grid, kThreads, 0, ch::stream()>>>(a, b, c, M, N, K, batch, sa, sb, sc);
+// One product or batch as a kernel takes it.
+struct Args {
+    const double *a, *b;
+    double* c;
+    int M, N, K, batch;
+};
+
+int64_t tile_count(const Args& g, int tm, int tn) {
+    return (int64_t)((g.M + tm - 1) / tm) * ((g.N + tn - 1) / tn) * g.batch;
+}
+
+template <bool KCA, bool KCB, bool V2A, bool V2B, int FM, int FN, int WK, int PF>
+int32_t launch(const Args& g, int slices) {
+    constexpr int TM = 16 * FM * (WK == 1 ? 2 : 1), TN = 16 * FN * (WK == 1 ? 2 : 1);
+    const int64_t tiles = tile_count(g, TM, TN);
+    int64_t kslice = g.K;
+    double* part = nullptr;
+    if (slices > 1) {
+        kslice = (((int64_t)g.K + slices - 1) / slices + kStep - 1) / kStep * kStep;
+        slices = (int)((g.K + kslice - 1) / kslice);
+        part = (double*)ch::scratch_try(11, sizeof(double) * (size_t)(tiles * slices * FM * FN * 256));
+        if (!part) slices = 1, kslice = g.K;  // no room: K in one piece
+    }
+    gemm_f64_kernel<KCA, KCB, V2A, V2B, FM, FN, WK, PF><<<(unsigned)(tiles * slices), kThreads, 0, ch::stream()>>>(
+        g.a, g.b, g.c, g.M, g.N, g.K, KCA ? g.K : g.M, KCB ? g.K : g.N, (int64_t)g.M * g.K, (int64_t)g.K * g.N,
+        (int64_t)g.M * g.N, (g.M + TM - 1) / TM, (g.N + TN - 1) / TN, g.batch, slices, kslice, part);
+    CH_LAUNCHED("gemm_f64_kernel");
+    return CLEAVE_HIP_OK;
+}
+
+// The wave tiles, and the time of a product on each as fitted to sweeps on
+// MI355X (48 shapes and layouts from 33 x 77 x 1000 to 4096^3; the choice was
+// within 19% of the best of all measured, within 5% for 38 of them):
+//   base + max(busiest CU's MFMA time / eff, one wave's steps x (MFMA + lat)) + fold
+// A step of a wave is FM FN x 256 cycles of MFMA, 0.107 us a fragment pair.
+// lat is what a wave's load latency adds where nothing else runs on its SIMD;
+// eff_k applies where both operands are k-contiguous (A.B^T), whose 64-byte
+// row pieces use the L1 less well.  Past one slice, each partial tile is
+// written and read past the L2: about 3 TB/s for the two, and 3 us.
+struct TileCost {
+    int fm, fn, wk;
+    double base, eff, eff_k, lat;  // us, share of the MFMA rate, us a step
+};
+constexpr TileCost kTiles[] = {
+    {1, 1, 4, 3.5, 0.32, 0.27, 0.3},
+    {2, 2, 4, 4.0, 0.65, 0.53, 0.6},
+    {4, 2, 4, 6.0, 0.72, 0.63, 0.6},
+    {4, 4, 1, 9.0, 0.81, 0.81, 0.6},
+};
+constexpr int kSlices[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
+
+struct Plan {
+    int tile = 3, slices = 1;
+};
+
+Plan choose_tile(const Args& g, bool both_k) {
+    Plan best;
+    double best_us = 1e300;
+    const int cus = ch::num_cus();
+    for (int i = 0; i < 4; ++i) {
+        const TileCost& t = kTiles[i];
+        const int tm = 16 * t.fm * (t.wk == 1 ? 2 : 1), tn = 16 * t.fn * (t.wk == 1 ? 2 : 1);
+        const int64_t tiles = tile_count(g, tm, tn);
+        if (tiles > 0x7FFFFFFF) continue;  // the 128 x 128 tiles' count is checked by the caller
+        for (const int s : kSlices) {
+            // slices of at least 128, at most 16 workgroups a CU, a counter per tile
+            if (s > 1 && (t.wk == 1 || g.K / s < 128 || tiles * s > 16 * (int64_t)cus || tiles > kCounters)) break;
+            const double steps = (double)((((int64_t)g.K + s - 1) / s + kStep * t.wk - 1) / (kStep * t.wk));
+            const double mfma = 0.107 * t.fm * t.fn;
+            const double busy = (double)((tiles * s + cus - 1) / cus) * steps * mfma / (both_k ? t.eff_k : t.eff);
+            const double chain = steps * (mfma + t.lat);
+            const double us = t.base + (busy > chain ? busy : chain) +
+                              (s > 1 ? 3.0 + (double)(tiles * s) * tm * tn * 16.0 / 3e6 : 0.0);
+            if (us < best_us) best_us = us, best.tile = i, best.slices = s;
+        }
+    }
+    return best;
+}
+
+// Narrow products (M or N up to 16) stream the wide operand: 32 x 16 wave tiles
+// (FM = 2, FN = 1, or the other way round), with as many slices as give every CU
+// a workgroup while each keeps 256 of K, and on to four a CU while each keeps
+// 1024.  8192 x 1 x 16384 188 us (5.7 TB/s) with 4 slices, 246 with one; 8192 x
+// 16 x 1024 14.5 us with one, 15.5 with 2 or 4; 300 x 2 x 5000 36 with one, 9.8
+// with 8.  The 64 x 16 tiles were level or slower on all of them.
+int narrow_slices(const Args& g, int64_t tiles) {
+    const int64_t cus = ch::num_cus();
+    if (tiles > kCounters) return 1;
+    int64_t s = (cus + tiles - 1) / tiles;
+    if (s > g.K / 256) s = g.K / 256;
+    int64_t more = 4 * cus / tiles;
+    if (more > g.K / 1024) more = g.K / 1024;
+    if (s < more) s = more;
+    if (s > 64) s = 64;
+    return s < 1 ? 1 : (int)s;
+}
+
+template <bool KCA, bool KCB, bool V2A, bool V2B>
+int32_t run_shape(const Args& g) {
+    if (g.N <= 16 && tile_count(g, 32, 16) <= 0x7FFFFFFF)
+        return launch<KCA, KCB, V2A, V2B, 2, 1, 4, 2>(g, narrow_slices(g, tile_count(g, 32, 16)));
+    if (g.M <= 16 && tile_count(g, 16, 32) <= 0x7FFFFFFF)
+        return launch<KCA, KCB, V2A, V2B, 1, 2, 4, 2>(g, narrow_slices(g, tile_count(g, 16, 32)));
+    const Plan p = choose_tile(g, KCA && KCB);
+    switch (p.tile) {
+        case 0: return launch<KCA, KCB, V2A, V2B, 1, 1, 4, 4>(g, p.slices);
+        case 1: return launch<KCA, KCB, V2A, V2B, 2, 2, 4, 1>(g, p.slices);
+        case 2: return launch<KCA, KCB, V2A, V2B, 4, 2, 4, 1>(g, p.slices);
+        default: return launch<KCA, KCB, V2A, V2B, 4, 4, 1, 1>(g, 1);
+    }
+}
+
+template <bool KCA, bool KCB>
+int32_t run_layout(const Args& g) {
+    // 16-byte loads along K need every row to start 16-byte aligned.
+    const bool va = KCA && g.K % 2 == 0 && aligned16(g.a), vb = KCB && g.K % 2 == 0 && aligned16(g.b);
+    if (va && vb) return run_shape<KCA, KCB, KCA, KCB>(g);
+    if (va) return run_shape<KCA, KCB, KCA, false>(g);
+    if (vb) return run_shape<KCA, KCB, false, KCB>(g);
+    return run_shape<KCA, KCB, false, false>(g);
 }
 
 int32_t run_matmul_f64(const char* fn, const double* a, int64_t alen, const double* b, int64_t blen, double* c,
@@ -212,7 +375,6 @@ int32_t run_matmul_f64(const char* fn, const double* a, int64_t alen, const doub
                N, K);
     CH_REQUIRE((trans_a == 0 || trans_a == 1) && (trans_b == 0 || trans_b == 1), "%s: trans flags must be 0 or 1",
                fn);
-    const int64_t sa = (int64_t)M * K, sb = (int64_t)K * N, sc = (int64_t)M * N;
     const int64_t na = ch::count3(batch, M, K), nb = ch::count3(batch, K, N), nc = ch::count3(batch, M, N);
     CH_REQUIRE(na >= 0 && nb >= 0 && nc >= 0 && alen == na && blen == nb && clen == nc,
                "%s: lengths (%lld, %lld, %lld) do not match batch %d of %d x %d x %d", fn, (long long)alen,
@@ -225,15 +387,13 @@ int32_t run_matmul_f64(const char* fn, const double* a, int64_t alen, const doub
         CH_DEVICE(fn, b, blen * 8);
     }
     CH_DEVICE(fn, c, clen * 8);
-    const int64_t tiles = (int64_t)((M + BM - 1) / BM) * ((N + BN - 1) / BN) * batch;
-    CH_REQUIRE(tiles <= 0x7FFFFFFF, "%s: %lld workgroups exceed the grid limit", fn, (long long)tiles);
-    const unsigned grid = (unsigned)tiles;
-    if (!trans_a && !trans_b) launch_layout<false, false>(a, b, c, M, N, K, batch, sa, sb, sc, grid);
-    else if (!trans_a && trans_b) launch_layout<false, true>(a, b, c, M, N, K, batch, sa, sb, sc, grid);
-    else if (trans_a && !trans_b) launch_layout<true, false>(a, b, c, M, N, K, batch, sa, sb, sc, grid);
-    else launch_layout<true, true>(a, b, c, M, N, K, batch, sa, sb, sc, grid);
-    CH_LAUNCHED(fn);
-    return CLEAVE_HIP_OK;
+    const Args g{a, b, c, M, N, K, batch};
+    CH_REQUIRE(tile_count(g, 128, 128) <= 0x7FFFFFFF, "%s: %lld workgroups exceed the grid limit", fn,
+               (long long)tile_count(g, 128, 128));
+    if (!trans_a && !trans_b) return run_layout<true, false>(g);
+    if (!trans_a) return run_layout<true, true>(g);
+    if (!trans_b) return run_layout<false, false>(g);
+    return run_layout<false, true>(g);
 }
 
 }  // namespace

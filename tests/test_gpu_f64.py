@@ -276,3 +276,44 @@ def test_memref_forms(hip, oracle, ta, tb):
     want = np.zeros((17, 9))
     want[16, 8] = 1.25
     assert np.array_equal(g.numpy(), want)
+
+
+# Every wave tile of the f64 product (16 x 16, 32 x 32, 64 x 32, 128 x 128 and the two
+# narrow ones), with and without K slices, at tile edges and K remainders; whole-number
+# operands, so that every order of the sums gives the exact product.
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("batch,M,N,K", [
+    (1, 17, 33, 15), (1, 33, 77, 1001), (1, 128, 128, 128), (1, 257, 255, 256),  # 16 x 16
+    (1, 40, 40, 8191), (1, 512, 500, 65), (1, 700, 701, 130), (3, 65, 417, 300),  # 32 x 32
+    (1, 300, 300, 9999), (1, 1100, 690, 2001), (40, 129, 127, 60),  # 64 x 32
+    (1, 2049, 1153, 33), (1, 4097, 2047, 17), (70, 257, 255, 40),  # 128 x 128
+    (1, 1, 1, 70001), (1, 16, 16, 20000), (1, 300, 2, 4097), (1, 5000, 16, 300), (1, 33, 1, 1023),  # narrow N
+    (1, 1, 300, 4097), (1, 16, 2047, 1030), (9, 3, 65, 700)])  # narrow M
+def test_tiles_and_slices_exact(hip, batch, M, N, K, ta, tb):
+    rng = np.random.default_rng(M * 7 + N * 3 + K + 11 * ta + tb)
+    A = rng.integers(-9, 10, (batch, K, M) if ta else (batch, M, K)).astype(np.float64)
+    B = rng.integers(-9, 10, (batch, N, K) if tb else (batch, K, N)).astype(np.float64)
+    want = (A.transpose(0, 2, 1) if ta else A) @ (B.transpose(0, 2, 1) if tb else B)
+    a, b = hip.from_numpy(A), hip.from_numpy(B)
+    if batch > 1:
+        got = hip.matmul_batched(a, b, trans_a=bool(ta), trans_b=bool(tb)).numpy()
+    else:
+        c = hip.from_numpy(np.full((M, N), np.nan))
+        hip.matmul(a.view(A.shape[1:]), b.view(B.shape[1:]), trans_a=bool(ta), trans_b=bool(tb), out=c)
+        got = c.numpy()[None]
+    assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_k_tail_keeps_nan_and_inf_where_they_belong(hip, ta, tb):
+    # a NaN row of A and an infinite column of B: only their own entries, whatever K's remainder
+    for M, N, K in ((37, 50, 19), (20, 3, 2003)):
+        A, B = np.ones((M, K)), np.ones((K, N))
+        A[5, K - 1], B[0, 2] = np.nan, np.inf
+        want = np.full((M, N), float(K))
+        want[:, 2] = np.inf
+        want[5] = np.nan
+        got = hip.matmul(hip.from_numpy(np.ascontiguousarray(A.T if ta else A)),
+                         hip.from_numpy(np.ascontiguousarray(B.T if tb else B)), trans_a=bool(ta),
+                         trans_b=bool(tb)).numpy()
+        assert np.array_equal(np.nan_to_num(got, nan=-1.0), np.nan_to_num(want, nan=-1.0))
