@@ -16,8 +16,9 @@
 // gives the same |zr|, |zi| ever after, and NaN equals nothing and runs on.)
 // Rounding makes the orbits inside the set fall onto such cycles: over
 // [-2,1] x [-1.5,1.5] at 16384^2 x 1000 a wave's longest lane runs 64
-// iterations on average instead of 189, and the map takes 2.46 ms instead of
-// 5.65, bound by VALU issue as before.
+// iterations on average instead of 189, and the map takes 2.26 ms instead of
+// 5.64, bound by VALU issue as before; windows at the set's edge without such
+// orbits take the same time (2112 x 968, span 0.024, 236 iterations: 22.7 us).
 //
 // Bit-exactness: the library is compiled with -ffp-contract=off, so no mul+add
 // is fused behind the code's back.  Three rewrites are exact and save work:
@@ -46,40 +47,38 @@ namespace {
 // compare on the VALU, one scalar AND -- no branch, no count update.  Only in
 // a block where some lane escapes are the escaping lanes' counts formed, from
 // the block's masks: n = the block's first iteration + the number of the
-// block's masks that still hold the lane.  The wave leaves once no lane is
-// alive.  With 9 VALU per iteration (before 2p + ci became one fma), at
+// block's masks that still hold the lane, taken bit by bit from the masks with
+// scalar operations (eight adds with carry took 2-4% more over small windows).
+// The wave leaves once no lane is alive.  With 9 VALU per iteration (before 2p + ci became one fma), at
 // 16384^2 x 1000 blocks of 8 measured 6.10 ms, blocks of 16 6.28 ms, and a
 // count added every iteration 6.69 ms; on another box blocks of 4, 6, 8 and
 // 12 measured 6.40, 6.19, 6.12 and 6.21 ms.  The fma form: 5.61 ms.
 constexpr int kBlockIters = 8;
 
-// The state each block's end is compared with is retaken when the iteration
-// count reaches kFirstSave, and from then on each time it has grown by half:
-// the distance between takes grows, so cycles of any length fit in sooner or
-// later, and at most half as many iterations again pass before a settled
-// orbit is seen.  A block's end meets a cycle of p iterations lcm(p,
-// kBlockIters) after the take.  Iterations of a wave's longest lane, on
-// average over 6000 waves of the grid above and of a window at its edge,
-// [-0.9, -0.6] x [-0.05, 0.25] at 4096^2: without 189 / 863; takes at twice
-// the count 64.0 / 422, half as much again 63.7 / 410, a third 68 / 424, every
-// 64 iterations 82 / 501; blocks of 16, 82 / 473.
-constexpr uint32_t kFirstSave = 16;
-
-// count + 1 in the lanes set in `lanes` (a wave lane mask), as one
-// v_addc_co_u32 whose carry-in is that mask.  The carry-out goes to a scratch
-// SGPR pair of its own, so consecutive adds do not serialise on VCC.
-__device__ __forceinline__ uint32_t count_lanes(uint32_t count, uint64_t lanes) {
-    uint32_t r;
-    uint64_t carry_out;
-    asm("v_addc_co_u32_e64 %0, %1, 0, %2, %3" : "=v"(r), "=s"(carry_out) : "v"(count), "s"(lanes));
-    (void)carry_out;
-    return r;
-}
+// The state each block's end is compared with is first taken after kFirstTake
+// iterations, so a wave that is done by then pays nothing for it, and retaken
+// each time the count has grown by half: the distance between takes grows, so
+// cycles of any length fit in sooner or later, and at most half as many
+// iterations again pass before a settled orbit is seen.  A block's end meets a
+// cycle of p iterations lcm(p, kBlockIters) after the take.  Iterations of a
+// wave's longest lane, on average over 6000 waves of the grid above and of a
+// window at its edge, [-0.9, -0.6] x [-0.05, 0.25] at 4096^2: without 189 / 863;
+// first after 16 63.7 / 409.9, 48 63.6 / 409.9, 96 66.9 / 412.5; takes at twice
+// the count 64.6 / 423, every 64 iterations 82 / 501; blocks of 16, 82 / 473.
+constexpr int kFirstTake = 48;
 
 // if_set in the lanes set in `lanes`, if_clear in the others.
 __device__ __forceinline__ uint32_t select_lanes(uint64_t lanes, uint32_t if_set, uint32_t if_clear) {
     uint32_t r;
     asm("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(r) : "v"(if_clear), "v"(if_set), "s"(lanes));
+    return r;
+}
+
+// Bit (1, 2 or 4) in the lanes set in `lanes`, 0 in the others.
+template <int Bit>
+__device__ __forceinline__ uint32_t bit_lanes(uint64_t lanes) {
+    uint32_t r;
+    asm("v_cndmask_b32_e64 %0, 0, %1, %2" : "=v"(r) : "n"(Bit), "s"(lanes));
     return r;
 }
 
@@ -93,15 +92,13 @@ __global__ __launch_bounds__(256) void mandelbrot_kernel(uint32_t* __restrict__ 
     const float cr = x0 + (float)col * dx;
     const float ci = y0 + (float)row * dy;
     float zr = 0.0f, zi = 0.0f, zr2 = 0.0f, zi2 = 0.0f;
-    float sr = __builtin_nanf(""), si = 0.0f;  // the state kept for comparison: none yet
-    uint32_t next_save = kFirstSave;
     uint32_t count = 0;  // final in the lanes that have escaped
     uint64_t alive = __builtin_amdgcn_ballot_w64(inside);
     uint64_t cycling = 0;  // lanes that have met the state kept
     int n = 0;
     // Whole blocks: lanes past their escape keep iterating (z may overflow to
     // inf/NaN, which no longer matters: the count is latched).
-    for (; n + kBlockIters <= max_iter; n += kBlockIters) {
+    auto block = [&]() {
         const uint64_t before = alive;
         uint64_t after[kBlockIters];  // alive after each iteration of the block
 #pragma unroll
@@ -117,19 +114,36 @@ __global__ __launch_bounds__(256) void mandelbrot_kernel(uint32_t* __restrict__ 
         }
         const uint64_t escaped = before & ~alive;
         if (escaped != 0) {  // wave-uniform
-            uint32_t c = (uint32_t)n;
-#pragma unroll
-            for (int u = 0; u < kBlockIters; ++u) c = count_lanes(c, after[u]);
+            // the number of the block's masks that still hold an escaped lane,
+            // 0..7, bit by bit: each mask lies inside the one before
+            const uint64_t b0 = (after[0] & ~after[1]) | (after[2] & ~after[3]) | (after[4] & ~after[5]) | after[6];
+            const uint64_t b1 = (after[1] & ~after[3]) | after[5];
+            const uint32_t c = (uint32_t)n + (bit_lanes<4>(after[3]) | bit_lanes<2>(b1) | bit_lanes<1>(b0));
             count = select_lanes(escaped, c, count);
         }
-        const uint64_t met = __builtin_amdgcn_ballot_w64(zr == sr) & __builtin_amdgcn_ballot_w64(zi == si) & alive;
-        cycling |= met;
-        alive &= ~met;
-        if (alive == 0) break;
-        if ((uint32_t)(n + kBlockIters) >= next_save) {  // wave-uniform
-            sr = zr;
-            si = zi;
-            next_save += next_save / 2;
+    };
+    const int whole = max_iter & ~(kBlockIters - 1);
+    // A wave with no lane left sets n to kDone: one loop condition, one exit.
+    constexpr int kDone = 0x7FFFFFFF;
+    uint32_t next_take = kFirstTake;
+    int stop = whole < kFirstTake ? whole : kFirstTake;
+    while (n < stop) {
+        block();
+        n = alive != 0 ? n + kBlockIters : kDone;
+    }
+    while (n < whole) {
+        const float sr = zr, si = zi;  // the state that the next blocks' ends are compared with
+        next_take += next_take / 2;
+        stop = (uint32_t)whole < next_take ? whole : (int)next_take;
+        while (n < stop) {
+            block();
+            uint64_t met = __builtin_amdgcn_ballot_w64(zr == sr) & alive;
+            if (met != 0) {  // wave-uniform
+                met &= __builtin_amdgcn_ballot_w64(zi == si);
+                cycling |= met;
+                alive &= ~met;
+            }
+            n = alive != 0 ? n + kBlockIters : kDone;
         }
     }
     // Remaining max_iter % kBlockIters iterations (only when some lane survived).
