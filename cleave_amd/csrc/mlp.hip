@@ -9,14 +9,13 @@
 //   sigmoid via quotient + exp rules (num.cleave:132-134, :222) -> s(1-s)
 //
 // Kernel sequence on the library stream (device-resident, no host sync):
-//   1. H = X W1                         gemm_f32 NN   (M=B, N=Hd, K=D)
-//   2. H = sigmoid(H)                   map, in place
-//   3. row pass: z2 = H W2, yhat, e, sq = e*e, d2 = (e+e)/B * yhat(1-yhat)
-//   4. loss = sum(sq) / B               2-stage reduction
-//   5. column pass over H: dW2 partials += h*d2[m]; H <- d1 = (d2[m] W2[n]) h(1-h)
-//   6. dW2 = sum of partials; W2 -= lr dW2
-//   7. dW1 partials = X^T d1            gemm_f32 TN, split-K slices
-//   8. dW1 = sum of slices; W1 -= lr dW1
+//   1. X W1                             gemm_f32 NN   (M=B, N=Hd, K=D)
+//   2. per row: H = sigmoid(X W1), z2 = H W2, yhat, e, e*e,
+//      d2 = (e+e)/B * yhat(1-yhat), d1 = (d2 W2) h(1-h) over X W1, and
+//      partial sums of h*d2 and e*e     mlp_rows_kernel
+//   3. dW1 partials = X^T d1            gemm_f32 TN, split-K slices
+//   4. dW1, dW2 = sums of partials; W1 -= lr dW1, W2 -= lr dW2;
+//      loss = sum(e*e) / B              mlp_finish_kernel
 #include "common.hpp"
 #include "gemm_f32_pingpong.hpp"
 
@@ -31,59 +30,9 @@ constexpr int kThreads = 256;
 
 __device__ __forceinline__ float sigmoidf_ref(float x) { return 1.0f / (1.0f + expf(-x)); }
 
-__global__ __launch_bounds__(kThreads) void sigmoid_inplace_kernel(float* __restrict__ h, int64_t n) {
-    const int64_t nv = n / 4;
-    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < nv; i += (int64_t)gridDim.x * kThreads) {
-        float4 v = reinterpret_cast<float4*>(h)[i];
-        v.x = sigmoidf_ref(v.x);
-        v.y = sigmoidf_ref(v.y);
-        v.z = sigmoidf_ref(v.z);
-        v.w = sigmoidf_ref(v.w);
-        reinterpret_cast<float4*>(h)[i] = v;
-    }
-    if (blockIdx.x == 0 && threadIdx.x < (n & 3)) h[nv * 4 + threadIdx.x] = sigmoidf_ref(h[nv * 4 + threadIdx.x]);
-}
-
-// H[row,:] . W2 by one wave (every lane returns the sum).
-__device__ __forceinline__ float row_dot(const float* __restrict__ h, const float* __restrict__ W2, int Hd) {
-    const int lane = threadIdx.x & 63;
-    float acc = 0.0f;
-    if ((Hd & 3) == 0) {
-        for (int c = lane * 4; c < Hd; c += 256) {
-            float4 a = *reinterpret_cast<const float4*>(h + c);
-            float4 w = *reinterpret_cast<const float4*>(W2 + c);
-            acc += a.x * w.x + a.y * w.y + a.z * w.z + a.w * w.w;
-        }
-    } else {
-        for (int c = lane; c < Hd; c += 64) acc += h[c] * W2[c];
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
-    return acc;
-}
-
-// One wave per row: z2 = H[m,:] . W2, then the per-row loss pieces.
-__global__ __launch_bounds__(kThreads) void row_pass_kernel(const float* __restrict__ H,
-                                                            const float* __restrict__ W2,
-                                                            const float* __restrict__ y, int B,
-                                                            int Hd, float* __restrict__ sq,
-                                                            float* __restrict__ d2) {
-    const int lane = threadIdx.x & 63;
-    const int row = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
-    if (row >= B) return;
-    const float acc = row_dot(H + (int64_t)row * Hd, W2, Hd);
-    if (lane == 0) {
-        float yh = sigmoidf_ref(acc);
-        float e = yh - y[row];
-        sq[row] = e * e;
-        float gy = (e + e) / (float)B;
-        d2[row] = gy * yh * (1.0f - yh);
-    }
-}
-
 // Fused path, after the MODE-1 GEMM: z2[row] = sum of the P partials of
 // H[row] . W2 (in order; loads eight at a time), then the same per-row loss
-// pieces as row_pass_kernel.  Each block also reduces its rows' squared
+// pieces as mlp_rows_kernel.  Each block also reduces its rows' squared
 // errors into sqpart[block] (wave shuffles, then the 4 wave sums in order),
 // which loss_kernel adds up.
 constexpr int kPartUnroll = 8;
@@ -129,48 +78,262 @@ __global__ __launch_bounds__(kThreads) void row_finish_kernel(const float* __res
     }
 }
 
-// The hidden layer's z = H W2 alone: from the fused GEMM's partials (the z of
-// row_finish_kernel), or one wave per row (the z of row_pass_kernel).
+// The hidden layer's z = H W2 alone, from the fused GEMM's partials.
 __global__ __launch_bounds__(kThreads) void z_finish_kernel(const float* __restrict__ zpart, int P, int B,
                                                             float* __restrict__ z) {
     const int row = blockIdx.x * kThreads + threadIdx.x;
     if (row < B) z[row] = sum_row_partials(zpart, P, B, row);
 }
 
-__global__ __launch_bounds__(kThreads) void row_dot_kernel(const float* __restrict__ H, const float* __restrict__ W2,
-                                                           int B, int Hd, float* __restrict__ z) {
-    const int row = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
-    if (row >= B) return;
-    const float acc = row_dot(H + (int64_t)row * Hd, W2, Hd);
-    if ((threadIdx.x & 63) == 0) z[row] = acc;
+// Step 2 of the unfused path, and the hidden layer's two halves alone.  TPR threads
+// own a row, E elements of it each, in registers from the load to the store, so X W1
+// is read once and only d1 (or H) is written; dW2 partials stay in registers over the
+// rows a thread meets, and each workgroup writes one row of them.
+//   kStep  H holds X W1; v is y; writes d1 over H, dW2 and squared-error partials
+//   kFwd   H holds X W1; writes H over it and z = H W2 to z
+//   kBwd   H holds sigmoid(X W1), v is g = dL/dz; writes d1 to D1, dW2 partials
+// 1000 x 300 took 217 us in a column pass on 4 workgroups, after 14 us in three
+// launches for the sigmoid, the row products and the loss; it takes 8 us here.
+enum class Rows { kStep, kFwd, kBwd };
+template <int TPR, int E, bool VEC, Rows MODE>
+__global__ __launch_bounds__(kThreads) void mlp_rows_kernel(float* H, float* D1, const float* __restrict__ W2,
+                                                            const float* __restrict__ v, int B, int Hd,
+                                                            float* __restrict__ part, float* __restrict__ sqpart,
+                                                            float* __restrict__ z) {
+    typedef float v4 __attribute__((ext_vector_type(4)));
+    constexpr int RL = kThreads / TPR;  // rows in flight a workgroup
+    static_assert(E % 4 == 0 && (TPR == 64 || TPR == kThreads), "row shape");
+    __shared__ float cross[4];
+    __shared__ float red[RL > 1 ? RL * TPR * E : 1];
+    const int t = threadIdx.x % TPR, rl = threadIdx.x / TPR;
+    auto col = [&](int i) { return VEC ? ((i / 4) * TPR + t) * 4 + i % 4 : i * TPR + t; };
+    auto load = [&](const float* __restrict__ p, float (&x)[E]) {
+        if constexpr (VEC) {
+#pragma unroll
+            for (int i = 0; i < E; i += 4) {
+                const v4 q = col(i) < Hd ? *reinterpret_cast<const v4*>(p + col(i)) : v4(0.0f);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) x[i + j] = q[j];
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < E; ++i) x[i] = col(i) < Hd ? p[col(i)] : 0.0f;
+        }
+    };
+    auto store = [&](float* p, const float (&x)[E]) {
+        if constexpr (VEC) {
+#pragma unroll
+            for (int i = 0; i < E; i += 4)
+                if (col(i) < Hd) *reinterpret_cast<v4*>(p + col(i)) = v4{x[i], x[i + 1], x[i + 2], x[i + 3]};
+        } else {
+#pragma unroll
+            for (int i = 0; i < E; ++i)
+                if (col(i) < Hd) p[col(i)] = x[i];
+        }
+    };
+    float w[E], s[E], h[E], next[E];
+    load(W2, w);
+#pragma unroll
+    for (int i = 0; i < E; ++i) s[i] = 0.0f;
+    float sq = 0.0f;
+    const int step = (int)gridDim.x * RL;
+    int64_t r = (int64_t)blockIdx.x * RL + rl;
+    if (r < B) load(H + r * Hd, next);
+    for (; r < B; r += step) {
+#pragma unroll
+        for (int i = 0; i < E; ++i) h[i] = next[i];
+        if (r + step < B) load(H + (r + step) * Hd, next);
+        float d2;
+        if constexpr (MODE == Rows::kBwd) {
+            d2 = v[r];
+        } else {
+            float acc = 0.0f;
+#pragma unroll
+            for (int i = 0; i < E; ++i) {
+                h[i] = sigmoidf_ref(h[i]);
+                acc += h[i] * w[i];
+            }
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
+            if constexpr (TPR > 64) {
+                __syncthreads();
+                if ((t & 63) == 0) cross[t >> 6] = acc;
+                __syncthreads();
+                acc = (cross[0] + cross[1]) + (cross[2] + cross[3]);
+            }
+            if constexpr (MODE == Rows::kFwd) {
+                if (t == 0) z[r] = acc;
+                store(H + r * Hd, h);
+                continue;
+            }
+            const float yh = sigmoidf_ref(acc);
+            const float e = yh - v[r];
+            sq += e * e;
+            const float gy = (e + e) / (float)B;
+            d2 = gy * yh * (1.0f - yh);
+        }
+        float d1[E];
+#pragma unroll
+        for (int i = 0; i < E; ++i) {
+            s[i] += h[i] * d2;
+            const float g = d2 * w[i];
+            d1[i] = g * h[i] * (1.0f - h[i]);
+        }
+        store((MODE == Rows::kBwd ? D1 : H) + r * Hd, d1);
+    }
+    if constexpr (MODE == Rows::kFwd) return;
+    // the workgroup's row of dW2 partials: its RL rows' sums in order
+    if constexpr (RL > 1) {
+#pragma unroll
+        for (int i = 0; i < E; ++i) red[(rl * E + i) * TPR + t] = s[i];
+        if (t == 0) cross[rl] = sq;
+        __syncthreads();
+        if (rl != 0) return;
+#pragma unroll
+        for (int i = 0; i < E; ++i)
+#pragma unroll
+            for (int q = 1; q < RL; ++q) s[i] += red[(q * E + i) * TPR + t];
+        sq = ((cross[0] + cross[1]) + cross[2]) + cross[3];
+    }
+    store(part + (int64_t)blockIdx.x * Hd, s);
+    if (MODE == Rows::kStep && t == 0) sqpart[blockIdx.x] = sq;
 }
 
-// Column pass: each thread owns 4 consecutive columns of a band of rows.
-// Writes d1 (over H when D1 is H) and one dW2 partial per (row band, column).
-constexpr int kRowsPerBand = 256;
-__global__ __launch_bounds__(kThreads) void col_pass_kernel(const float* H, float* D1,
-                                                            const float* __restrict__ W2,
-                                                            const float* __restrict__ d2, int B,
-                                                            int Hd, float* __restrict__ part) {
-    const int c = (blockIdx.x * kThreads + threadIdx.x) * 4;
-    if (c >= Hd) return;
-    const int r0 = blockIdx.y * kRowsPerBand;
-    const int r1 = min(B, r0 + kRowsPerBand);
-    const int nc = min(4, Hd - c);
-    float w[4], s[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int j = 0; j < 4; ++j) w[j] = j < nc ? W2[c + j] : 0.0f;
-    for (int r = r0; r < r1; ++r) {
-        const float* h = H + (int64_t)r * Hd + c;
-        float* d1 = D1 + (int64_t)r * Hd + c;
-        const float dm = d2[r];
-        for (int j = 0; j < nc; ++j) {
-            float hv = h[j];
-            s[j] += hv * dm;
-            float g = dm * w[j];
-            d1[j] = g * hv * (1.0f - hv);
+// The same for rows past 16 elements a thread (Hd > 4096): a workgroup walks its row
+// twice, with H in memory between, and adds to its row of partials in place.
+template <Rows MODE>
+__global__ __launch_bounds__(kThreads) void mlp_rows_wide_kernel(float* H, float* D1, const float* __restrict__ W2,
+                                                                 const float* __restrict__ v, int B, int Hd,
+                                                                 float* part, float* __restrict__ sqpart,
+                                                                 float* __restrict__ z) {
+    __shared__ float cross[4];
+    float sq = 0.0f;
+    float* mine = part + (int64_t)blockIdx.x * Hd;
+    for (int64_t r = blockIdx.x; r < B; r += gridDim.x) {
+        float* h = H + r * Hd;
+        float d2;
+        if constexpr (MODE == Rows::kBwd) {
+            d2 = v[r];
+        } else {
+            float acc = 0.0f;
+            for (int c = threadIdx.x; c < Hd; c += kThreads) {
+                const float x = sigmoidf_ref(h[c]);
+                h[c] = x;
+                acc += x * W2[c];
+            }
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
+            __syncthreads();
+            if ((threadIdx.x & 63) == 0) cross[threadIdx.x >> 6] = acc;
+            __syncthreads();
+            acc = (cross[0] + cross[1]) + (cross[2] + cross[3]);
+            if constexpr (MODE == Rows::kFwd) {
+                if (threadIdx.x == 0) z[r] = acc;
+                continue;
+            }
+            const float yh = sigmoidf_ref(acc);
+            const float e = yh - v[r];
+            sq += e * e;
+            const float gy = (e + e) / (float)B;
+            d2 = gy * yh * (1.0f - yh);
+        }
+        float* d1 = (MODE == Rows::kBwd ? D1 : H) + r * Hd;
+        for (int c = threadIdx.x; c < Hd; c += kThreads) {  // each thread meets its own columns again
+            const float x = h[c], g = d2 * W2[c];
+            const float s = x * d2;
+            mine[c] = r == blockIdx.x ? s : mine[c] + s;
+            d1[c] = g * x * (1.0f - x);
         }
     }
-    for (int j = 0; j < nc; ++j) part[(int64_t)blockIdx.y * Hd + c + j] = s[j];
+    if (MODE == Rows::kStep && threadIdx.x == 0) sqpart[blockIdx.x] = sq;
+}
+
+// Workgroups of the row pass: one row a thread group, up to two workgroups a CU.
+int row_groups(int B, int Hd) {
+    const int lanes = Hd <= 1024 ? kThreads / 64 : 1;
+    const int64_t want = ((int64_t)B + lanes - 1) / lanes, cap = 2 * (int64_t)ch::num_cus();
+    return (int)(want < cap ? want : cap);
+}
+
+template <Rows MODE>
+int32_t run_rows(float* H, float* D1, const float* W2, const float* v, int B, int Hd, float* part, float* sqpart,
+                 float* z, hipStream_t st) {
+    const unsigned grid = (unsigned)row_groups(B, Hd);
+    const bool vec = Hd % 4 == 0 && (((uintptr_t)H | (uintptr_t)D1 | (uintptr_t)W2 | (uintptr_t)part) & 15) == 0;
+    auto go = [&](auto kernel) { kernel<<<grid, kThreads, 0, st>>>(H, D1, W2, v, B, Hd, part, sqpart, z); };
+    if (Hd <= 256) vec ? go(mlp_rows_kernel<64, 4, true, MODE>) : go(mlp_rows_kernel<64, 4, false, MODE>);
+    else if (Hd <= 512) vec ? go(mlp_rows_kernel<64, 8, true, MODE>) : go(mlp_rows_kernel<64, 8, false, MODE>);
+    else if (Hd <= 1024) vec ? go(mlp_rows_kernel<64, 16, true, MODE>) : go(mlp_rows_kernel<64, 16, false, MODE>);
+    else if (Hd <= 2048) vec ? go(mlp_rows_kernel<256, 8, true, MODE>) : go(mlp_rows_kernel<256, 8, false, MODE>);
+    else if (Hd <= 4096) vec ? go(mlp_rows_kernel<256, 16, true, MODE>) : go(mlp_rows_kernel<256, 16, false, MODE>);
+    else go(mlp_rows_wide_kernel<MODE>);
+    CH_LAUNCHED("mlp_rows_kernel");
+    return CLEAVE_HIP_OK;
+}
+
+// Step 4: workgroups [0, blocks1) sum the dW1 slices and update W1; the next
+// ceil(Hd / kFoldCols) sum the dW2 partials (kFoldLanes threads a column, each its
+// run of them in order, then the runs in order) and update W2; the last one, if
+// there is a loss to write, sums the squared errors.  A null dw or w is left out.
+constexpr int kFoldCols = 16, kFoldLanes = kThreads / kFoldCols;
+struct Finish {
+    const float* part1;  // slices x n1
+    int slices, blocks1;
+    int64_t n1;
+    float *dw1, *w1;
+    const float* part2;  // groups x Hd
+    int groups, Hd;
+    float *dw2, *w2;
+    const float* sqpart;  // groups
+    float* loss;
+    float count, lr;
+};
+unsigned finish_grid(const Finish& f) {
+    return (unsigned)(f.blocks1 + (f.Hd + kFoldCols - 1) / kFoldCols + (f.loss ? 1 : 0));
+}
+__global__ __launch_bounds__(kThreads) void mlp_finish_kernel(Finish f) {
+    auto update = [&](float g, float* dw, float* w, int64_t i) {
+        if (dw) dw[i] = g;
+        if (f.lr != 0.0f && w) w[i] = w[i] - f.lr * g;
+    };
+    if ((int)blockIdx.x < f.blocks1) {
+        for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < f.n1; i += (int64_t)f.blocks1 * kThreads) {
+            float g = f.part1[i];
+            for (int s = 1; s < f.slices; ++s) g += f.part1[(int64_t)s * f.n1 + i];
+            update(g, f.dw1, f.w1, i);
+        }
+        return;
+    }
+    __shared__ float red[kThreads];
+    const int fold = (f.Hd + kFoldCols - 1) / kFoldCols;
+    const bool errors = (int)blockIdx.x == f.blocks1 + fold;
+    // a run of partials: a column's, or the squared errors (a thread each)
+    const int cols = errors ? 1 : kFoldCols, lanes = errors ? kThreads : kFoldLanes;
+    const int lane = threadIdx.x / cols;
+    const int c = errors ? 0 : ((int)blockIdx.x - f.blocks1) * kFoldCols + (int)threadIdx.x % cols;
+    const float* p = errors ? f.sqpart : f.part2 + c;
+    const int64_t pitch = errors ? 1 : f.Hd;
+    const int q0 = (int)((int64_t)f.groups * lane / lanes), q1 = (int)((int64_t)f.groups * (lane + 1) / lanes);
+    float acc = 0.0f;
+    if (errors || c < f.Hd) {
+        int q = q0;
+        for (; q + kPartUnroll <= q1; q += kPartUnroll) {
+            float x[kPartUnroll];
+#pragma unroll
+            for (int u = 0; u < kPartUnroll; ++u) x[u] = p[(q + u) * pitch];
+#pragma unroll
+            for (int u = 0; u < kPartUnroll; ++u) acc += x[u];
+        }
+        for (; q < q1; ++q) acc += p[q * pitch];
+    }
+    red[threadIdx.x] = acc;
+    for (int half = lanes / 2; half > 0; half /= 2) {
+        __syncthreads();
+        if (lane < half) red[threadIdx.x] += red[threadIdx.x + half * cols];
+    }
+    if (lane != 0) return;
+    if (errors) *f.loss = red[threadIdx.x] / f.count;
+    else if (c < f.Hd) update(red[threadIdx.x], f.dw2, f.w2, c);
 }
 
 // out[i] = sum_s part[s*n + i] (fixed order); optional copy to dW; W -= lr * out.
@@ -368,12 +531,7 @@ int32_t hidden_fwd(const float* x, const float* w1, const float* w2, float* h, f
     }
     int32_t rc = ch::gemm_f32_device(x, w1, h, B, Hd, D, 0, 0, 1);
     if (rc != CLEAVE_HIP_OK) return rc;
-    const int64_t nH = (int64_t)B * Hd;
-    sigmoid_inplace_kernel<<<capped_grid(nH / 4 + 1), kThreads, 0, st>>>(h, nH);
-    CH_LAUNCHED("sigmoid_inplace_kernel");
-    row_dot_kernel<<<(B + 3) / 4, kThreads, 0, st>>>(h, w2, B, Hd, z);
-    CH_LAUNCHED("row_dot_kernel");
-    return CLEAVE_HIP_OK;
+    return run_rows<Rows::kFwd>(h, nullptr, w2, nullptr, B, Hd, nullptr, nullptr, z, st);
 }
 
 int32_t hidden_bwd(const float* x, const float* h, const float* w2, const float* g, float* dw1, float* dw2, int B,
@@ -406,27 +564,28 @@ int32_t hidden_bwd(const float* x, const float* h, const float* w2, const float*
         }
         return CLEAVE_HIP_OK;
     }
-    const int splits = choose_splits(D, Hd, B);
-    const int bands = (B + kRowsPerBand - 1) / kRowsPerBand;
-    const size_t nH = (size_t)B * Hd, nPart = (size_t)bands * Hd, nSl = (size_t)splits * D * Hd;
+    const int splits = dw1 ? choose_splits(D, Hd, B) : 0;
+    const int groups = row_groups(B, Hd);
+    const size_t nH = (size_t)B * Hd, nPart = (size_t)groups * Hd, nSl = splits > 1 ? (size_t)splits * D * Hd : 0;
     float* d1 = (float*)ch::scratch(4, sizeof(float) * (up(nH) + up(nPart) + up(nSl)));
     if (!d1) return CLEAVE_HIP_ERR_OOM;
     float* part = d1 + up(nH);
-    float* slices = part + up(nPart);
-    dim3 cgrid((unsigned)((Hd + 4 * kThreads - 1) / (4 * kThreads)), (unsigned)bands);
-    col_pass_kernel<<<cgrid, kThreads, 0, st>>>(h, d1, w2, g, B, Hd, part);
-    CH_LAUNCHED("col_pass_kernel");
-    if (dw2) {
-        sum_slices_sgd_kernel<<<capped_grid(Hd), kThreads, 0, st>>>(part, bands, Hd, dw2, nullptr, 0.0f);
-        CH_LAUNCHED("sum_slices_sgd_kernel(dW2)");
-    }
+    float* slices = splits > 1 ? part + up(nPart) : dw1;
+    int32_t rc = run_rows<Rows::kBwd>(const_cast<float*>(h), d1, w2, g, B, Hd, part, nullptr, nullptr, st);
+    if (rc != CLEAVE_HIP_OK) return rc;
     if (dw1) {
-        int32_t rc = ch::gemm_f32_device(x, d1, slices, D, Hd, B, 1, 0, splits);
+        rc = ch::gemm_f32_device(x, d1, slices, D, Hd, B, 1, 0, splits);
         if (rc != CLEAVE_HIP_OK) return rc;
-        sum_slices_sgd_kernel<<<capped_grid((int64_t)D * Hd), kThreads, 0, st>>>(slices, splits, (int64_t)D * Hd,
-                                                                                  dw1, nullptr, 0.0f);
-        CH_LAUNCHED("sum_slices_sgd_kernel(dW1)");
     }
+    Finish f{};
+    if (splits > 1) {
+        f.part1 = slices, f.slices = splits, f.n1 = (int64_t)D * Hd, f.blocks1 = (int)capped_grid(f.n1);
+        f.dw1 = dw1;
+    }
+    if (dw2) f.part2 = part, f.groups = groups, f.Hd = Hd, f.dw2 = dw2;
+    if (finish_grid(f) == 0) return CLEAVE_HIP_OK;
+    mlp_finish_kernel<<<finish_grid(f), kThreads, 0, st>>>(f);
+    CH_LAUNCHED("mlp_finish_kernel");
     return CLEAVE_HIP_OK;
 }
 
@@ -460,37 +619,29 @@ extern "C" int32_t cleave_hip_mlp_step_f32(const float* x, int64_t xlen, const f
     if (fused_fits(x, w1, B, D, Hd)) return fused_step(x, y, w1, w2, dw1, dw2, loss_dev, B, D, Hd, lr, st);
 
     const int splits = choose_splits(D, Hd, B);
-    const int bands = (B + kRowsPerBand - 1) / kRowsPerBand;
-    // Scratch slot 4: H/d1 | sq | d2 | dW2 partials | dW1 slices | loss.
-    const size_t nH = (size_t)B * Hd, nPart = (size_t)bands * Hd, nSl = (size_t)splits * D * Hd;
+    const int groups = row_groups(B, Hd);
+    // Scratch slot 4: H/d1 | dW2 partials | squared errors | dW1 slices.
+    const size_t nH = (size_t)B * Hd, nPart = (size_t)groups * Hd, nSl = (size_t)splits * D * Hd;
     auto up = [](size_t n) { return (n + 63) & ~(size_t)63; };
-    const size_t total = up(nH) + up(B) + up(B) + up(nPart) + up(nSl) + 64;
-    float* base = (float*)ch::scratch(4, total * sizeof(float));
-    if (!base) return CLEAVE_HIP_ERR_OOM;
-    float* H = base;
-    float* sq = H + up(nH);
-    float* d2 = sq + up(B);
-    float* part = d2 + up(B);
-    float* slices = part + up(nPart);
-    float* loss_tmp = slices + up(nSl);
+    float* H = (float*)ch::scratch(4, sizeof(float) * (up(nH) + up(nPart) + up(groups) + up(nSl)));
+    if (!H) return CLEAVE_HIP_ERR_OOM;
+    float* part = H + up(nH);
+    float* sq = part + up(nPart);
+    float* slices = splits > 1 || !dw1 ? sq + up(groups) : dw1;
 
     int32_t rc = ch::gemm_f32_device(x, w1, H, B, Hd, D, 0, 0, 1);
     if (rc != CLEAVE_HIP_OK) return rc;
-    sigmoid_inplace_kernel<<<capped_grid(nH / 4 + 1), kThreads, 0, st>>>(H, (int64_t)nH);
-    CH_LAUNCHED("sigmoid_inplace_kernel");
-    row_pass_kernel<<<(B + 3) / 4, kThreads, 0, st>>>(H, w2, y, B, Hd, sq, d2);
-    CH_LAUNCHED("row_pass_kernel");
-    loss_kernel<<<1, kThreads, 0, st>>>(sq, B, (float)B, loss_dev ? loss_dev : loss_tmp);
-    CH_LAUNCHED("loss_kernel");
-    dim3 cgrid((unsigned)((Hd + 4 * kThreads - 1) / (4 * kThreads)), (unsigned)bands);
-    col_pass_kernel<<<cgrid, kThreads, 0, st>>>(H, H, w2, d2, B, Hd, part);
-    CH_LAUNCHED("col_pass_kernel");
-    sum_slices_sgd_kernel<<<capped_grid(Hd), kThreads, 0, st>>>(part, bands, Hd, dw2, w2, lr);
-    CH_LAUNCHED("sum_slices_sgd_kernel(dW2)");
+    rc = run_rows<Rows::kStep>(H, nullptr, w2, y, B, Hd, part, sq, nullptr, st);
+    if (rc != CLEAVE_HIP_OK) return rc;
     rc = ch::gemm_f32_device(x, H, slices, D, Hd, B, 1, 0, splits);
     if (rc != CLEAVE_HIP_OK) return rc;
-    sum_slices_sgd_kernel<<<capped_grid((int64_t)D * Hd), kThreads, 0, st>>>(slices, splits, (int64_t)D * Hd, dw1, w1, lr);
-    CH_LAUNCHED("sum_slices_sgd_kernel(dW1)");
+    Finish f{};
+    f.part1 = slices, f.slices = splits, f.n1 = (int64_t)D * Hd, f.blocks1 = (int)capped_grid(f.n1);
+    f.dw1 = slices == dw1 ? nullptr : dw1, f.w1 = w1;
+    f.part2 = part, f.groups = groups, f.Hd = Hd, f.dw2 = dw2, f.w2 = w2;
+    f.sqpart = sq, f.loss = loss_dev, f.count = (float)B, f.lr = lr;
+    mlp_finish_kernel<<<finish_grid(f), kThreads, 0, st>>>(f);
+    CH_LAUNCHED("mlp_finish_kernel");
     return CLEAVE_HIP_OK;
 }
 

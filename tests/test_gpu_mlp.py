@@ -230,3 +230,44 @@ def test_hidden_layer_forward_and_rule(hip, oracle, B, D, Hd):
     tol = 1e-5 * np.sqrt(B)
     assert np.all(np.abs(dw1.numpy() - dW1r) <= tol * a1 + 1e-6 * np.abs(dW1r))
     assert np.all(np.abs(dw2.numpy().ravel() - dW2r) <= tol * a2)
+
+
+# The row pass at every register shape (64 or 256 threads a row, 4 to 16 elements each,
+# in chunks or single elements) and past it, with fewer rows than workgroups and more.
+@pytest.mark.parametrize("B", [1, 3, 130])
+@pytest.mark.parametrize("Hd", [1, 3, 64, 255, 256, 257, 510, 512, 1000, 1024, 1025, 2047, 2048, 2052, 4095, 4096,
+                                4100, 5003])
+def test_row_pass_widths(hip, oracle, B, Hd):
+    rng = np.random.default_rng(B * 10007 + Hd)
+    D = 7
+    X = rng.standard_normal((B, D)).astype(np.float32)
+    y = (rng.random(B) < 0.5).astype(np.float32)
+    W1 = _xavier(rng, D, Hd, (D, Hd))
+    W2 = _xavier(rng, Hd, 1, Hd)
+    loss_r, dW1_r, dW2_r, _, _ = oracle.mlp_step(X, y, W1, W2, lr=0.01, threads=8)
+    x, yd, w1, w2 = (hip.from_numpy(v) for v in (X, y, W1, W2))
+    dw1, dw2, loss = hip.empty((D, Hd)), hip.empty(Hd), hip.empty(1)
+    hip.mlp_step(x, yd, w1, w2, 0.01, dw1=dw1, dw2=dw2, loss=loss)
+    assert abs(loss.numpy()[0] - loss_r) <= 1e-5 * abs(loss_r)
+    assert_mlp_grads_close(dw1.numpy(), dw2.numpy(), dW1_r, dW2_r, X, y, W1, W2, f"B={B} Hd={Hd}")
+    assert np.array_equal(w1.numpy(), W1 - np.float32(0.01) * dw1.numpy())
+    assert np.array_equal(w2.numpy(), W2 - np.float32(0.01) * dw2.numpy())
+
+    # the hidden layer alone: float64 values of the same layer, GEMM bounds
+    w1, w2 = hip.from_numpy(W1), hip.from_numpy(W2.reshape(Hd, 1))
+    h, z = hip.sigmoid_hidden_fwd(x, w1, w2)
+    H = 1.0 / (1.0 + np.exp(-(X.astype(np.float64) @ W1)))
+    assert np.allclose(h.numpy(), H, rtol=2e-6, atol=0)
+    # |z - H w2| <= 1e-5 sqrt(Hd) |H| |w2|: H carries a few roundings, the sum sqrt(Hd)
+    assert np.all(np.abs(z.numpy()[:, 0] - H @ W2) <= 1e-5 * np.sqrt(Hd) * (H @ np.abs(W2)))
+    g = hip.from_numpy(rng.standard_normal((B, 1)).astype(np.float32))
+    G, Hn = g.numpy().astype(np.float64), h.numpy().astype(np.float64)
+    d1 = (G * W2) * Hn * (1.0 - Hn)
+    tol = 1e-5 * np.sqrt(B)
+    for which in ("both", "dw1", "dw2"):
+        a, b = hip.empty((D, Hd)), hip.empty((Hd, 1))
+        hip.sigmoid_hidden_bwd(x, h, w2, g, a if which != "dw2" else None, b if which != "dw1" else None)
+        if which != "dw2":
+            assert np.all(np.abs(a.numpy() - X.T @ d1) <= tol * (np.abs(X).T @ np.abs(d1)) + 1e-30)
+        if which != "dw1":
+            assert np.all(np.abs(b.numpy() - Hn.T @ G) <= tol * (Hn.T @ np.abs(G)) + 1e-30)
