@@ -39,6 +39,8 @@
 #include "gemm_pad.hpp"
 
 namespace ch {
+bool try_direct_f32(const float* a, const float* b, float* c, int M, int N, int K, int batch, int ta, int tb,
+                    double most_us, int32_t* st);
 int32_t matmul_vector_f32(const float* a, const float* b, float* c, int M, int N, int K, int batch, int ta, int tb);
 int32_t matmul_skinny_f32(const float* a, const float* b, float* c, int M, int N, int K, int batch, int ta, int tb);
 }
@@ -249,7 +251,7 @@ bool launch_tiled(const float* a, const float* b, float* c, int M, int N, int K,
     if ((int64_t)tiles_m * tiles_n * batch > 0x7FFFFFFF) return false;
     dim3 grid((unsigned)(tiles_m * tiles_n * batch));
     ch::gemm_f32_tiled_kernel<BM, BN, BK, WM, WN, STAGES, !TA, TB><<<grid, P::THREADS, 0, ch::stream()>>>(
-        a, b, c, M, N, K, lda, ldb, sA, sB, sC, tiles_m, tiles_n, batch);
+        a, b, c, M, N, K, lda, ldb, sA, sB, sC, tiles_m, tiles_n, batch, 0);
     *status = ch::check_hip(hipGetLastError(), "gemm_f32_tiled_kernel");
     return true;
 }
@@ -259,7 +261,7 @@ bool launch_tiled(const float* a, const float* b, float* c, int M, int N, int K,
 template <int BM, int BN, int BK, int WM, int WN, int STAGES, bool TA, bool TB>
 bool launch_tiled_edge(const float* a, const float* b, float* c, int M, int N, int K, int64_t lda,
                        int64_t ldb, int batch, int64_t sA, int64_t sB, int64_t sC, int32_t* status,
-                       bool padded = false) {
+                       bool padded = false, int ktotal = 0) {
     using P = ch::F32Tiled<BM, BN, BK, WM, WN, STAGES, !TA, TB>;
     if (!P::fits_edge(M, N, K, lda, ldb, padded) || ((uintptr_t)a & 15) || ((uintptr_t)b & 15) || (sA % 4) || (sB % 4))
         return false;
@@ -267,7 +269,7 @@ bool launch_tiled_edge(const float* a, const float* b, float* c, int M, int N, i
     if ((int64_t)tiles_m * tiles_n * batch > 0x7FFFFFFF) return false;
     dim3 grid((unsigned)(tiles_m * tiles_n * batch));
     ch::gemm_f32_tiled_kernel<BM, BN, BK, WM, WN, STAGES, !TA, TB, true><<<grid, P::THREADS, 0, ch::stream()>>>(
-        a, b, c, M, N, K, lda, ldb, sA, sB, sC, tiles_m, tiles_n, batch);
+        a, b, c, M, N, K, lda, ldb, sA, sB, sC, tiles_m, tiles_n, batch, ktotal);
     *status = ch::check_hip(hipGetLastError(), "gemm_f32_tiled_kernel");
     return true;
 }
@@ -638,6 +640,9 @@ constexpr double kEdgeTileKUs = 0.0163;
 // CUs, 479 us): 8% less per flop than 64 x 64 when the tiles are many.
 constexpr double kEdge128TileKUs = 0.0599;
 
+// Depth of S K slices: whole 16-deep k-tiles; the last slice takes what is left.
+int slice_depth(int K, int S) { return (int)(((int64_t)K + S - 1) / S + 15) / 16 * 16; }
+
 // One ragged product (an M or N off the 64 grid) with a long K as S K
 // slices on the 64 x 64 kernel's guarded-edge form, its batch running over
 // the slices, added in order (deterministic); each slice at least 512 deep
@@ -669,32 +674,28 @@ bool try_edge_slices(const float* a, const float* b, float* c, int M, int N, int
     // the slices written and read back at 5 TB/s
     auto cost = [&](int64_t t, double tile_k_us, int s) {
         const double busiest = (double)((t * s + cus - 1) / cus);
-        return busiest * ((double)K / s) * tile_k_us + (s > 1 ? 8.0 * s * (double)M * N / 5.0e6 : 0.0);
+        return busiest * slice_depth(K, s) * tile_k_us + (s > 1 ? 4.0 + 8.0 * s * (double)M * N / 5.0e6 : 0.0);
     };
     int S = 1;
-    if (tiles <= cus) {
-        S = (int)std::min<int64_t>(kEdgeTilesPerCu * cus / tiles, K / 512);
-        while (S >= 2 && K % (4 * S) != 0) --S;
-    } else {
-        if (tiles > kEdgeTilesPerCu * cus || K < 4096) return false;
-        double best = 0.95 * cost(tiles, kEdgeTileKUs, 1);
-        for (int s = 2; s <= 16 && K / s >= 512; ++s)
-            if (K % (4 * s) == 0 && cost(tiles, kEdgeTileKUs, s) < best) best = cost(tiles, kEdgeTileKUs, s), S = s;
-    }
+    if (tiles > cus && (tiles > kEdgeTilesPerCu * cus || K < 4096)) return false;
+    double best = (tiles <= cus ? 1.0 : 0.95) * cost(tiles, kEdgeTileKUs, 1);
+    for (int s = 2; s <= 64 && K / s >= 512 && tiles * s <= 8 * cus; ++s)
+        if (cost(tiles, kEdgeTileKUs, s) < best) best = cost(tiles, kEdgeTileKUs, s), S = s;
     bool big = false;  // 128 x 128 tiles, at least three per CU (the rate kEdge128TileKUs holds for)
     if (K >= 4096) {
         const int64_t t128 = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
-        double best = 0.97 * cost(tiles, kEdgeTileKUs, S);
+        best *= 0.97;
         for (int s = 2; s <= 64 && K / s >= 512 && t128 * s <= kEdgeTilesPerCu * cus; ++s)
-            if (K % (4 * s) == 0 && t128 * s >= 3 * cus && cost(t128, kEdge128TileKUs, s) < best)
+            if (t128 * s >= 3 * cus && cost(t128, kEdge128TileKUs, s) < best)
                 best = cost(t128, kEdge128TileKUs, s), S = s, big = true;
     }
     if (S < 2) return false;
-    const int kk = K / S;
+    const int kk = slice_depth(K, S);
+    S = (K + kk - 1) / kk;
     const int64_t sA = TA ? (int64_t)kk * lda : kk, sB = TB ? kk : (int64_t)kk * ldb;
     using P = ch::F32Tiled<64, 64, 16, 2, 2, 4, !TA, TB>;
-    if (!P::fits_edge(M, N, kk, lda, ldb, padded) || ((uintptr_t)a & 15) || ((uintptr_t)b & 15) || sA % 4 ||
-        sB % 4)
+    if (!P::fits_edge(M, N, kk, lda, ldb, padded) || ((!TA || TB) && K % 4) || ((uintptr_t)a & 15) ||
+        ((uintptr_t)b & 15) || sA % 4 || sB % 4)
         return false;
     const int64_t n = (int64_t)M * N, n4 = (n + 3) / 4 * 4;
     float* part = (float*)ch::scratch_try(9, sizeof(float) * (size_t)S * n4);
@@ -702,13 +703,13 @@ bool try_edge_slices(const float* a, const float* b, float* c, int M, int N, int
     bool launched;
     if (big)
         launched =
-            launch_tiled_edge<128, 128, 16, 2, 2, 2, TA, TB>(a, b, part, M, N, kk, lda, ldb, S, sA, sB, n4, st, padded);
+            launch_tiled_edge<128, 128, 16, 2, 2, 2, TA, TB>(a, b, part, M, N, kk, lda, ldb, S, sA, sB, n4, st, padded, K);
     else
         launched =
             (tiles * S <= 2 * cus &&
-             launch_tiled_edge<64, 64, 32, 2, 2, 4, TA, TB>(a, b, part, M, N, kk, lda, ldb, S, sA, sB, n4, st, padded)) ||
-            launch_tiled_edge<64, 64, 16, 2, 2, 4, TA, TB>(a, b, part, M, N, kk, lda, ldb, S, sA, sB, n4, st, padded);
-    if (!launched) *st = launch_general<TA, TB>(a, b, part, M, N, kk, lda, ldb, N, S, sA, sB, n4);
+             launch_tiled_edge<64, 64, 32, 2, 2, 4, TA, TB>(a, b, part, M, N, kk, lda, ldb, S, sA, sB, n4, st, padded, K)) ||
+            launch_tiled_edge<64, 64, 16, 2, 2, 4, TA, TB>(a, b, part, M, N, kk, lda, ldb, S, sA, sB, n4, st, padded, K);
+    if (!launched) return false;
     if (*st == CLEAVE_HIP_OK) *st = ch::sum_slices_f32(part, c, n, S, n4);
     return true;
 }
@@ -829,46 +830,67 @@ bool try_batched_k_slices(const float* a, const float* b, float* c, int M, int N
     return true;
 }
 
-// batch >= 1 independent products packed back to back, or (splits > 1, batch
-// must be 1) one product whose K range is cut into `splits` equal slices,
-// slice s writing its partial sum to c + s*M*N.
-int32_t dispatch(const float* a, const float* b, float* c, int M, int N, int K, int batch,
-                 int ta, int tb, int splits) {
+// Rough time, in us, of a product or batch on the LDS-staged kernels or the
+// skinny ones (gemv.hip), where these leave CUs idle: up to a 64 x 64 tile per
+// CU.  The wave tiles of gemm_f32_direct.hip take it where they are expected
+// at least 5% under that.  0: more tiles than that, never the wave tiles
+// (1000^3 24.9 us staged, 24.5 on wave tiles; 1500^3 79 against 88-102).
+// Measured, staged -> wave tiles: 300^3 8.5 -> 4.8 us, 784 x 500 x 1000 21.4
+// -> 14.2, 1001^3 (copies of misaligned operands) 33 -> 24.7, 128^2 x 4000 73
+// -> 7.5, 100^2 x 5000 23.9 -> 7.7, 32 x 300^2 (skinny) 11.4 -> 5.0; staged
+// stays for 512^3 (6.0 against 6.3), 1500 x 500^2 (13.2 against 15.0), 784 x
+// 256 x 4096 (24.9 against 26.3).
+double est_staged_us(const float* a, const float* b, int M, int N, int K, int batch, int ta, int tb) {
+    const int64_t cus = ch::num_cus() > 0 ? ch::num_cus() : 1;
+    const int64_t tiles = (int64_t)((M + 63) / 64) * ((N + 63) / 64) * batch;
+    const double flops = 2.0 * M * N * K * batch;
+    if (tiles > cus) return 0.0;
+    const bool base16 = (((uintptr_t)a | (uintptr_t)b) & 15) == 0;
+    const int64_t tiles32 = (int64_t)(M / 32) * (N / 32) * batch;
+    if (M % 64 == 0 && N % 64 == 0 && batch == 1 && split_count(M, N, K) > 1) return 0.0;  // K slices fill the chip
+    // the small kernel's shapes: level with the wave tiles (256^3 5.4 against 5.1-5.4 us)
+    if (base16 && tiles32 <= 2 * cus && ch::F32Small::fits(M, N, K, ta ? M : K, tb ? K : N, !ta, tb)) return 0.0;
+    if ((M <= 32 || N <= 32) && flops >= kSkinnyMinFlops)
+        return 8.0 + 4.0 * batch * ((double)M * K + (double)K * N) / 5.0e6;
+    if (flops < kPadMinFlops) return 6.0;
+    // 64 x 64 tiles, one launch, or K slices of a ragged product (try_edge_slices)
+    double us = K * kEdgeTileKUs;
+    if (batch == 1 && (M % 64 || N % 64))
+        for (int s = 2; s <= 64 && K / s >= 512; ++s) {
+            const double t = (double)((tiles * s + cus - 1) / cus) * slice_depth(K, s) * kEdgeTileKUs + 4.0 +
+                             8.0 * s * (double)M * N / 5.0e6;
+            if (t < us) us = t;
+        }
+    const bool rows16 = base16 && (ta ? M : K) % 4 == 0 && (tb ? K : N) % 4 == 0;
+    // misaligned rows: aligned copies first, a launch and both operands read and written at 4 TB/s
+    return 4.0 + us + (rows16 ? 0.0 : 4.5 + 8.0 * batch * ((double)M * K + (double)K * N) / 4.0e6);
+}
+
+// batch >= 1 independent products packed back to back.
+int32_t dispatch(const float* a, const float* b, float* c, int M, int N, int K, int batch, int ta, int tb) {
     // a dimension of 1: matrix-vector or outer products (gemv.hip)
-    if (splits <= 1 && (M == 1 || N == 1 || K == 1)) return ch::matmul_vector_f32(a, b, c, M, N, K, batch, ta, tb);
-    const int64_t lda = ta ? M : K, ldb = tb ? K : N, ldc = N;
-    if (splits <= 1 && batch == 1) return product(a, b, c, M, N, K, lda, ldb, ta, tb, 0);
-    if (splits <= 1) {
-        int32_t st = CLEAVE_HIP_OK;
-        bool done;
-        if (!ta && !tb) done = try_batched_k_slices<false, false>(a, b, c, M, N, K, batch, &st);
-        else if (!ta && tb) done = try_batched_k_slices<false, true>(a, b, c, M, N, K, batch, &st);
-        else if (ta && !tb) done = try_batched_k_slices<true, false>(a, b, c, M, N, K, batch, &st);
-        else done = try_batched_k_slices<true, true>(a, b, c, M, N, K, batch, &st);
-        if (done) return st;
-    }
-    int64_t sA = (int64_t)M * K, sB = (int64_t)K * N, sC = (int64_t)M * N;
-    int kk = K;
-    if (splits > 1) {
-        kk = K / splits;
-        sA = ta ? (int64_t)kk * lda : kk;
-        sB = tb ? kk : (int64_t)kk * ldb;
-        batch = splits;
-    }
-    if (!ta && !tb) return launch<false, false>(a, b, c, M, N, kk, lda, ldb, ldc, batch, sA, sB, sC);
-    if (!ta && tb) return launch<false, true>(a, b, c, M, N, kk, lda, ldb, ldc, batch, sA, sB, sC);
-    if (ta && !tb) return launch<true, false>(a, b, c, M, N, kk, lda, ldb, ldc, batch, sA, sB, sC);
-    return launch<true, true>(a, b, c, M, N, kk, lda, ldb, ldc, batch, sA, sB, sC);
+    if (M == 1 || N == 1 || K == 1) return ch::matmul_vector_f32(a, b, c, M, N, K, batch, ta, tb);
+    int32_t st = CLEAVE_HIP_OK;
+    const double us = est_staged_us(a, b, M, N, K, batch, ta, tb);
+    if (us > 0.0 && ch::try_direct_f32(a, b, c, M, N, K, batch, ta, tb, 0.95 * us, &st)) return st;
+    const int64_t lda = ta ? M : K, ldb = tb ? K : N;
+    if (batch == 1) return product(a, b, c, M, N, K, lda, ldb, ta, tb, 0);
+    bool done;
+    if (!ta && !tb) done = try_batched_k_slices<false, false>(a, b, c, M, N, K, batch, &st);
+    else if (!ta && tb) done = try_batched_k_slices<false, true>(a, b, c, M, N, K, batch, &st);
+    else if (ta && !tb) done = try_batched_k_slices<true, false>(a, b, c, M, N, K, batch, &st);
+    else done = try_batched_k_slices<true, true>(a, b, c, M, N, K, batch, &st);
+    if (done) return st;
+    return launch_layout(ta, tb, a, b, c, M, N, K, lda, ldb, N, batch, (int64_t)M * K, (int64_t)K * N,
+                         (int64_t)M * N);
 }
 
 }  // namespace
 
 namespace ch {
 // Internal entry used by the MLP step (same kernels, no argument checks).
-// splits > 1 requires K % splits == 0 and c sized splits*M*N.
-int32_t gemm_f32_device(const float* a, const float* b, float* c, int M, int N, int K, int ta,
-                        int tb, int splits) {
-    return dispatch(a, b, c, M, N, K, 1, ta, tb, splits);
+int32_t gemm_f32_device(const float* a, const float* b, float* c, int M, int N, int K, int ta, int tb) {
+    return dispatch(a, b, c, M, N, K, 1, ta, tb);
 }
 }  // namespace ch
 
@@ -888,7 +910,7 @@ int32_t cleave_hip_matmul_f32(const float* a, int64_t alen, const float* b, int6
     CH_DEVICE("cleave_hip_matmul_f32", a, alen * 4);
     CH_DEVICE("cleave_hip_matmul_f32", b, blen * 4);
     CH_DEVICE("cleave_hip_matmul_f32", c, clen * 4);
-    return dispatch(a, b, c, M, N, K, 1, trans_a, trans_b, 1);
+    return dispatch(a, b, c, M, N, K, 1, trans_a, trans_b);
 }
 
 int32_t cleave_hip_matmul_batched_f32(const float* a, int64_t alen, const float* b,
@@ -907,7 +929,7 @@ int32_t cleave_hip_matmul_batched_f32(const float* a, int64_t alen, const float*
     CH_DEVICE("cleave_hip_matmul_batched_f32", a, alen * 4);
     CH_DEVICE("cleave_hip_matmul_batched_f32", b, blen * 4);
     CH_DEVICE("cleave_hip_matmul_batched_f32", c, clen * 4);
-    return dispatch(a, b, c, M, N, K, batch, trans_a, trans_b, 1);
+    return dispatch(a, b, c, M, N, K, batch, trans_a, trans_b);
 }
 
 }  // extern "C"

@@ -64,7 +64,7 @@ template <int BM, int BN, int BK, int WM, int WN, int STAGES, bool AKC, bool BKC
 __global__ __launch_bounds__(64 * WM * WN) void gemm_f32_tiled_kernel(
     const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C, int M, int N,
     int K, int64_t lda, int64_t ldb, int64_t strideA, int64_t strideB, int64_t strideC, int tiles_m,
-    int tiles_n, int batch) {
+    int tiles_n, int batch, int ktotal) {
     using namespace ch::tiles;
     using P = F32Tiled<BM, BN, BK, WM, WN, STAGES, AKC, BKC>;
     constexpr int FM = P::FM, FN = P::FN, NW = P::NW;
@@ -76,6 +76,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_f32_tiled_kernel(
     int bt, tm, tn;  // product (batch entry or K-slice) and tile of this workgroup
     ch::block_coords(blockIdx.x, tiles_m, tiles_n, batch, bt, tm, tn);
     const int m0 = tm * BM, n0 = tn * BN;
+    if constexpr (EDGE)
+        if (ktotal > 0) K = min(K, ktotal - bt * K);  // the last K slice may be shorter
     A += (int64_t)bt * strideA;
     B += (int64_t)bt * strideB;
     C += (int64_t)bt * strideC;

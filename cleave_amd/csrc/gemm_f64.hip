@@ -310,6 +310,7 @@ Plan choose_tile(const Args& g, bool both_k) {
         const int tm = 16 * t.fm * (t.wk == 1 ? 2 : 1), tn = 16 * t.fn * (t.wk == 1 ? 2 : 1);
         const int64_t tiles = tile_count(g, tm, tn);
         if (tiles > 0x7FFFFFFF) continue;  // the 128 x 128 tiles' count is checked by the caller
+        double last = 1e300;
         for (const int s : kSlices) {
             // slices of at least 128, at most 16 workgroups a CU, a counter per tile
             if (s > 1 && (t.wk == 1 || g.K / s < 128 || tiles * s > 16 * (int64_t)cus || tiles > kCounters)) break;
@@ -320,6 +321,8 @@ Plan choose_tile(const Args& g, bool both_k) {
             const double us = t.base + (busy > chain ? busy : chain) +
                               (s > 1 ? 3.0 + (double)(tiles * s) * tm * tn * 16.0 / 3e6 : 0.0);
             if (us < best_us) best_us = us, best.tile = i, best.slices = s;
+            if (us > last) break;  // more slices only add to the fold
+            last = us;
         }
     }
     return best;

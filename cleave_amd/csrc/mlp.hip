@@ -13,15 +13,14 @@
 //   2. per row: H = sigmoid(X W1), z2 = H W2, yhat, e, e*e,
 //      d2 = (e+e)/B * yhat(1-yhat), d1 = (d2 W2) h(1-h) over X W1, and
 //      partial sums of h*d2 and e*e     mlp_rows_kernel
-//   3. dW1 partials = X^T d1            gemm_f32 TN, split-K slices
-//   4. dW1, dW2 = sums of partials; W1 -= lr dW1, W2 -= lr dW2;
+//   3. dW1 = X^T d1                     gemm_f32 TN
+//   4. dW2 = sum of partials; W1 -= lr dW1, W2 -= lr dW2;
 //      loss = sum(e*e) / B              mlp_finish_kernel
 #include "common.hpp"
 #include "gemm_f32_pingpong.hpp"
 
 namespace ch {
-int32_t gemm_f32_device(const float* a, const float* b, float* c, int M, int N, int K, int ta,
-                        int tb, int splits);
+int32_t gemm_f32_device(const float* a, const float* b, float* c, int M, int N, int K, int ta, int tb);
 }
 
 namespace {
@@ -271,16 +270,16 @@ int32_t run_rows(float* H, float* D1, const float* W2, const float* v, int B, in
     return CLEAVE_HIP_OK;
 }
 
-// Step 4: workgroups [0, blocks1) sum the dW1 slices and update W1; the next
+// Step 4: workgroups [0, blocks1) update W1; the next
 // ceil(Hd / kFoldCols) sum the dW2 partials (kFoldLanes threads a column, each its
 // run of them in order, then the runs in order) and update W2; the last one, if
 // there is a loss to write, sums the squared errors.  A null dw or w is left out.
 constexpr int kFoldCols = 16, kFoldLanes = kThreads / kFoldCols;
 struct Finish {
-    const float* part1;  // slices x n1
-    int slices, blocks1;
+    const float* g1;  // dW1
+    int blocks1;
     int64_t n1;
-    float *dw1, *w1;
+    float* w1;
     const float* part2;  // groups x Hd
     int groups, Hd;
     float *dw2, *w2;
@@ -298,9 +297,7 @@ __global__ __launch_bounds__(kThreads) void mlp_finish_kernel(Finish f) {
     };
     if ((int)blockIdx.x < f.blocks1) {
         for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < f.n1; i += (int64_t)f.blocks1 * kThreads) {
-            float g = f.part1[i];
-            for (int s = 1; s < f.slices; ++s) g += f.part1[(int64_t)s * f.n1 + i];
-            update(g, f.dw1, f.w1, i);
+            f.w1[i] = f.w1[i] - f.lr * f.g1[i];
         }
         return;
     }
@@ -413,14 +410,6 @@ unsigned capped_grid(int64_t n) {
     return (unsigned)(want < 1 ? 1 : want);
 }
 
-// Split count for X^T d1: enough workgroups to fill the chip, K divisible.
-int choose_splits(int D, int Hd, int B) {
-    const int tiles = ((D + 127) / 128) * ((Hd + 127) / 128);
-    int splits = 1;
-    while (splits < 16 && tiles * splits < 4 * ch::num_cus() && B % (splits * 2 * 16) == 0) splits *= 2;
-    return splits;
-}
-
 // ---- fused path (shapes that divide the 256 x 256 x 16 f32 tile) -----------
 //   1. H = sigmoid(X W1) and partials of H W2      f32 ping-pong GEMM, MODE 1
 //   2. z2, yhat, e, sq, d2 per row; loss           row_finish, loss kernels
@@ -529,7 +518,7 @@ int32_t hidden_fwd(const float* x, const float* w1, const float* w2, float* h, f
         CH_LAUNCHED("z_finish_kernel");
         return CLEAVE_HIP_OK;
     }
-    int32_t rc = ch::gemm_f32_device(x, w1, h, B, Hd, D, 0, 0, 1);
+    int32_t rc = ch::gemm_f32_device(x, w1, h, B, Hd, D, 0, 0);
     if (rc != CLEAVE_HIP_OK) return rc;
     return run_rows<Rows::kFwd>(h, nullptr, w2, nullptr, B, Hd, nullptr, nullptr, z, st);
 }
@@ -564,24 +553,18 @@ int32_t hidden_bwd(const float* x, const float* h, const float* w2, const float*
         }
         return CLEAVE_HIP_OK;
     }
-    const int splits = dw1 ? choose_splits(D, Hd, B) : 0;
     const int groups = row_groups(B, Hd);
-    const size_t nH = (size_t)B * Hd, nPart = (size_t)groups * Hd, nSl = splits > 1 ? (size_t)splits * D * Hd : 0;
-    float* d1 = (float*)ch::scratch(4, sizeof(float) * (up(nH) + up(nPart) + up(nSl)));
+    const size_t nH = (size_t)B * Hd, nPart = (size_t)groups * Hd;
+    float* d1 = (float*)ch::scratch(4, sizeof(float) * (up(nH) + up(nPart)));
     if (!d1) return CLEAVE_HIP_ERR_OOM;
     float* part = d1 + up(nH);
-    float* slices = splits > 1 ? part + up(nPart) : dw1;
     int32_t rc = run_rows<Rows::kBwd>(const_cast<float*>(h), d1, w2, g, B, Hd, part, nullptr, nullptr, st);
     if (rc != CLEAVE_HIP_OK) return rc;
     if (dw1) {
-        rc = ch::gemm_f32_device(x, d1, slices, D, Hd, B, 1, 0, splits);
+        rc = ch::gemm_f32_device(x, d1, dw1, D, Hd, B, 1, 0);
         if (rc != CLEAVE_HIP_OK) return rc;
     }
     Finish f{};
-    if (splits > 1) {
-        f.part1 = slices, f.slices = splits, f.n1 = (int64_t)D * Hd, f.blocks1 = (int)capped_grid(f.n1);
-        f.dw1 = dw1;
-    }
     if (dw2) f.part2 = part, f.groups = groups, f.Hd = Hd, f.dw2 = dw2;
     if (finish_grid(f) == 0) return CLEAVE_HIP_OK;
     mlp_finish_kernel<<<finish_grid(f), kThreads, 0, st>>>(f);
@@ -618,26 +601,25 @@ extern "C" int32_t cleave_hip_mlp_step_f32(const float* x, int64_t xlen, const f
     hipStream_t st = ch::stream();
     if (fused_fits(x, w1, B, D, Hd)) return fused_step(x, y, w1, w2, dw1, dw2, loss_dev, B, D, Hd, lr, st);
 
-    const int splits = choose_splits(D, Hd, B);
     const int groups = row_groups(B, Hd);
-    // Scratch slot 4: H/d1 | dW2 partials | squared errors | dW1 slices.
-    const size_t nH = (size_t)B * Hd, nPart = (size_t)groups * Hd, nSl = (size_t)splits * D * Hd;
+    // Scratch slot 4: H/d1 | dW2 partials | squared errors | dW1 if not asked for.
+    const size_t nH = (size_t)B * Hd, nPart = (size_t)groups * Hd, nG = dw1 ? 0 : (size_t)D * Hd;
     auto up = [](size_t n) { return (n + 63) & ~(size_t)63; };
-    float* H = (float*)ch::scratch(4, sizeof(float) * (up(nH) + up(nPart) + up(groups) + up(nSl)));
+    float* H = (float*)ch::scratch(4, sizeof(float) * (up(nH) + up(nPart) + up(groups) + up(nG)));
     if (!H) return CLEAVE_HIP_ERR_OOM;
     float* part = H + up(nH);
     float* sq = part + up(nPart);
-    float* slices = splits > 1 || !dw1 ? sq + up(groups) : dw1;
+    float* g1 = dw1 ? dw1 : sq + up(groups);
 
-    int32_t rc = ch::gemm_f32_device(x, w1, H, B, Hd, D, 0, 0, 1);
+    int32_t rc = ch::gemm_f32_device(x, w1, H, B, Hd, D, 0, 0);
     if (rc != CLEAVE_HIP_OK) return rc;
     rc = run_rows<Rows::kStep>(H, nullptr, w2, y, B, Hd, part, sq, nullptr, st);
     if (rc != CLEAVE_HIP_OK) return rc;
-    rc = ch::gemm_f32_device(x, H, slices, D, Hd, B, 1, 0, splits);
+    rc = ch::gemm_f32_device(x, H, g1, D, Hd, B, 1, 0);
     if (rc != CLEAVE_HIP_OK) return rc;
     Finish f{};
-    f.part1 = slices, f.slices = splits, f.n1 = (int64_t)D * Hd, f.blocks1 = (int)capped_grid(f.n1);
-    f.dw1 = slices == dw1 ? nullptr : dw1, f.w1 = w1;
+    f.g1 = g1, f.n1 = (int64_t)D * Hd, f.blocks1 = lr != 0.0f ? (int)capped_grid(f.n1) : 0;
+    f.w1 = w1;
     f.part2 = part, f.groups = groups, f.Hd = Hd, f.dw2 = dw2, f.w2 = w2;
     f.sqpart = sq, f.loss = loss_dev, f.count = (float)B, f.lr = lr;
     mlp_finish_kernel<<<finish_grid(f), kThreads, 0, st>>>(f);

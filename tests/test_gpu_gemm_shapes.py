@@ -143,3 +143,49 @@ def test_batched_shape_every_entry(hip, oracle, dtype, bsz, M, N, K, ta, tb):
         else:
             den = np.abs(Ak).astype(np.float64) @ np.abs(Bk).astype(np.float64).T
             assert_gemm_close(got[i], ref, den, K, f"{dtype} batch {i}/{bsz} {M}x{N}x{K} ta={ta} tb={tb}")
+
+
+# f32 products with few tiles: every wave tile of the unstaged kernel (16 x 16, 32 x 32,
+# 64 x 32 and its turn, 64 x 64) with and without K slices, operands narrower than a tile,
+# misaligned rows, batches; and K slices of uneven depth on the staged tiles.  Whole-number
+# operands under 2^24 in every sum, so that each order gives the exact product.
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("batch,M,N,K", [
+    (1, 2, 2, 2), (1, 3, 5, 7), (1, 17, 33, 15), (1, 50, 70, 20), (1, 300, 300, 300), (1, 2, 300, 513),
+    (1, 300, 3, 1025), (1, 32, 301, 300), (1, 100, 100, 5000), (1, 64, 64, 10000), (1, 129, 127, 4001),
+    (1, 333, 301, 1000), (1, 784, 300, 1000), (1, 699, 701, 700), (1, 1001, 1001, 999), (1, 1000, 300, 784),
+    (16, 99, 101, 100), (64, 65, 33, 100), (40, 33, 50, 2000), (5, 3, 2, 9000),
+    (1, 784, 500, 10000), (1, 1000, 300, 5004), (1, 2500, 640, 4100), (1, 500, 500, 7777), (1, 1100, 1030, 5000)])
+def test_few_tiles_exact(hip, batch, M, N, K, ta, tb):
+    rng = np.random.default_rng(M * 7 + N * 3 + K + 11 * ta + tb)
+    A = rng.integers(-9, 10, (batch, K, M) if ta else (batch, M, K)).astype(np.float32)
+    B = rng.integers(-9, 10, (batch, N, K) if tb else (batch, K, N)).astype(np.float32)
+    want = (A.transpose(0, 2, 1) if ta else A).astype(np.float64) @ (B.transpose(0, 2, 1) if tb else B)
+    a, b = hip.from_numpy(A), hip.from_numpy(B)
+    if batch > 1:
+        got = hip.matmul_batched(a, b, trans_a=bool(ta), trans_b=bool(tb)).numpy()
+    else:
+        c = hip.from_numpy(np.full((M, N), np.nan, np.float32))
+        hip.matmul(a.view(A.shape[1:]), b.view(B.shape[1:]), trans_a=bool(ta), trans_b=bool(tb), out=c)
+        got = c.numpy()[None]
+    assert np.array_equal(got, want)
+    if batch == 1:  # views one element in: rows and bases aligned to 4 bytes only
+        a1, b1, c1 = (hip.from_numpy(np.concatenate([np.zeros(1, np.float32), v.reshape(-1)]))
+                      for v in (A, B, np.full((M, N), np.nan, np.float32)))
+        c1 = c1.sub(1, (M, N))
+        hip.matmul(a1.sub(1, A.shape[1:]), b1.sub(1, B.shape[1:]), trans_a=bool(ta), trans_b=bool(tb), out=c1)
+        assert np.array_equal(c1.numpy(), want[0])
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K", [(37, 50, 19), (301, 45, 1003), (20, 3, 2003)])
+def test_few_tiles_keep_nan_and_inf_where_they_belong(hip, M, N, K, ta, tb):
+    A, B = np.ones((M, K), np.float32), np.ones((K, N), np.float32)
+    A[5, K - 1], A[M - 1, 0], B[0, 2] = np.nan, -np.inf, np.inf
+    with np.errstate(invalid="ignore"):
+        want = A.astype(np.float64) @ B
+    got = hip.matmul(hip.from_numpy(np.ascontiguousarray(A.T if ta else A)),
+                     hip.from_numpy(np.ascontiguousarray(B.T if tb else B)), trans_a=bool(ta),
+                     trans_b=bool(tb)).numpy()
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[~np.isnan(got)], want[~np.isnan(want)])
