@@ -62,6 +62,11 @@ inline int64_t count3(int64_t a, int64_t b, int64_t c) {
 constexpr int kNoAllocFloats = 16384;  // 64 KiB
 float* noalloc_workspace();
 
+// A pinned host word (64 bytes) that kernels write and a host-returning call
+// reads after synchronising the stream; nullptr (with the error recorded) when
+// it cannot be allocated.  Allocated once and kept.
+void* host_word();
+
 // Tensor operands of the device entry points must be device memory: a host
 // address handed to a kernel faults the GPU.  Fails with CLEAVE_HIP_ERR_ARG
 // when `p` is not device (or managed) memory of this process, or when its

@@ -76,4 +76,18 @@ __device__ __forceinline__ bool last_block(uint32_t* counter, uint32_t total) {
     return true;
 }
 
+// The same for up to kTreeGroups * kTreeArity workgroups of a 1-D grid (all of
+// it): arrivals at one address are served one after the other, about 10 ns
+// each (a thousand took 10 us), so workgroups arrive in groups of kTreeArity
+// at counters a cache line apart, and the groups' last ones at the root.
+// `counters`: kTreeWords words.
+constexpr unsigned kTreeArity = 32, kTreeGroups = 64, kTreeWords = 32 * (kTreeGroups + 1);
+__device__ __forceinline__ bool last_block_tree(uint32_t* counters) {
+    const unsigned group = blockIdx.x / kTreeArity, groups = (gridDim.x + kTreeArity - 1) / kTreeArity;
+    const unsigned left = gridDim.x - group * kTreeArity;
+    if (!last_block(counters + 32 * (group + 1), left < kTreeArity ? left : kTreeArity)) return false;
+    __syncthreads();  // the first arrival's word in LDS is read by all before the next
+    return last_block(counters, groups);
+}
+
 }  // namespace ch

@@ -2,11 +2,15 @@
 // u64 sum of u32 escape counts, and the exact i64 sum of i32 arrays (the
 // same counts as cleave's i32 type carries them).
 //
-// Two stages, both deterministic for a given length: stage 1 runs a fixed
-// grid (a function of the length and the CU count only); each thread folds
-// 16-byte vectors in registers, the wave combines lanes with cross-lane
-// shuffles, LDS carries the 4 wave results to one block result.  Stage 2 is
-// one block over the block results.
+// One launch, deterministic for a given length and device: each workgroup of a
+// fixed grid folds its run of the array's 16-byte vectors in registers, the
+// wave combines lanes with cross-lane shuffles, LDS carries the 4 wave results
+// to one, and the workgroup that arrives last folds the workgroups' results in
+// their order (last_block.hpp).  HBM-bound from a few MB; below that, latency.
+// The host-returning forms have the kernel write the result into pinned host
+// memory.  With a second launch for the fold and a copy of the result, a Mean of
+// 10^6 f32 took 26.7 us, now 17; Mean, Max and argmax of 10^7 together 96, now 71.
+// Queued sums from 10^7 elements on are level (10^7 10.2 us, 2^28 159).
 //
 // Max semantics: the reference folds acc = v[0]; if v[i] > acc then acc = v[i]
 // (cmpf ogt, stdlib/num/num.cleave:303).  A NaN at i > 0 never wins; a NaN at
@@ -14,26 +18,40 @@
 // the largest non-NaN value, which is associative as (value desc, index asc)
 // -- that is what the tree combines (-0 and +0 compare equal, so the earlier
 // one is kept, as in the fold).
+#include <algorithm>
 #include <cfloat>
 
 #include "common.hpp"
+#include "last_block.hpp"
 
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kUnroll = 4;
+constexpr int kUnroll = 8;
+// Workgroups of the running reduction that have arrived, 0 between launches; the
+// allocation-free Sum has its own, as it has its own workspace.
+static __device__ uint32_t g_arrived[2][ch::kTreeWords];
 
 // Native clang vectors (register-promoted; HIP's float4/uint4 structs are not
-// always) loaded with non-temporal hints: the data is streamed once.
+// always).  Loads are non-temporal: the data is read once.
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 
-// Stage-1 grid: enough blocks for 16 per CU (a function of the length and the
-// CU count only, so results are reproducible on a given device).
-unsigned stage1_blocks(int64_t nvec) {
-    int64_t want = (nvec + (int64_t)kThreads * kUnroll - 1) / ((int64_t)kThreads * kUnroll);
-    int64_t cap = (int64_t)ch::num_cus() * 16;
-    if (want > cap) want = cap;
-    return (unsigned)(want < 1 ? 1 : want);
+// The array as rows of kThreads vectors; workgroup b of G takes rows
+// [R b / G, R (b + 1) / G), so that none has more than one row over another, and up
+// to four workgroups a CU keep 128 KiB a CU in flight.  (Rows b, b + G, ... instead
+// took 207 us at 2^28 f32 against 159; eight workgroups a CU 167.)
+struct Rows {
+    int64_t begin, end;
+};
+__device__ __forceinline__ Rows my_rows(int64_t nvec) {
+    const int64_t rows = (nvec + kThreads - 1) / kThreads;
+    return {rows * blockIdx.x / gridDim.x, rows * (blockIdx.x + 1) / gridDim.x};
+}
+unsigned row_blocks(int64_t nvec) {
+    const int64_t rows = (nvec + kThreads - 1) / kThreads, want = (rows + 3) / 4;
+    const int64_t most = ch::kTreeArity * ch::kTreeGroups;  // of the arrival tree
+    const int64_t cap = std::min<int64_t>(4 * (int64_t)ch::num_cus(), most);
+    return (unsigned)(want < 1 ? 1 : want < cap ? want : cap);
 }
 
 // ---- sum f32 / f64 ------------------------------------------------------------
@@ -55,6 +73,7 @@ template <class T>
 __device__ T block_sum(T v) {
     __shared__ T part[kThreads / 64];
     v = wave_sum(v);
+    __syncthreads();  // the last use's reads of part
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
     __syncthreads();
     T r = T(0);
@@ -63,64 +82,77 @@ __device__ T block_sum(T v) {
     return r;  // valid in thread 0
 }
 
+// Calls fold(vector, vector index) for this workgroup's vectors in ascending order
+// per thread, kUnroll loads in flight.
+template <class VT, class Fold>
+__device__ __forceinline__ void fold_rows(const void* x, int64_t nvec, Fold fold) {
+    const VT* p = reinterpret_cast<const VT*>(x);
+    const Rows r = my_rows(nvec);
+    for (int64_t row = r.begin; row < r.end; row += kUnroll) {
+        VT v[kUnroll];
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) {
+            const int64_t i = (row + u) * kThreads + threadIdx.x;
+            if (row + u < r.end && i < nvec) {
+                v[u] = __builtin_nontemporal_load(p + i);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) {
+            const int64_t i = (row + u) * kThreads + threadIdx.x;
+            if (row + u < r.end && i < nvec) fold(v[u], i);
+        }
+    }
+}
+
+// The last workgroup's partials t, t + 256, ... of thread t in that order, all
+// loads of a run of kFoldLoads in flight together.
+constexpr int kFoldLoads = 4;
+template <class U, class Fold>
+__device__ __forceinline__ void fold_partials(const U* partial, Fold fold) {
+    const int n = (int)gridDim.x;
+    for (int i0 = threadIdx.x; i0 < n; i0 += kThreads * kFoldLoads) {
+        U v[kFoldLoads];
+#pragma unroll
+        for (int u = 0; u < kFoldLoads; ++u) v[u] = ch::fetch(partial + min(i0 + u * kThreads, n - 1));
+#pragma unroll
+        for (int u = 0; u < kFoldLoads; ++u)
+            if (i0 + u * kThreads < n) fold(v[u]);
+    }
+}
+
 // Each lane keeps one accumulator per vector element and adds them in a
 // fixed tree at the end: (a0 + a1) + (a2 + a3) for f32, a0 + a1 for f64.
 template <class T>
-__global__ __launch_bounds__(kThreads) void sum_stage1(const T* __restrict__ x, int64_t n, T* __restrict__ partial,
-                                                       int aligned) {
+__global__ __launch_bounds__(kThreads) void sum_kernel(const T* __restrict__ x, int64_t n, T* partial,
+                                                       T* __restrict__ out, int aligned, int counter) {
     constexpr int V = Vec16<T>::kN;
     typedef typename Vec16<T>::type VT;
     T acc[V];
 #pragma unroll
     for (int e = 0; e < V; ++e) acc[e] = T(0);
     if (aligned) {
-        const int64_t nv = n / V;
-        const int64_t step = (int64_t)gridDim.x * kThreads * kUnroll;
-        for (int64_t base = (int64_t)blockIdx.x * kThreads * kUnroll + threadIdx.x; base < nv; base += step) {
-            VT v[kUnroll];
+        fold_rows<VT>(x, n / V, [&](VT v, int64_t) {
 #pragma unroll
-            for (int u = 0; u < kUnroll; ++u) {
-                int64_t i = base + (int64_t)u * kThreads;
-                v[u] = i < nv ? __builtin_nontemporal_load(reinterpret_cast<const VT*>(x) + i) : VT(T(0));
-            }
-#pragma unroll
-            for (int u = 0; u < kUnroll; ++u)
-#pragma unroll
-                for (int e = 0; e < V; ++e) acc[e] += v[u][e];
-        }
-        if (blockIdx.x == 0 && threadIdx.x < (n % V)) acc[0] += x[nv * V + threadIdx.x];
+            for (int e = 0; e < V; ++e) acc[e] += v[e];
+        });
+        if (blockIdx.x == 0 && threadIdx.x < (n % V)) acc[0] += x[n / V * V + threadIdx.x];
     } else {
-        for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kThreads)
-            acc[0] += x[i];
+        fold_rows<T>(x, n, [&](T v, int64_t) { acc[0] += v; });
     }
     T lane;
     if constexpr (V == 4) lane = (acc[0] + acc[1]) + (acc[2] + acc[3]);
     else lane = acc[0] + acc[1];
     T r = block_sum(lane);
-    if (threadIdx.x == 0) partial[blockIdx.x] = r;
-}
-
-// Stage 2 folds thread t's partials t, t + 256, ... in that order.  The
-// loads of a run of kStage2Loads go out together before the adds: one memory
-// latency per run instead of one per partial (5.2 us -> ~1.5 us for 4096
-// partials; the order, and so the result, is unchanged).
-constexpr int kStage2Loads = 16;
-
-template <class T>
-__global__ __launch_bounds__(kThreads) void sum_stage2(const T* __restrict__ partial, int nparts, T* __restrict__ out) {
-    T acc = T(0);
-    for (int i0 = threadIdx.x; i0 < nparts; i0 += kThreads * kStage2Loads) {
-        T v[kStage2Loads];
-#pragma unroll
-        for (int u = 0; u < kStage2Loads; ++u) {
-            const int i = i0 + u * kThreads;
-            v[u] = i < nparts ? partial[i] : T(0);
-        }
-#pragma unroll
-        for (int u = 0; u < kStage2Loads; ++u)
-            if (i0 + u * kThreads < nparts) acc += v[u];
+    if (gridDim.x == 1) {
+        if (threadIdx.x == 0) *out = r;
+        return;
     }
-    T r = block_sum(acc);
+    if (threadIdx.x == 0) ch::publish(partial + blockIdx.x, r);
+    if (!ch::last_block_tree(g_arrived[counter])) return;
+    T total = T(0);
+    fold_partials(partial, [&](T v) { total += v; });
+    r = block_sum(total);
     if (threadIdx.x == 0) *out = r;
 }
 
@@ -153,6 +185,7 @@ __device__ Best<T> block_best(Best<T> b) {
     __shared__ T pv[kThreads / 64];
     __shared__ int64_t pi[kThreads / 64];
     b = wave_best(b);
+    __syncthreads();  // the last use's reads of pv, pi
     if ((threadIdx.x & 63) == 0) {
         pv[threadIdx.x >> 6] = b.v;
         pi[threadIdx.x >> 6] = b.i;
@@ -164,68 +197,72 @@ __device__ Best<T> block_best(Best<T> b) {
     return r;
 }
 
+// A thread meets its vectors in ascending order, so in one of its element
+// slots a later value replaces the best only if it is greater: a compare and
+// two selects an element, where the full rule takes seven operations.
+// -infinity never replaces the initial one; if nothing else is there the
+// fold's own answer, v[0], is taken at the end.
 template <class T>
-__global__ __launch_bounds__(kThreads) void max_stage1(const T* __restrict__ x, int64_t n, T* __restrict__ pv,
-                                                       int64_t* __restrict__ pi, int aligned) {
+__global__ __launch_bounds__(kThreads) void max_kernel(const T* __restrict__ x, int64_t n, T* pv, int64_t* pi,
+                                                       T* __restrict__ out_v, int64_t* __restrict__ out_i,
+                                                       int aligned) {
     constexpr int V = Vec16<T>::kN;
     typedef typename Vec16<T>::type VT;
+    constexpr uint32_t kNone = 0xFFFFFFFFu;
+    T bv[V];
+    uint32_t bk[V];  // how many vectors the thread had met
+    uint32_t met = 0;
+#pragma unroll
+    for (int e = 0; e < V; ++e) bv[e] = T(-INFINITY), bk[e] = kNone;
     Best<T> b{-INFINITY, INT64_MAX};
+    const int64_t first = my_rows(aligned ? n / V : n).begin * kThreads + threadIdx.x;
+    auto index = [&](uint32_t k) { return first + (int64_t)k * kThreads; };  // of the vector
     if (aligned) {
-        const int64_t nv = n / V;
-        const int64_t step = (int64_t)gridDim.x * kThreads * kUnroll;
-        for (int64_t base = (int64_t)blockIdx.x * kThreads * kUnroll + threadIdx.x; base < nv; base += step) {
-            VT v[kUnroll];
+        fold_rows<VT>(x, n / V, [&](VT v, int64_t) {
 #pragma unroll
-            for (int u = 0; u < kUnroll; ++u) {
-                int64_t i = base + (int64_t)u * kThreads;
-                if (i < nv) v[u] = __builtin_nontemporal_load(reinterpret_cast<const VT*>(x) + i);
-            }
+            for (int e = 0; e < V; ++e)
+                if (v[e] > bv[e]) bv[e] = v[e], bk[e] = met;
+            ++met;
+        });
 #pragma unroll
-            for (int u = 0; u < kUnroll; ++u) {
-                int64_t i = base + (int64_t)u * kThreads;
-                if (i < nv) {
-#pragma unroll
-                    for (int e = 0; e < V; ++e) take_better(b, v[u][e], V * i + e);
-                }
-            }
-        }
-        if (blockIdx.x == 0 && threadIdx.x < (n % V)) take_better(b, x[nv * V + threadIdx.x], nv * V + threadIdx.x);
+        for (int e = 0; e < V; ++e)
+            if (bk[e] != kNone) take_better(b, bv[e], V * index(bk[e]) + e);
+        if (blockIdx.x == 0 && threadIdx.x < (n % V)) take_better(b, x[n / V * V + threadIdx.x], n / V * V + threadIdx.x);
     } else {
-        for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kThreads)
-            take_better(b, x[i], i);
+        fold_rows<T>(x, n, [&](T v, int64_t) {
+            if (v > bv[0]) bv[0] = v, bk[0] = met;
+            ++met;
+        });
+        if (bk[0] != kNone) take_better(b, bv[0], index(bk[0]));
     }
     Best<T> r = block_best(b);
-    if (threadIdx.x == 0) {
-        pv[blockIdx.x] = r.v;
-        pi[blockIdx.x] = r.i;
-    }
-}
-
-template <class T>
-__global__ __launch_bounds__(kThreads) void max_stage2(const T* __restrict__ x, const T* __restrict__ pv,
-                                                       const int64_t* __restrict__ pi, int nparts,
-                                                       T* __restrict__ out_v, int64_t* __restrict__ out_i) {
-    Best<T> b{-INFINITY, INT64_MAX};
-    for (int i0 = threadIdx.x; i0 < nparts; i0 += kThreads * kStage2Loads) {
-        T v[kStage2Loads];
-        int64_t ix[kStage2Loads];
-#pragma unroll
-        for (int u = 0; u < kStage2Loads; ++u) {
-            const int i = i0 + u * kThreads;
-            v[u] = i < nparts ? pv[i] : T(-INFINITY);
-            ix[u] = i < nparts ? pi[i] : INT64_MAX;
+    if (gridDim.x > 1) {
+        if (threadIdx.x == 0) {
+            ch::publish(pv + blockIdx.x, r.v);
+            ch::publish(pi + blockIdx.x, r.i);
         }
+        if (!ch::last_block_tree(g_arrived[0])) return;
+        b = Best<T>{-INFINITY, INT64_MAX};
+        const int parts = (int)gridDim.x;
+        for (int i0 = threadIdx.x; i0 < parts; i0 += kThreads * kFoldLoads) {
+            T v[kFoldLoads];
+            int64_t ix[kFoldLoads];
 #pragma unroll
-        for (int u = 0; u < kStage2Loads; ++u)
-            if (i0 + u * kThreads < nparts) take_better(b, v[u], ix[u]);
+            for (int u = 0; u < kFoldLoads; ++u) {
+                const int i = min(i0 + u * kThreads, parts - 1);
+                v[u] = ch::fetch(pv + i);
+                ix[u] = ch::fetch(pi + i);
+            }
+#pragma unroll
+            for (int u = 0; u < kFoldLoads; ++u) take_better(b, v[u], ix[u]);  // the last one again changes nothing
+        }
+        r = block_best(b);
     }
-    Best<T> r = block_best(b);
     if (threadIdx.x == 0) {
         T x0 = x[0];
-        if (x0 != x0) {  // nothing compares > NaN, so the fold keeps a NaN v[0]
-            r.v = x0;
-            r.i = 0;
-        } else if (r.i == INT64_MAX) {  // every other element is NaN
+        // nothing compares > NaN, so the fold keeps a NaN v[0]; and a best of
+        // -infinity means that every other element is NaN or -infinity too
+        if (x0 != x0 || !(r.v > T(-INFINITY))) {
             r.v = x0;
             r.i = 0;
         }
@@ -243,6 +280,7 @@ __device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v) {
 __device__ uint64_t block_sum_u64(uint64_t v) {
     __shared__ uint64_t part[kThreads / 64];
     v = wave_sum_u64(v);
+    __syncthreads();  // the last use's reads of part
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
     __syncthreads();
     uint64_t r = 0;
@@ -252,117 +290,123 @@ __device__ uint64_t block_sum_u64(uint64_t v) {
 }
 
 // Signed: each element is sign-extended to 64 bits, so the u64 total is the
-// two's-complement bits of the exact i64 sum (stage 2 is the same add).
+// two's-complement bits of the exact i64 sum.
 template <bool Signed>
 __device__ __forceinline__ uint64_t widen(uint32_t v) {
     return Signed ? (uint64_t)(int64_t)(int32_t)v : (uint64_t)v;
 }
 
 template <bool Signed>
-__global__ __launch_bounds__(kThreads) void sum_u32_stage1(const uint32_t* __restrict__ x, int64_t n,
-                                                           uint64_t* __restrict__ partial,
+__global__ __launch_bounds__(kThreads) void sum_u32_kernel(const uint32_t* __restrict__ x, int64_t n,
+                                                           uint64_t* partial, uint64_t* __restrict__ out,
                                                            int aligned) {
     uint64_t acc = 0;
     if (aligned) {
-        const int64_t nv = n / 4;
-        const int64_t step = (int64_t)gridDim.x * kThreads * kUnroll;
-        for (int64_t base = (int64_t)blockIdx.x * kThreads * kUnroll + threadIdx.x; base < nv; base += step) {
-            u4 v[kUnroll];
-#pragma unroll
-            for (int u = 0; u < kUnroll; ++u) {
-                int64_t i = base + (int64_t)u * kThreads;
-                v[u] = i < nv ? __builtin_nontemporal_load(reinterpret_cast<const u4*>(x) + i) : u4{0, 0, 0, 0};
-            }
-            // Add in 64 bits (mod 2^64, exact for both forms).
-#pragma unroll
-            for (int u = 0; u < kUnroll; ++u)
-                acc += (widen<Signed>(v[u][0]) + widen<Signed>(v[u][1])) +
-                       (widen<Signed>(v[u][2]) + widen<Signed>(v[u][3]));
-        }
-        if (blockIdx.x == 0 && threadIdx.x < (n & 3)) acc += widen<Signed>(x[nv * 4 + threadIdx.x]);
+        // Add in 64 bits (mod 2^64, exact for both forms).
+        fold_rows<u4>(x, n / 4, [&](u4 v, int64_t) {
+            acc += (widen<Signed>(v[0]) + widen<Signed>(v[1])) + (widen<Signed>(v[2]) + widen<Signed>(v[3]));
+        });
+        if (blockIdx.x == 0 && threadIdx.x < (n & 3)) acc += widen<Signed>(x[n / 4 * 4 + threadIdx.x]);
     } else {
-        for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kThreads)
-            acc += widen<Signed>(x[i]);
+        fold_rows<uint32_t>(x, n, [&](uint32_t v, int64_t) { acc += widen<Signed>(v); });
     }
     uint64_t r = block_sum_u64(acc);
-    if (threadIdx.x == 0) partial[blockIdx.x] = r;
-}
-
-__global__ __launch_bounds__(kThreads) void sum_u64_stage2(const uint64_t* __restrict__ partial,
-                                                           int nparts, uint64_t* __restrict__ out) {
-    uint64_t acc = 0;
-    for (int i0 = threadIdx.x; i0 < nparts; i0 += kThreads * kStage2Loads) {
-        uint64_t v[kStage2Loads];
-#pragma unroll
-        for (int u = 0; u < kStage2Loads; ++u) {
-            const int i = i0 + u * kThreads;
-            v[u] = i < nparts ? partial[i] : 0;
-        }
-#pragma unroll
-        for (int u = 0; u < kStage2Loads; ++u) acc += v[u];
+    if (gridDim.x > 1) {
+        if (threadIdx.x == 0) ch::publish(partial + blockIdx.x, r);
+        if (!ch::last_block_tree(g_arrived[0])) return;
+        uint64_t total = 0;
+        fold_partials(partial, [&](uint64_t v) { total += v; });
+        r = block_sum_u64(total);
     }
-    uint64_t r = block_sum_u64(acc);
     if (threadIdx.x == 0) *out = r;
 }
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
-// Sum into a device scalar: stage-1 partials in scratch slot 0.
+// Queues the sum of x into *out, a word that the device can write; the
+// partials (one of T a workgroup, never more than ch::kNoAllocFloats) in part.
 template <class T>
-int32_t run_reduce_sum(const char* fn, const T* x, int64_t len, T* out_dev) {
+int32_t queue_sum(const T* x, int64_t len, T* part, T* out, int counter) {
     constexpr int V = Vec16<T>::kN;
-    CH_REQUIRE(len >= 1, "%s: length must be >= 1 (sum reads v[0])", fn);
-    CH_REQUIRE(x && out_dev, "%s: null buffer", fn);
-    CH_INIT_OR_RETURN();
-    CH_DEVICE(fn, x, len * sizeof(T));
-    CH_DEVICE(fn, out_dev, sizeof(T));
     const int aligned = aligned16(x);
-    unsigned blocks = stage1_blocks(aligned ? len / V + 1 : len / kUnroll + 1);
-    T* part = (T*)ch::scratch(0, sizeof(T) * blocks);
-    if (!part) return CLEAVE_HIP_ERR_OOM;
-    sum_stage1<T><<<blocks, kThreads, 0, ch::stream()>>>(x, len, part, aligned);
-    CH_LAUNCHED("sum_stage1");
-    sum_stage2<T><<<1, kThreads, 0, ch::stream()>>>(part, (int)blocks, out_dev);
-    CH_LAUNCHED("sum_stage2");
+    const unsigned blocks = row_blocks(aligned ? len / V : len);
+    sum_kernel<T><<<blocks, kThreads, 0, ch::stream()>>>(x, len, part, out, aligned, counter);
+    CH_LAUNCHED("sum_kernel");
     return CLEAVE_HIP_OK;
 }
 
-// max_of / argmax into device scalars: partial indices then values in slot 1.
+// Workspace of the partials of any reduction here: 16 bytes a workgroup.
+char* partials() { return (char*)ch::scratch(0, 16 * 4 * (size_t)ch::num_cus()); }
+
 template <class T>
-int32_t run_reduce_max(const char* fn, const T* x, int64_t len, T* max_dev, int64_t* argmax_dev) {
-    constexpr int V = Vec16<T>::kN;
-    CH_REQUIRE(len >= 1, "%s: length must be >= 1 (max_of reads v[0])", fn);
-    CH_REQUIRE(x && (max_dev || argmax_dev), "%s: null buffer", fn);
+int32_t check_sum(const char* fn, const T* x, int64_t len, const void* out) {
+    CH_REQUIRE(len >= 1, "%s: length must be >= 1 (sum reads v[0])", fn);
+    CH_REQUIRE(x && out, "%s: null buffer", fn);
     CH_INIT_OR_RETURN();
     CH_DEVICE(fn, x, len * sizeof(T));
-    if (max_dev) CH_DEVICE(fn, max_dev, sizeof(T));
-    if (argmax_dev) CH_DEVICE(fn, argmax_dev, 8);
+    return CLEAVE_HIP_OK;
+}
+
+// Sum into a device scalar (out_dev), or into the library's host word.
+template <class T>
+int32_t run_sum(const char* fn, const T* x, int64_t len, T* out, bool host) {
+    int32_t st = check_sum(fn, x, len, out);
+    if (st != CLEAVE_HIP_OK) return st;
+    if (!host) CH_DEVICE(fn, out, sizeof(T));
+    char* part = partials();
+    if (!part) return CLEAVE_HIP_ERR_OOM;
+    return queue_sum<T>(x, len, (T*)part, out, 0);
+}
+
+// max_of / argmax likewise: partial indices, then values.
+template <class T>
+int32_t run_max(const char* fn, const T* x, int64_t len, T* out_max, int64_t* out_argmax, bool host) {
+    constexpr int V = Vec16<T>::kN;
+    CH_REQUIRE(len >= 1, "%s: length must be >= 1 (max_of reads v[0])", fn);
+    CH_REQUIRE(x && (out_max || out_argmax), "%s: null buffer", fn);
+    CH_INIT_OR_RETURN();
+    CH_DEVICE(fn, x, len * sizeof(T));
+    if (!host && out_max) CH_DEVICE(fn, out_max, sizeof(T));
+    if (!host && out_argmax) CH_DEVICE(fn, out_argmax, 8);
     const int aligned = aligned16(x);
-    unsigned blocks = stage1_blocks(aligned ? len / V + 1 : len / kUnroll + 1);
-    char* base = (char*)ch::scratch(1, (sizeof(T) + sizeof(int64_t)) * blocks + 64);
+    const unsigned blocks = row_blocks(aligned ? len / V : len);
+    char* base = partials();
     if (!base) return CLEAVE_HIP_ERR_OOM;
     int64_t* pi = (int64_t*)base;
     T* pv = (T*)(base + sizeof(int64_t) * blocks);
-    max_stage1<T><<<blocks, kThreads, 0, ch::stream()>>>(x, len, pv, pi, aligned);
-    CH_LAUNCHED("max_stage1");
-    max_stage2<T><<<1, kThreads, 0, ch::stream()>>>(x, pv, pi, (int)blocks, max_dev, argmax_dev);
-    CH_LAUNCHED("max_stage2");
+    max_kernel<T><<<blocks, kThreads, 0, ch::stream()>>>(x, len, pv, pi, out_max, out_argmax, aligned);
+    CH_LAUNCHED("max_kernel");
     return CLEAVE_HIP_OK;
 }
 
-// Host-returning forms: queue the reduction into a library-owned device word,
-// then copy it back (synchronising the stream).  `bad` comes back after an
-// error (NaN, or -1 for an index).
+template <bool Signed>
+int32_t run_sum_u32(const char* fn, const uint32_t* x, int64_t len, uint64_t* out, bool host) {
+    CH_REQUIRE(len >= 0, "%s: negative length", fn);
+    CH_REQUIRE(x && out, "%s: null buffer", fn);
+    CH_INIT_OR_RETURN();
+    CH_DEVICE(fn, x, len * 4);
+    if (!host) CH_DEVICE(fn, out, 8);
+    const int aligned = aligned16(x);
+    const unsigned blocks = row_blocks(aligned ? len / 4 : len);
+    uint64_t* part = (uint64_t*)partials();
+    if (!part) return CLEAVE_HIP_ERR_OOM;
+    sum_u32_kernel<Signed><<<blocks, kThreads, 0, ch::stream()>>>(x, len, part, out, aligned);
+    CH_LAUNCHED("sum_u32_kernel");
+    return CLEAVE_HIP_OK;
+}
+
+// Host-returning forms: queue the reduction into a pinned host word of the
+// library, wait for the stream and read it, without a copy of its own.  `bad`
+// comes back after an error (NaN, or -1 for an index).
 template <class R, class Queue>
 R reduce_to_host(Queue queue, R bad) {
     ch::clear_error();
     if (ch::ensure_init() != CLEAVE_HIP_OK) return bad;
-    R* d = (R*)ch::scratch(3, 64);
-    if (!d) return bad;
-    if (queue(d) != CLEAVE_HIP_OK) return bad;
-    R r = bad;
-    if (cleave_hip_download(&r, d, sizeof(R)) != (int64_t)sizeof(R)) return bad;
-    return r;
+    R* h = (R*)ch::host_word();
+    if (!h) return bad;
+    if (queue(h) != CLEAVE_HIP_OK) return bad;
+    if (ch::check_hip(hipStreamSynchronize(ch::stream()), "hipStreamSynchronize") != CLEAVE_HIP_OK) return bad;
+    return *(volatile R*)h;
 }
 
 }  // namespace
@@ -370,85 +414,49 @@ R reduce_to_host(Queue queue, R bad) {
 extern "C" {
 
 int32_t cleave_hip_reduce_sum_f32(const float* x, int64_t len, float* out_dev) {
-    return run_reduce_sum<float>("cleave_hip_reduce_sum_f32", x, len, out_dev);
+    return run_sum<float>("cleave_hip_reduce_sum_f32", x, len, out_dev, false);
 }
 
 int32_t cleave_hip_reduce_sum_f64(const double* x, int64_t len, double* out_dev) {
-    return run_reduce_sum<double>("cleave_hip_reduce_sum_f64", x, len, out_dev);
+    return run_sum<double>("cleave_hip_reduce_sum_f64", x, len, out_dev, false);
 }
 
-// cleave_hip_reduce_sum_f32 with its stage-1 partials in the library's static
-// workspace instead of allocated scratch: the same kernels, grid and result,
-// and no hipMalloc/hipFree on any call.  The partials are all written by
-// stage 1 before stage 2 reads them, so nothing needs clearing between calls.
+// cleave_hip_reduce_sum_f32 with its partials in the library's static
+// workspace instead of allocated scratch: the same kernel, grid and result,
+// and no hipMalloc/hipFree on any call.  The partials are all written before
+// the last workgroup reads them, so nothing needs clearing between calls.
 int32_t cleave_hip_reduce_sum_f32_noalloc(const float* x, int64_t len, float* out_dev) {
     const char* fn = "cleave_hip_reduce_sum_f32_noalloc";
-    CH_REQUIRE(len >= 1, "%s: length must be >= 1 (sum reads v[0])", fn);
-    CH_REQUIRE(x && out_dev, "%s: null buffer", fn);
-    CH_INIT_OR_RETURN();
-    CH_DEVICE(fn, x, len * 4);
+    const int32_t st = check_sum(fn, x, len, out_dev);
+    if (st != CLEAVE_HIP_OK) return st;
     CH_DEVICE(fn, out_dev, 4);
     float* part = ch::noalloc_workspace();
     if (!part) return ch::fail(CLEAVE_HIP_ERR_RUNTIME, "%s: the static workspace has no device address", fn);
-    const int aligned = aligned16(x);
-    unsigned blocks = stage1_blocks(aligned ? len / 4 + 1 : len / kUnroll + 1);
-    CH_REQUIRE(blocks <= (unsigned)ch::kNoAllocFloats,
-               "%s: %u partial sums exceed the static workspace of %d floats", fn, blocks, ch::kNoAllocFloats);
-    sum_stage1<float><<<blocks, kThreads, 0, ch::stream()>>>(x, len, part, aligned);
-    CH_LAUNCHED("sum_stage1");
-    sum_stage2<float><<<1, kThreads, 0, ch::stream()>>>(part, (int)blocks, out_dev);
-    CH_LAUNCHED("sum_stage2");
-    return CLEAVE_HIP_OK;
+    CH_REQUIRE(4 * ch::num_cus() <= ch::kNoAllocFloats, "%s: %d partial sums exceed the static workspace of %d floats",
+               fn, 4 * ch::num_cus(), ch::kNoAllocFloats);
+    return queue_sum<float>(x, len, part, out_dev, 1);
 }
 
 int32_t cleave_hip_reduce_max_f32(const float* x, int64_t len, float* max_dev, int64_t* argmax_dev) {
-    return run_reduce_max<float>("cleave_hip_reduce_max_f32", x, len, max_dev, argmax_dev);
+    return run_max<float>("cleave_hip_reduce_max_f32", x, len, max_dev, argmax_dev, false);
 }
 
 int32_t cleave_hip_reduce_max_f64(const double* x, int64_t len, double* max_dev, int64_t* argmax_dev) {
-    return run_reduce_max<double>("cleave_hip_reduce_max_f64", x, len, max_dev, argmax_dev);
+    return run_max<double>("cleave_hip_reduce_max_f64", x, len, max_dev, argmax_dev, false);
 }
 
 int32_t cleave_hip_reduce_sum_u32_u64(const uint32_t* x, int64_t len, uint64_t* out_dev) {
-    CH_REQUIRE(len >= 0, "cleave_hip_reduce_sum_u32_u64: negative length");
-    CH_REQUIRE(x && out_dev, "cleave_hip_reduce_sum_u32_u64: null buffer");
-    CH_INIT_OR_RETURN();
-    CH_DEVICE("cleave_hip_reduce_sum_u32_u64", x, len * 4);
-    CH_DEVICE("cleave_hip_reduce_sum_u32_u64", out_dev, 8);
-    const int aligned = aligned16(x);
-    unsigned blocks = stage1_blocks(aligned ? len / 4 + 1 : len / kUnroll + 1);
-    uint64_t* part = (uint64_t*)ch::scratch(2, sizeof(uint64_t) * blocks);
-    if (!part) return CLEAVE_HIP_ERR_OOM;
-    sum_u32_stage1<false><<<blocks, kThreads, 0, ch::stream()>>>(x, len, part, aligned);
-    CH_LAUNCHED("sum_u32_stage1");
-    sum_u64_stage2<<<1, kThreads, 0, ch::stream()>>>(part, (int)blocks, out_dev);
-    CH_LAUNCHED("sum_u64_stage2");
-    return CLEAVE_HIP_OK;
+    return run_sum_u32<false>("cleave_hip_reduce_sum_u32_u64", x, len, out_dev, false);
 }
 
 int32_t cleave_hip_reduce_sum_i32_i64(const int32_t* x, int64_t len, int64_t* out_dev) {
-    const char* fn = "cleave_hip_reduce_sum_i32_i64";
-    CH_REQUIRE(len >= 0, "%s: negative length", fn);
-    CH_REQUIRE(x && out_dev, "%s: null buffer", fn);
-    CH_INIT_OR_RETURN();
-    CH_DEVICE(fn, x, len * 4);
-    CH_DEVICE(fn, out_dev, 8);
-    const int aligned = aligned16(x);
-    unsigned blocks = stage1_blocks(aligned ? len / 4 + 1 : len / kUnroll + 1);
-    uint64_t* part = (uint64_t*)ch::scratch(2, sizeof(uint64_t) * blocks);
-    if (!part) return CLEAVE_HIP_ERR_OOM;
-    sum_u32_stage1<true><<<blocks, kThreads, 0, ch::stream()>>>(reinterpret_cast<const uint32_t*>(x), len, part,
-                                                                 aligned);
-    CH_LAUNCHED("sum_i32_stage1");
-    sum_u64_stage2<<<1, kThreads, 0, ch::stream()>>>(part, (int)blocks, reinterpret_cast<uint64_t*>(out_dev));
-    CH_LAUNCHED("sum_u64_stage2");
-    return CLEAVE_HIP_OK;
+    return run_sum_u32<true>("cleave_hip_reduce_sum_i32_i64", reinterpret_cast<const uint32_t*>(x), len,
+                             reinterpret_cast<uint64_t*>(out_dev), false);
 }
 
-// Host-returning forms (synchronise): the reduction lands in a library-owned
-// device word that is copied back.
+// Host-returning forms (synchronise).
 float cleave_hip_sum_f32(const float* x, int64_t len) {
-    return reduce_to_host<float>([&](float* d) { return cleave_hip_reduce_sum_f32(x, len, d); }, NAN);
+    return reduce_to_host<float>([&](float* h) { return run_sum<float>("cleave_hip_sum_f32", x, len, h, true); }, NAN);
 }
 
 float cleave_hip_mean_f32(const float* x, int64_t len) {
@@ -457,15 +465,18 @@ float cleave_hip_mean_f32(const float* x, int64_t len) {
 }
 
 float cleave_hip_max_of_f32(const float* x, int64_t len) {
-    return reduce_to_host<float>([&](float* d) { return cleave_hip_reduce_max_f32(x, len, d, nullptr); }, NAN);
+    return reduce_to_host<float>(
+        [&](float* h) { return run_max<float>("cleave_hip_max_of_f32", x, len, h, nullptr, true); }, NAN);
 }
 
 int64_t cleave_hip_argmax_f32(const float* x, int64_t len) {
-    return reduce_to_host<int64_t>([&](int64_t* d) { return cleave_hip_reduce_max_f32(x, len, nullptr, d); }, -1);
+    return reduce_to_host<int64_t>(
+        [&](int64_t* h) { return run_max<float>("cleave_hip_argmax_f32", x, len, nullptr, h, true); }, -1);
 }
 
 double cleave_hip_sum_f64(const double* x, int64_t len) {
-    return reduce_to_host<double>([&](double* d) { return cleave_hip_reduce_sum_f64(x, len, d); }, NAN);
+    return reduce_to_host<double>([&](double* h) { return run_sum<double>("cleave_hip_sum_f64", x, len, h, true); },
+                                  NAN);
 }
 
 double cleave_hip_mean_f64(const double* x, int64_t len) {
@@ -474,19 +485,27 @@ double cleave_hip_mean_f64(const double* x, int64_t len) {
 }
 
 double cleave_hip_max_of_f64(const double* x, int64_t len) {
-    return reduce_to_host<double>([&](double* d) { return cleave_hip_reduce_max_f64(x, len, d, nullptr); }, NAN);
+    return reduce_to_host<double>(
+        [&](double* h) { return run_max<double>("cleave_hip_max_of_f64", x, len, h, nullptr, true); }, NAN);
 }
 
 int64_t cleave_hip_argmax_f64(const double* x, int64_t len) {
-    return reduce_to_host<int64_t>([&](int64_t* d) { return cleave_hip_reduce_max_f64(x, len, nullptr, d); }, -1);
+    return reduce_to_host<int64_t>(
+        [&](int64_t* h) { return run_max<double>("cleave_hip_argmax_f64", x, len, nullptr, h, true); }, -1);
 }
 
 int64_t cleave_hip_sum_i32_i64(const int32_t* x, int64_t len) {
-    return reduce_to_host<int64_t>([&](int64_t* d) { return cleave_hip_reduce_sum_i32_i64(x, len, d); }, 0);
+    return reduce_to_host<int64_t>(
+        [&](int64_t* h) {
+            return run_sum_u32<true>("cleave_hip_sum_i32_i64", reinterpret_cast<const uint32_t*>(x), len,
+                                     reinterpret_cast<uint64_t*>(h), true);
+        },
+        0);
 }
 
 uint64_t cleave_hip_sum_u32_u64(const uint32_t* x, int64_t len) {
-    return reduce_to_host<uint64_t>([&](uint64_t* d) { return cleave_hip_reduce_sum_u32_u64(x, len, d); }, 0);
+    return reduce_to_host<uint64_t>(
+        [&](uint64_t* h) { return run_sum_u32<false>("cleave_hip_sum_u32_u64", x, len, h, true); }, 0);
 }
 
 }  // extern "C"

@@ -31,6 +31,7 @@ struct State {
     void* scratch[kScratchSlots] = {};
     size_t scratch_bytes[kScratchSlots] = {};
     float* noalloc = nullptr;  // device address of ::scratch on device 0
+    void* host_word = nullptr;
 };
 State g;
 int g_abort_on_error = 1;
@@ -41,6 +42,12 @@ thread_local char t_last_msg[512] = "";
 hipStream_t stream() { return g.stream; }
 int num_cus() { return g.cus; }
 float* noalloc_workspace() { return g.noalloc; }
+
+void* host_word() {
+    if (!g.host_word && check_hip(hipHostMalloc(&g.host_word, 64, hipHostMallocDefault), "hipHostMalloc") != CLEAVE_HIP_OK)
+        g.host_word = nullptr;
+    return g.host_word;
+}
 
 int32_t fail(int32_t code, const char* fmt, ...) {
     va_list ap;

@@ -117,3 +117,30 @@ def test_one_launch_reductions_back_to_back(hip, oracle):
             assert hip.max_of(d) == oracle.max_of(x), (rep, n)
             assert hip.argmax(d) == oracle.argmax(x), (rep, n)
             assert hip.sum_u64(dc) == int(c.astype(np.uint64).sum()), (rep, n)
+
+
+# Around one workgroup, the first fold over workgroups, a group of the arrival tree (32
+# workgroups) and the full grid, aligned and one element in; whole numbers, so every order
+# of the sum is exact, and the maximum planted at the ends of runs.
+@pytest.mark.parametrize("dtype", ["f32", "f64"])
+@pytest.mark.parametrize("n", [1, 255, 256, 257, 1023, 1025, 4095, 4097, 8193, 131071, 131073, 1 << 20, (1 << 22) + 5])
+def test_one_launch_edges(hip, n, dtype):
+    np_t = np.float32 if dtype == "f32" else np.float64
+    x = np.random.default_rng(n).integers(-3, 4, n + 1).astype(np_t)
+    buf = hip.from_numpy(x)
+    for off in (0, 1):
+        t, v = buf.sub(off, (n,)), x[off:off + n]
+        assert hip.sum(t) == v.sum(dtype=np.float64)
+        assert hip.max_of(t) == v.max() and hip.argmax(t) == int(v.argmax())
+    for at in sorted({0, n // 2, max(0, n - 2), n - 1}):
+        y = np.full(n, -np.inf, np_t)
+        y[at] = -5.0
+        t = hip.from_numpy(y)
+        assert hip.max_of(t) == -5.0 and hip.argmax(t) == at
+        if at:
+            y[0] = np.nan  # a NaN first value is the answer, a later one never is
+            t = hip.from_numpy(y)
+            assert np.isnan(hip.max_of(t)) and hip.argmax(t) == 0
+            y[0], y[at] = -np.inf, np.nan
+            t = hip.from_numpy(y)
+            assert hip.max_of(t) == -np.inf and hip.argmax(t) == 0
