@@ -843,13 +843,14 @@ bool try_batched_k_slices(const float* a, const float* b, float* c, int M, int N
 double est_staged_us(const float* a, const float* b, int M, int N, int K, int batch, int ta, int tb) {
     const int64_t cus = ch::num_cus() > 0 ? ch::num_cus() : 1;
     const int64_t tiles = (int64_t)((M + 63) / 64) * ((N + 63) / 64) * batch;
-    const double flops = 2.0 * M * N * K * batch;
     if (tiles > cus) return 0.0;
     const bool base16 = (((uintptr_t)a | (uintptr_t)b) & 15) == 0;
-    const int64_t tiles32 = (int64_t)(M / 32) * (N / 32) * batch;
-    if (M % 64 == 0 && N % 64 == 0 && batch == 1 && split_count(M, N, K) > 1) return 0.0;  // K slices fill the chip
     // the small kernel's shapes: level with the wave tiles (256^3 5.4 against 5.1-5.4 us)
-    if (base16 && tiles32 <= 2 * cus && ch::F32Small::fits(M, N, K, ta ? M : K, tb ? K : N, !ta, tb)) return 0.0;
+    if (base16 && (int64_t)(M / 32) * (N / 32) * batch <= 2 * cus &&
+        ch::F32Small::fits(M, N, K, ta ? M : K, tb ? K : N, !ta, tb))
+        return 0.0;
+    if (M % 64 == 0 && N % 64 == 0 && batch == 1 && split_count(M, N, K) > 1) return 0.0;  // K slices fill the chip
+    const double flops = 2.0 * M * N * K * batch;
     if ((M <= 32 || N <= 32) && flops >= kSkinnyMinFlops)
         return 8.0 + 4.0 * batch * ((double)M * K + (double)K * N) / 5.0e6;
     if (flops < kPadMinFlops) return 6.0;

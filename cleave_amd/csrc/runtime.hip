@@ -265,6 +265,16 @@ size_t buf_cached_bytes() {
 }
 
 int32_t require_device(const char* fn, const char* what, const void* p, uint64_t bytes) {
+    // A live buffer of the library's own is device memory of a known extent: one
+    // map lookup, where hipPointerGetAttributes takes about 0.3 us an operand.
+    uint64_t avail = 0;
+    if (pool_extent(p, &avail)) {
+        if (bytes > avail)
+            return fail(CLEAVE_HIP_ERR_ARG,
+                        "%s: %s needs %llu bytes from %p, but its allocation holds %llu bytes from there", fn, what,
+                        (unsigned long long)bytes, p, (unsigned long long)avail);
+        return CLEAVE_HIP_OK;
+    }
     hipPointerAttribute_t at{};
     if (hipPointerGetAttributes(&at, p) != hipSuccess) {
         // A pointer the runtime does not know at all.
@@ -283,14 +293,6 @@ int32_t require_device(const char* fn, const char* what, const void* p, uint64_t
         return fail(CLEAVE_HIP_ERR_ARG,
                     "%s: %s (%p) points into a buffer that was freed (cleave_hip_buf_free); allocate a new one",
                     fn, what, p);
-    uint64_t avail = 0;
-    if (pool_extent(p, &avail)) {
-        if (bytes > avail)
-            return fail(CLEAVE_HIP_ERR_ARG,
-                        "%s: %s needs %llu bytes from %p, but its allocation holds %llu bytes from there", fn, what,
-                        (unsigned long long)bytes, p, (unsigned long long)avail);
-        return CLEAVE_HIP_OK;
-    }
     hipDeviceptr_t base = nullptr;
     size_t size = 0;
     if (hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)p) == hipSuccess) {
