@@ -20,8 +20,9 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kRowUnroll = 4;
 
-// Past the 256 MiB MALL a matrix read once streams with non-temporal loads; a
-// smaller one is often still there from the kernel that wrote it.
+// Past the 256 MiB MALL a matrix read once streams with non-temporal loads, and one
+// written streams out; a smaller one is often still there from the kernel that wrote
+// it, and is left there for the one that reads it.
 constexpr int64_t kStreamBytes = 256LL << 20;
 
 // A 16-byte column chunk: 4 floats or 2 doubles.
@@ -34,9 +35,10 @@ template <class T>
 __device__ __forceinline__ typename Chunk<T>::type ldnt(const T* p) {
     return __builtin_nontemporal_load(reinterpret_cast<const typename Chunk<T>::type*>(p));
 }
-template <class T>
-__device__ __forceinline__ void stnt(T* p, typename Chunk<T>::type v) {
-    __builtin_nontemporal_store(v, reinterpret_cast<typename Chunk<T>::type*>(p));
+template <class T, bool NT>
+__device__ __forceinline__ void st(T* p, typename Chunk<T>::type v) {
+    if constexpr (NT) __builtin_nontemporal_store(v, reinterpret_cast<typename Chunk<T>::type*>(p));
+    else *reinterpret_cast<typename Chunk<T>::type*>(p) = v;
 }
 
 // Launch shape of both kernels: blockIdx.x = group * nseg + seg, where seg
@@ -60,7 +62,7 @@ Tiling tiling_rows(int64_t rows, int64_t cols, int64_t rows_per_group, int per_c
 // one-shot map) keep the most bytes in flight: 8 rows per block measured
 // 6.6 TB/s at 65536 x 4096 against 4.8 TB/s for 128.
 Tiling tiling_bias(int64_t rows, int64_t cols, int per_chunk) { return tiling_rows(rows, cols, 8, per_chunk); }
-template <class T>
+template <class T, bool NT>
 __global__ __launch_bounds__(kThreads) void add_row_bias_kernel(const T* __restrict__ a, const T* __restrict__ bias,
                                                                 T* __restrict__ out, int64_t rows, int64_t cols,
                                                                 int64_t nseg, int64_t rpg) {
@@ -77,9 +79,9 @@ __global__ __launch_bounds__(kThreads) void add_row_bias_kernel(const T* __restr
 #pragma unroll
         for (int u = 0; u < kRowUnroll; ++u) v[u] = ldnt(a + (r + u) * cols + c);
 #pragma unroll
-        for (int u = 0; u < kRowUnroll; ++u) stnt(out + (r + u) * cols + c, v[u] + b);
+        for (int u = 0; u < kRowUnroll; ++u) st<T, NT>(out + (r + u) * cols + c, v[u] + b);
     }
-    for (; r < r1; ++r) stnt(out + r * cols + c, ldnt(a + r * cols + c) + b);
+    for (; r < r1; ++r) st<T, NT>(out + r * cols + c, ldnt(a + r * cols + c) + b);
 }
 
 // Column sums, out[j] = sum_i g[i][j], in one launch for any width.
@@ -191,7 +193,36 @@ __global__ __launch_bounds__(kThreads) void col_sums_kernel(const U* __restrict_
     if (mine && lane == 0) out[c] = acc;
 }
 
-// Scalar form for widths that are not a multiple of 4 or unaligned pointers.
+// Rows that are not whole chunks (a classifier's 10 outputs): the array is one run of
+// chunks all the same, and a chunk's bias elements are gathered from its first column
+// on.  One division a chunk, in 32 bits below 2^31 elements, where a thread an element
+// took a 64-bit one each (a layer's bias, tanh, its backward and column sums over 20000
+// x 1001 f32: 137 us, now 115, of which the cached stores give about 12).
+template <class T, class I>
+__global__ __launch_bounds__(kThreads) void add_row_bias_flat(const T* __restrict__ a, const T* __restrict__ bias,
+                                                              T* __restrict__ out, I n, uint32_t cols) {
+    constexpr int V = Chunk<T>::kN;
+    typedef typename Chunk<T>::type vec;
+    for (I i = ((I)blockIdx.x * kThreads + threadIdx.x) * V; i < n; i += (I)gridDim.x * kThreads * V) {
+        uint32_t c = (uint32_t)(i % cols);
+        if (n - i >= V) {
+            vec v = ldnt(a + i);
+#pragma unroll
+            for (int e = 0; e < V; ++e) {
+                v[e] = v[e] + bias[c];
+                if (++c == cols) c = 0;
+            }
+            st<T, false>(out + i, v);
+        } else {
+            for (I e = i; e < n; ++e) {
+                out[e] = a[e] + bias[c];
+                if (++c == cols) c = 0;
+            }
+        }
+    }
+}
+
+// Scalar form for unaligned pointers.
 template <class T>
 __global__ void add_row_bias_scalar(const T* a, const T* bias, T* out, int64_t rows, int64_t cols) {
     const int64_t n = rows * cols;
@@ -222,8 +253,20 @@ int32_t run_add_row_bias(const char* fn, const T* a, int64_t alen, const T* bias
     CH_DEVICE(fn, out, outlen * sizeof(T));
     if (cols % V == 0 && aligned16(a) && aligned16(bias) && aligned16(out)) {
         const Tiling t = tiling_bias(rows, cols, V);
-        add_row_bias_kernel<T><<<(unsigned)(t.nseg * t.groups), kThreads, 0, ch::stream()>>>(
-            a, bias, out, rows, cols, t.nseg, t.rows_per_group);
+        const unsigned grid = (unsigned)(t.nseg * t.groups);
+        if (alen * (int64_t)sizeof(T) > kStreamBytes)
+            add_row_bias_kernel<T, true><<<grid, kThreads, 0, ch::stream()>>>(a, bias, out, rows, cols, t.nseg,
+                                                                             t.rows_per_group);
+        else
+            add_row_bias_kernel<T, false><<<grid, kThreads, 0, ch::stream()>>>(a, bias, out, rows, cols, t.nseg,
+                                                                              t.rows_per_group);
+    } else if (aligned16(a) && aligned16(out)) {
+        const unsigned grid = (unsigned)((alen / V + kThreads) / kThreads < 0x7FFFFFFF ? (alen / V + kThreads) / kThreads
+                                                                                       : 0x7FFFFFFF);
+        if (alen < (int64_t)1 << 31)
+            add_row_bias_flat<T, uint32_t><<<grid, kThreads, 0, ch::stream()>>>(a, bias, out, (uint32_t)alen, cols);
+        else
+            add_row_bias_flat<T, uint64_t><<<grid, kThreads, 0, ch::stream()>>>(a, bias, out, (uint64_t)alen, cols);
     } else {
         add_row_bias_scalar<T><<<blocks_for(alen), kThreads, 0, ch::stream()>>>(a, bias, out, rows, cols);
     }
@@ -332,7 +375,7 @@ __device__ __forceinline__ void bcast_row_offsets(const BDims& d, I row, I& oa, 
 // the row and the output stream through non-temporal loads and stores, as in
 // the same-shape maps.  Requires the VEC conditions.
 constexpr int kRowChunks = 64;
-template <class Op, class T, class I>
+template <class Op, class T, class I, bool NT>
 __global__ __launch_bounds__(kThreads) void bcast_rows_kernel(const T* __restrict__ a, const T* __restrict__ b,
                                                               T* __restrict__ out, BDims d, I rows, I chunks) {
     constexpr int V = Chunk<T>::kN;
@@ -366,7 +409,7 @@ __global__ __launch_bounds__(kThreads) void bcast_rows_kernel(const T* __restric
                     vec r;
 #pragma unroll
                     for (int t = 0; t < V; ++t) r[t] = op(va[u][t], vb[u][t]);
-                    stnt(o + c * V, r);
+                    st<T, NT>(o + c * V, r);
                 }
             }
         }
@@ -515,11 +558,14 @@ int32_t run_bcast(const char* fn, const T* a, int64_t alen, const int32_t* ash, 
     const bool narrow = outlen < (int64_t)1 << 31 && alen < (int64_t)1 << 31 && blen < (int64_t)1 << 31;
     if (vec && chunks >= kRowChunks) {
         const unsigned grid = (unsigned)(rows < 65536 * 8 ? rows : 65536 * 8);
-        if (narrow)
-            bcast_rows_kernel<Op, T, uint32_t><<<grid, kThreads, 0, ch::stream()>>>(a, b, out, d, (uint32_t)rows,
-                                                                                   (uint32_t)chunks);
+        if (outlen * (int64_t)sizeof(T) <= kStreamBytes && narrow)
+            bcast_rows_kernel<Op, T, uint32_t, false><<<grid, kThreads, 0, ch::stream()>>>(a, b, out, d, (uint32_t)rows,
+                                                                                          (uint32_t)chunks);
+        else if (narrow)
+            bcast_rows_kernel<Op, T, uint32_t, true><<<grid, kThreads, 0, ch::stream()>>>(a, b, out, d, (uint32_t)rows,
+                                                                                         (uint32_t)chunks);
         else
-            bcast_rows_kernel<Op, T, int64_t><<<grid, kThreads, 0, ch::stream()>>>(a, b, out, d, rows, chunks);
+            bcast_rows_kernel<Op, T, int64_t, true><<<grid, kThreads, 0, ch::stream()>>>(a, b, out, d, rows, chunks);
         CH_LAUNCHED(fn);
         return CLEAVE_HIP_OK;
     }

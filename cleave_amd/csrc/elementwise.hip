@@ -2,8 +2,8 @@
 // Activation<Tensor> (stdlib/nn/nn.cleave:82-95) and the backward forms of the
 // reference's derivative rules (stdlib/num/num.cleave:123-136, :222-223).
 //
-// HBM-bound: each thread moves one 16-byte vector per operand with
-// non-temporal loads/stores, over a grid that covers the array.
+// HBM-bound: each thread moves one 16-byte vector per operand, over a grid that
+// covers the array.
 // The library is compiled with -ffp-contract=off, so every op below rounds
 // exactly where the reference's scalar loop does (add/sub/mul/div/neg/relu
 // are bit-exact; exp/tanh come from the device math library).
@@ -57,9 +57,9 @@ struct Vec16 {
 };
 
 // One 16-byte vector per thread over a grid that covers the whole array (a
-// grid-stride loop only past 2^31 blocks), with non-temporal loads and stores:
-// streamed data is not kept in L2, which lifts a read+write stream from ~5.5
-// to ~6.4 TB/s on MI355X.
+// grid-stride loop only past 2^31 blocks), with non-temporal loads, and stores
+// past kCachedBytes: streamed data is not kept in L2, which lifts a read+write
+// stream from ~5.5 to ~6.4 TB/s on MI355X.
 unsigned grid_for(int64_t nvec) {
     int64_t want = (nvec + kThreads - 1) / kThreads;
     if (want > 0x7FFFFFFF) want = 0x7FFFFFFF;
@@ -70,12 +70,19 @@ template <class T>
 __device__ __forceinline__ typename Vec16<T>::type ldv(const T* p) {
     return __builtin_nontemporal_load(reinterpret_cast<const typename Vec16<T>::type*>(p));
 }
-template <class T>
+// Results of up to the MALL's 256 MiB are stored through the caches: the map
+// that follows reads them from there (bias, tanh, its backward and the column
+// sums over 20000 x 1000 f32: 123 -> 110 us, over 65536 x 1024 350 -> 320), at
+// 0-6% on a map whose result nobody reads next.  Larger ones stream past them
+// (2^28 f32 sigmoid 327 us, through the caches 346).
+constexpr int64_t kCachedBytes = 256LL << 20;
+template <class T, bool NT>
 __device__ __forceinline__ void stv(T* p, typename Vec16<T>::type v) {
-    __builtin_nontemporal_store(v, reinterpret_cast<typename Vec16<T>::type*>(p));
+    if constexpr (NT) __builtin_nontemporal_store(v, reinterpret_cast<typename Vec16<T>::type*>(p));
+    else *reinterpret_cast<typename Vec16<T>::type*>(p) = v;
 }
 
-template <class Op, class T>
+template <class Op, class T, bool NT>
 __global__ __launch_bounds__(kThreads) void map1_kernel(const T* __restrict__ a, T* __restrict__ out, int64_t n) {
     constexpr int V = Vec16<T>::kN;
     Op op;
@@ -86,7 +93,7 @@ __global__ __launch_bounds__(kThreads) void map1_kernel(const T* __restrict__ a,
         typename Vec16<T>::type y;
 #pragma unroll
         for (int e = 0; e < V; ++e) y[e] = op(x[e]);
-        stv(out + V * i, y);
+        stv<T, NT>(out + V * i, y);
     }
     if (blockIdx.x == 0 && threadIdx.x < (n % V)) {
         int64_t i = nv * V + threadIdx.x;
@@ -94,7 +101,7 @@ __global__ __launch_bounds__(kThreads) void map1_kernel(const T* __restrict__ a,
     }
 }
 
-template <class Op, class T>
+template <class Op, class T, bool NT>
 __global__ __launch_bounds__(kThreads) void map2_kernel(const T* __restrict__ a, const T* __restrict__ b,
                                                         T* __restrict__ out, int64_t n) {
     constexpr int V = Vec16<T>::kN;
@@ -106,7 +113,7 @@ __global__ __launch_bounds__(kThreads) void map2_kernel(const T* __restrict__ a,
         typename Vec16<T>::type z;
 #pragma unroll
         for (int e = 0; e < V; ++e) z[e] = op(x[e], y[e]);
-        stv(out + V * i, z);
+        stv<T, NT>(out + V * i, z);
     }
     if (blockIdx.x == 0 && threadIdx.x < (n % V)) {
         int64_t i = nv * V + threadIdx.x;
@@ -140,10 +147,12 @@ int32_t run1(const char* name, const T* a, int64_t alen, T* out, int64_t outlen)
     CH_INIT_OR_RETURN();
     CH_DEVICE(name, a, alen * sizeof(T));
     CH_DEVICE(name, out, outlen * sizeof(T));
-    if (aligned16(a) && aligned16(out))
-        map1_kernel<Op, T><<<grid_for(alen / V), kThreads, 0, ch::stream()>>>(a, out, alen);
-    else
+    if (!aligned16(a) || !aligned16(out))
         map1_scalar_kernel<Op, T><<<grid_for(alen / V + 1), kThreads, 0, ch::stream()>>>(a, out, alen);
+    else if (alen * (int64_t)sizeof(T) > kCachedBytes)
+        map1_kernel<Op, T, true><<<grid_for(alen / V), kThreads, 0, ch::stream()>>>(a, out, alen);
+    else
+        map1_kernel<Op, T, false><<<grid_for(alen / V), kThreads, 0, ch::stream()>>>(a, out, alen);
     CH_LAUNCHED(name);
     return CLEAVE_HIP_OK;
 }
@@ -160,10 +169,12 @@ int32_t run2(const char* name, const T* a, int64_t alen, const T* b, int64_t ble
     CH_DEVICE(name, a, alen * sizeof(T));
     CH_DEVICE(name, b, blen * sizeof(T));
     CH_DEVICE(name, out, outlen * sizeof(T));
-    if (aligned16(a) && aligned16(b) && aligned16(out))
-        map2_kernel<Op, T><<<grid_for(alen / V), kThreads, 0, ch::stream()>>>(a, b, out, alen);
-    else
+    if (!aligned16(a) || !aligned16(b) || !aligned16(out))
         map2_scalar_kernel<Op, T><<<grid_for(alen / V + 1), kThreads, 0, ch::stream()>>>(a, b, out, alen);
+    else if (alen * (int64_t)sizeof(T) > kCachedBytes)
+        map2_kernel<Op, T, true><<<grid_for(alen / V), kThreads, 0, ch::stream()>>>(a, b, out, alen);
+    else
+        map2_kernel<Op, T, false><<<grid_for(alen / V), kThreads, 0, ch::stream()>>>(a, b, out, alen);
     CH_LAUNCHED(name);
     return CLEAVE_HIP_OK;
 }

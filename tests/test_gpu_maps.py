@@ -204,3 +204,15 @@ def test_sum_rows_keeps_nan_inf_and_negative_zero(hip, oracle):
     got, want = hip.sum_rows(hip.from_numpy(G)).numpy(), oracle.sum_rows(G)
     assert np.array_equal(np.isnan(got), np.isnan(want))
     assert np.array_equal(got[~np.isnan(got)], want[~np.isnan(want)]) and np.signbit(got[5])
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f64"])
+@pytest.mark.parametrize("rows,cols", [(1, 1), (1, 3), (5, 1), (3, 2), (7, 3), (257, 5), (4096, 10), (33, 1001), (2, 8191)])
+def test_add_row_bias_ragged_widths(hip, rows, cols, dtype):
+    rng = np.random.default_rng(rows * 31 + cols)
+    np_t = np.float32 if dtype == "f32" else np.float64
+    A, b = rng.standard_normal((rows, cols)).astype(np_t), rng.standard_normal(cols).astype(np_t)
+    out = hip.from_numpy(np.full(rows * cols + 8, 7.0, np_t))  # the entries past the result stay
+    hip.add_row_bias(hip.from_numpy(A), hip.from_numpy(b), out=out.sub(0, (rows, cols)))
+    got = out.numpy()
+    assert np.array_equal(got[:rows * cols].reshape(rows, cols), A + b) and np.all(got[rows * cols:] == 7.0)
