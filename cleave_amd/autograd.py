@@ -112,6 +112,13 @@ def _broadcast_scalar(g: Tensor, shape) -> Tensor:
     return out.view(shape)
 
 
+def _scalar(value: float, shape, dtype: str) -> Tensor:
+    """A one-element tensor of `value`, queued: 0 + value by Index's reverse rule.
+    An upload would wait for the stream, and drained the queue twice a step."""
+    t = ca.zero(ca.empty((1,), dtype))
+    return ca.index_bwd(value, t, (0,)).view(shape)
+
+
 # ---- operators -----------------------------------------------------------------------
 
 def _product_rule(a: Var, b: Var):
@@ -235,7 +242,7 @@ def sum(a: Var) -> Var:  # noqa: A001 - mirrors the stdlib name
 def mean(a: Var) -> Var:
     """Mean (stdlib/nn/nn.cleave:135-138): sum / N, differentiated through the
     quotient rule with a constant denominator."""
-    n = const(np.array([float(a.tensor.size)], _NP[a.tensor.dtype]))
+    n = const(_scalar(float(a.tensor.size), (1,), a.tensor.dtype))
     return div(sum(a), n)
 
 
@@ -326,7 +333,7 @@ def backward(loss: Var) -> None:
         stack.append((v, True))
         for p in edges(v)[0]:
             stack.append((p, False))
-    loss.grad = ca.from_numpy(np.ones(loss.shape, _NP[loss.tensor.dtype]))
+    loss.grad = _scalar(1.0, loss.shape, loss.tensor.dtype)
     for v in reversed(order):
         parents, rule = edges(v)
         if rule is None or v.grad is None:
