@@ -195,7 +195,7 @@ __global__ __launch_bounds__(kThreads) void col_sums_kernel(const U* __restrict_
 
 // Rows that are not whole chunks (a classifier's 10 outputs): the array is one run of
 // chunks all the same, and a chunk's bias elements are gathered from its first column
-// on.  One division a chunk, in 32 bits below 2^31 elements, where a thread an element
+// on.  One division a chunk, in 32 bits up to about 2^31 elements, where a thread an element
 // took a 64-bit one each (a layer's bias, tanh, its backward and column sums over 20000
 // x 1001 f32: 137 us, now 115, of which the cached stores give about 12).
 template <class T, class I>
@@ -263,7 +263,8 @@ int32_t run_add_row_bias(const char* fn, const T* a, int64_t alen, const T* bias
     } else if (aligned16(a) && aligned16(out)) {
         const unsigned grid = (unsigned)((alen / V + kThreads) / kThreads < 0x7FFFFFFF ? (alen / V + kThreads) / kThreads
                                                                                        : 0x7FFFFFFF);
-        if (alen < (int64_t)1 << 31)
+        // 32 bits hold an index and the grid's stride past it (up to alen + kThreads V).
+        if (2 * alen + 2 * kThreads * V <= (int64_t)UINT32_MAX)
             add_row_bias_flat<T, uint32_t><<<grid, kThreads, 0, ch::stream()>>>(a, bias, out, (uint32_t)alen, cols);
         else
             add_row_bias_flat<T, uint64_t><<<grid, kThreads, 0, ch::stream()>>>(a, bias, out, (uint64_t)alen, cols);
