@@ -70,11 +70,15 @@ template <class T>
 __device__ __forceinline__ typename Vec16<T>::type ldv(const T* p) {
     return __builtin_nontemporal_load(reinterpret_cast<const typename Vec16<T>::type*>(p));
 }
-// Results of up to the MALL's 256 MiB are stored through the caches: the map
-// that follows reads them from there (bias, tanh, its backward and the column
-// sums over 20000 x 1000 f32: 123 -> 110 us, over 65536 x 1024 350 -> 320), at
-// 0-6% on a map whose result nobody reads next.  Larger ones stream past them
-// (2^28 f32 sigmoid 327 us, through the caches 346).
+// Results of up to the MALL's 256 MiB are stored through the caches, as the map
+// that follows reads them there: bias, tanh, its backward and column sums over
+// n x 1024 f32 take 52.8 us instead of 60.4 at 32 MiB, 91 instead of 100 at 64,
+// 165 instead of 183 at 128, and with streaming stores between 20 and 48 MiB
+// 57.1 at 32.  A map whose result nobody reads next pays 4-6% (32 MiB 13.5 us
+// against 12.8), and one repeated on the same buffers up to a third around the
+// L2s' 32 MiB (24 MiB 9.7 against 7.1, 64 MiB 22.7 against 20.1, 192 MiB 58.7
+// against 60.7).  Larger ones stream past them (2^28 f32 sigmoid 327 us, through
+// the caches 346).
 constexpr int64_t kCachedBytes = 256LL << 20;
 template <class T, bool NT>
 __device__ __forceinline__ void stv(T* p, typename Vec16<T>::type v) {

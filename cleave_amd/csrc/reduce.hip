@@ -10,7 +10,9 @@
 // The host-returning forms have the kernel write the result into pinned host
 // memory.  With a second launch for the fold and a copy of the result, a Mean of
 // 10^6 f32 took 26.7 us, now 17; Mean, Max and argmax of 10^7 together 96, now 71.
-// Queued sums from 10^7 elements on are level (10^7 10.2 us, 2^28 159).
+// Queued sums: 2^20 f32 7.4 -> 5.4 us, 2^23 7.4 -> 6.4, 2^25 21.1 -> 21.8, 2^28 154 ->
+// 160 (a mean of 2^27 99 -> 94); 16 rows of loads in flight instead of 8 took the last to
+// 156-159 and cost the maximum of 2^27 4%.
 //
 // Max semantics: the reference folds acc = v[0]; if v[i] > acc then acc = v[i]
 // (cmpf ogt, stdlib/num/num.cleave:303).  A NaN at i > 0 never wins; a NaN at

@@ -275,7 +275,7 @@ CLEAVE_HIP_API int32_t cleave_hip_reduce_sum_i32_i64(const int32_t* x, int64_t l
  * under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  Same kernels, grid and result as cleave_hip_reduce_sum_f32;
  * its partial sums live in a static 64 KiB device workspace (16384 floats,
- * one per stage-1 block; a call needing more is CLEAVE_HIP_ERR_ARG) whose
+ * one per workgroup; a call needing more is CLEAVE_HIP_ERR_ARG) whose
  * address the library's init resolves, so call cleave_hip_init() first if
  * the first call must not initialise.  Every call on a device shares that
  * workspace: calls that overlap on one device race. */
