@@ -139,8 +139,10 @@ struct Frags {
 
 // `part`: tiles x slices partial tiles, unused with slices == 1.  A 1-D grid of
 // tiles_m * tiles_n * batch * slices workgroups.
+// (Two waves a SIMD for two k-contiguous operands on 4 x 4 fragments, which the
+// compiler gives 268 registers otherwise.)
 template <bool KCA, bool KCB, bool V2A, bool V2B, int FM, int FN, int WK, int PF, int STEP>
-__global__ __launch_bounds__(kThreads) void gemm_f64_kernel(
+__global__ __launch_bounds__(kThreads, KCA && KCB && FM * FN == 16 && PF < 3 ? 2 : 1) void gemm_f64_kernel(
     const double* __restrict__ A, const double* __restrict__ B, double* __restrict__ C, int M, int N, int K,
     int64_t lda, int64_t ldb, int64_t sa, int64_t sb, int64_t sc, int tiles_m, int tiles_n, int batch, int slices,
     int64_t kslice, double* part) {
@@ -331,24 +333,25 @@ int32_t launch(const Args& g, int slices) {
 }
 
 // The wave tiles, and the time of a product on each as fitted to sweeps on
-// MI355X (48 shapes and layouts from 33 x 77 x 1000 to 4096^3; the choice was
-// within 19% of the best of all measured, within 5% for 38 of them; the two
-// larger tiles' shares were raised when their loads got wider):
-//   base + max(busiest CU's MFMA time / eff, one wave's steps x (MFMA + lat)) + fold
+// MI355X (48 shapes and layouts from 33 x 77 x 1000 to 4096^3, and 26 outputs
+// with K of 128 and 256; within 19% of the best of all measured):
+//   base + max(busiest CU's (MFMA time / eff + end), one wave's steps x (MFMA + lat) + end) + fold
 // A step, 16 of K here, is FM FN x 256 cycles of MFMA, 0.107 us a fragment pair.
 // lat is what a wave's load latency adds where nothing else runs on its SIMD;
+// end is a workgroup's add of the partial tiles in LDS, by one wave: without it
+// 20000 x 500 x 128 took 85 us on the 64 x 32 tiles, 62 on the 128 x 128 ones.
 // eff_k applies where both operands are k-contiguous (A.B^T), whose 64-byte
 // row pieces use the L1 less well.  Past one slice, each partial tile is
 // written and read past the L2: about 3 TB/s for the two, and 3 us.
 struct TileCost {
     int fm, fn, wk;
-    double base, eff, eff_k, lat;  // us, share of the MFMA rate, us a step
+    double base, eff, eff_k, lat, end;  // us, share of the MFMA rate, us a step, us a tile
 };
 constexpr TileCost kTiles[] = {
-    {1, 1, 4, 3.5, 0.32, 0.27, 0.3},
-    {2, 2, 4, 4.0, 0.65, 0.53, 0.6},
-    {4, 2, 4, 6.0, 0.77, 0.70, 0.6},
-    {4, 4, 1, 9.0, 0.86, 0.80, 0.6},
+    {1, 1, 4, 3.3, 0.32, 0.27, 0.3, 0.2},
+    {2, 2, 4, 3.55, 0.65, 0.53, 0.6, 0.45},
+    {4, 2, 4, 5.0, 0.77, 0.70, 0.6, 0.8},
+    {4, 4, 1, 9.0, 0.86, 0.80, 0.6, 0.0},
 };
 constexpr int kSlices[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
 
@@ -373,8 +376,9 @@ Plan choose_tile(const Args& g, bool kca, bool kcb) {
             if (s > 1 && (t.wk == 1 || g.K / s < 128 || tiles * s > 16 * (int64_t)cus || tiles > kCounters)) break;
             const double steps = (double)((((int64_t)g.K + s - 1) / s + 16 * t.wk - 1) / (16 * t.wk));
             const double mfma = 0.107 * t.fm * t.fn;
-            const double busy = (double)((tiles * s + cus - 1) / cus) * steps * mfma / (both_k ? t.eff_k : t.eff);
-            const double chain = steps * (mfma + t.lat);
+            const double busy =
+                (double)((tiles * s + cus - 1) / cus) * (steps * mfma / (both_k ? t.eff_k : t.eff) + t.end);
+            const double chain = steps * (mfma + t.lat) + t.end;
             const double us = t.base + (busy > chain ? busy : chain) +
                               (s > 1 ? 3.0 + (double)(tiles * s) * tm * tn * 16.0 / 3e6 : 0.0);
             if (us < best_us) best_us = us, best.tile = i, best.slices = s;
@@ -403,22 +407,45 @@ int narrow_slices(const Args& g, int64_t tiles) {
     return s < 1 ? 1 : (int)s;
 }
 
+// Shallow products (K up to 64) of more than two and a half 64 x 64 tiles a CU
+// mostly write C: waves on tiles of their own, four workgroups a CU.  Quarters of
+// so short a K, and the 128 x 128 tiles' two workgroups a CU, left the stores
+// uncovered (us): 65536 x 100 x 64 50 -> 29, 4096^2 x 8 34 -> 23, 256 of 128^2 x
+// 64 23.6 -> 17.2, 2654 x 1520 x 3 12.8 -> 8.6.  Not where C fills under two thirds
+// of the tiles (4096 of 32^2 x 32 18.5 on 16 x 16 tiles, 29 here), nor past K = 8
+// with an odd N, whose rows the wider tiles store better (43 of 4031 x 267 x 16 104
+// against 117).  A.B^T keeps the 128 x 128 tiles past K = 8, where C fills them:
+// 4096^2 x 64 53 there, 67 here.
+bool shallow(const Args& g, bool both_k) {
+    const int64_t t64 = tile_count(g, 64, 64), t128 = tile_count(g, 128, 128);
+    if (g.K > 64 || 2 * t64 <= 5 * (int64_t)ch::num_cus() || t64 > 0x7FFFFFFF) return false;
+    if (2.0 * 64 * 64 * t64 > 3.0 * g.M * g.N * g.batch || (g.K > 8 && g.N % 2)) return false;
+    return !both_k || g.K <= 8 || t128 < ch::num_cus() || t64 < 3 * t128;
+}
+
 template <bool KCA, bool KCB, bool V2A, bool V2B>
 int32_t run_shape(const Args& g) {
     if (g.N <= 16 && (KCA || g.M >= 2) && tile_count(g, 32, 16) <= 0x7FFFFFFF)
         return launch<KCA, KCB, V2A, V2B, 2, 1, 4, 2, 16>(g, narrow_slices(g, tile_count(g, 32, 16)));
     if (g.M <= 16 && (KCB || g.N >= 2) && tile_count(g, 16, 32) <= 0x7FFFFFFF)
         return launch<KCA, KCB, V2A, V2B, 1, 2, 4, 2, 16>(g, narrow_slices(g, tile_count(g, 16, 32)));
+    if ((KCA || g.M >= 2) && (KCB || g.N >= 2) && shallow(g, KCA && KCB))
+        return launch<KCA, KCB, V2A, V2B, 2, 2, 1, 2, 8>(g, 1);
     const Plan p = choose_tile(g, KCA, KCB);
     switch (p.tile) {
         case 0: return launch<KCA, KCB, V2A, V2B, 1, 1, 4, 4, 16>(g, p.slices);
         case 1: return launch<KCA, KCB, V2A, V2B, 2, 2, 4, 1, 16>(g, p.slices);
         case 2: return launch<KCA, KCB, V2A, V2B, 4, 2, 4, 3, 8>(g, p.slices);
-        // A step ahead of 16 leaves the loads to the CU's other wave: 4096^3 A.B
-        // 1906 us against 2190 with three of 8, 2000^3 274 against 268; of two
-        // k-contiguous operands 2469 against 2235.
-        default: return launch<KCA, KCB, V2A, V2B, 4, 4, 1, KCA && KCB ? 3 : 1, KCA && KCB ? 8 : 16>(g, 1);
     }
+    // A step ahead of 16 leaves the loads to the CU's other wave: 4096^3 A.B
+    // 1906 us against 2190 with three of 8, 2000^3 274 against 268.
+    if constexpr (!KCA || !KCB) return launch<KCA, KCB, V2A, V2B, 4, 4, 1, 1, 16>(g, 1);
+    // Of two k-contiguous operands, aligned or not: up to K = 128 two steps of 8
+    // ahead on two waves a SIMD, then three on one.  4096^2 x 64 53 us against 61,
+    // 20000 x 500 x 128 71 against 70, x 256 142 against 119, 2000^3 276 against
+    // 268 (4096^3 2101 against 2228; one of 16 on two waves 2181, 2000^3 303).
+    else if (g.K <= 128) return launch<KCA, KCB, V2A, V2B, 4, 4, 1, 2, 8>(g, 1);
+    else return launch<KCA, KCB, V2A, V2B, 4, 4, 1, 3, 8>(g, 1);
 }
 
 template <bool KCA, bool KCB>

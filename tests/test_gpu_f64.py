@@ -304,6 +304,25 @@ def test_tiles_and_slices_exact(hip, batch, M, N, K, ta, tb):
     assert np.array_equal(got, want)
 
 
+# Shallow products on their own tiles (64 x 64, a tile a wave) at the edges of those
+# tiles and of a step of 8, on both sides of their bounds: K of 64, of 8 with an odd N,
+# of 128 for A.B^T on 128 x 128 tiles.
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("K", [1, 7, 8, 9, 63, 64, 65, 128, 129])
+@pytest.mark.parametrize("batch,M,N", [(1, 2047, 2050), (1, 2049, 2047), (180, 65, 126), (170, 66, 127), (700, 64, 63)])
+def test_shallow_products_exact(hip, batch, M, N, K, ta, tb):
+    rng = np.random.default_rng(M * 7 + N * 3 + K + 11 * ta + tb)
+    A = rng.integers(-9, 10, (batch, K, M) if ta else (batch, M, K)).astype(np.float64)
+    B = rng.integers(-9, 10, (batch, N, K) if tb else (batch, K, N)).astype(np.float64)
+    want = (A.transpose(0, 2, 1) if ta else A) @ (B.transpose(0, 2, 1) if tb else B)
+    a, b, c = hip.from_numpy(A), hip.from_numpy(B), hip.from_numpy(np.full((batch, M, N), np.nan))
+    if batch > 1:
+        hip.matmul_batched(a, b, out=c, trans_a=bool(ta), trans_b=bool(tb))
+    else:
+        hip.matmul(a.view(A.shape[1:]), b.view(B.shape[1:]), trans_a=bool(ta), trans_b=bool(tb), out=c.view((M, N)))
+    assert np.array_equal(c.numpy(), want)
+
+
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
 def test_k_tail_keeps_nan_and_inf_where_they_belong(hip, ta, tb):
     # a NaN row of A and an infinite column of B: only their own entries, whatever K's remainder
