@@ -12,10 +12,13 @@
 //   1. X W1                             gemm_f32 NN   (M=B, N=Hd, K=D)
 //   2. per row: H = sigmoid(X W1), z2 = H W2, yhat, e, e*e,
 //      d2 = (e+e)/B * yhat(1-yhat), d1 = (d2 W2) h(1-h) over X W1, and
-//      partial sums of h*d2 and e*e     mlp_rows_kernel
+//      partial sums of h*d2 and e*e     mlp_rows_kernel (Hd > 4096: mlp_wide_rows_kernel,
+//                                       mlp_cols_kernel)
 //   3. dW1 = X^T d1                     gemm_f32 TN
 //   4. dW2 = sum of partials; W1 -= lr dW1, W2 -= lr dW2;
 //      loss = sum(e*e) / B              mlp_finish_kernel
+#include <algorithm>
+
 #include "common.hpp"
 #include "gemm_f32_pingpong.hpp"
 
@@ -198,74 +201,177 @@ __global__ __launch_bounds__(kThreads) void mlp_rows_kernel(float* H, float* D1,
     if (MODE == Rows::kStep && t == 0) sqpart[blockIdx.x] = sq;
 }
 
-// The same for rows past 16 elements a thread (Hd > 4096): a workgroup walks its row
-// twice, with H in memory between, and adds to its row of partials in place.
-template <Rows MODE>
-__global__ __launch_bounds__(kThreads) void mlp_rows_wide_kernel(float* H, float* D1, const float* __restrict__ W2,
-                                                                 const float* __restrict__ v, int B, int Hd,
-                                                                 float* part, float* __restrict__ sqpart,
-                                                                 float* __restrict__ z) {
+// Rows past 16 elements a thread (Hd > 4096) take two passes.  This one forms H over
+// X W1 and z = H W2 a row at a time (8 workgroups a CU), and with STEP d2 and the
+// workgroup's squared errors; mlp_cols_kernel reads H again.  (One pass that walked its
+// row twice and added to a row of dW2 partials in memory moved those as often as H:
+// the step of 65536 x 16 x 4500 took 3334 us, 1623 here, the forward layer alone 1681, 745.)
+constexpr int kWideUnroll = 4;
+template <bool VEC, bool STEP>
+__global__ __launch_bounds__(kThreads) void mlp_wide_rows_kernel(float* H, const float* __restrict__ W2,
+                                                                 const float* __restrict__ y, int B, int Hd,
+                                                                 float* __restrict__ out, float* __restrict__ sqpart) {
+    constexpr int V = VEC ? 4 : 1;
+    typedef float vec __attribute__((ext_vector_type(V)));
     __shared__ float cross[4];
     float sq = 0.0f;
-    float* mine = part + (int64_t)blockIdx.x * Hd;
+    const int n = Hd / V;  // whole vectors: VEC needs Hd % 4 == 0
     for (int64_t r = blockIdx.x; r < B; r += gridDim.x) {
-        float* h = H + r * Hd;
-        float d2;
-        if constexpr (MODE == Rows::kBwd) {
-            d2 = v[r];
-        } else {
-            float acc = 0.0f;
-            for (int c = threadIdx.x; c < Hd; c += kThreads) {
-                const float x = sigmoidf_ref(h[c]);
-                h[c] = x;
-                acc += x * W2[c];
-            }
+        vec* h = reinterpret_cast<vec*>(H + r * Hd);
+        const vec* w = reinterpret_cast<const vec*>(W2);
+        float acc = 0.0f;
+        for (int c0 = threadIdx.x; c0 < n; c0 += kWideUnroll * kThreads) {
+            vec x[kWideUnroll];
 #pragma unroll
-            for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
-            __syncthreads();
-            if ((threadIdx.x & 63) == 0) cross[threadIdx.x >> 6] = acc;
-            __syncthreads();
-            acc = (cross[0] + cross[1]) + (cross[2] + cross[3]);
-            if constexpr (MODE == Rows::kFwd) {
-                if (threadIdx.x == 0) z[r] = acc;
-                continue;
-            }
-            const float yh = sigmoidf_ref(acc);
-            const float e = yh - v[r];
-            sq += e * e;
-            const float gy = (e + e) / (float)B;
-            d2 = gy * yh * (1.0f - yh);
+            for (int u = 0; u < kWideUnroll; ++u)
+                if (c0 + u * kThreads < n) x[u] = h[c0 + u * kThreads];
+#pragma unroll
+            for (int u = 0; u < kWideUnroll; ++u)
+                if (c0 + u * kThreads < n) {
+                    const vec q = w[c0 + u * kThreads];
+#pragma unroll
+                    for (int e = 0; e < V; ++e) {
+                        x[u][e] = sigmoidf_ref(x[u][e]);
+                        acc += x[u][e] * q[e];
+                    }
+                    h[c0 + u * kThreads] = x[u];
+                }
         }
-        float* d1 = (MODE == Rows::kBwd ? D1 : H) + r * Hd;
-        for (int c = threadIdx.x; c < Hd; c += kThreads) {  // each thread meets its own columns again
-            const float x = h[c], g = d2 * W2[c];
-            const float s = x * d2;
-            mine[c] = r == blockIdx.x ? s : mine[c] + s;
-            d1[c] = g * x * (1.0f - x);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
+        __syncthreads();  // the last row's reads of cross
+        if ((threadIdx.x & 63) == 0) cross[threadIdx.x >> 6] = acc;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            acc = (cross[0] + cross[1]) + (cross[2] + cross[3]);
+            if constexpr (STEP) {
+                const float yh = sigmoidf_ref(acc);
+                const float e = yh - y[r];
+                sq += e * e;
+                const float gy = (e + e) / (float)B;
+                out[r] = gy * yh * (1.0f - yh);
+            } else {
+                out[r] = acc;
+            }
         }
     }
-    if (MODE == Rows::kStep && threadIdx.x == 0) sqpart[blockIdx.x] = sq;
+    if (STEP && threadIdx.x == 0) sqpart[blockIdx.x] = sq;
 }
 
-// Workgroups of the row pass: one row a thread group, up to two workgroups a CU.
-int row_groups(int B, int Hd) {
+// d1 (over H, when D1 is H) and a row of dW2 partials per band of rows_per_band rows;
+// a workgroup owns kWideCols columns, four a thread, and keeps their sums in registers.
+constexpr int kWideCols = 4 * kThreads;
+template <bool VEC>
+__global__ __launch_bounds__(kThreads) void mlp_cols_kernel(const float* H, float* D1, const float* __restrict__ W2,
+                                                            const float* __restrict__ d2, int B, int Hd,
+                                                            int rows_per_band, float* __restrict__ part) {
+    typedef float v4 __attribute__((ext_vector_type(4)));
+    const int first = blockIdx.x * kWideCols + (VEC ? 4 : 1) * threadIdx.x;
+    auto col = [&](int j) { return first + (VEC ? j : j * kThreads); };
+    auto load = [&](const float* p, float (&x)[4]) {
+        if constexpr (VEC) {
+            const v4 q = first < Hd ? *reinterpret_cast<const v4*>(p + first) : v4(0.0f);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) x[j] = q[j];
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) x[j] = col(j) < Hd ? p[col(j)] : 0.0f;
+        }
+    };
+    auto store = [&](float* p, const float (&x)[4]) {
+        if constexpr (VEC) {
+            if (first < Hd) *reinterpret_cast<v4*>(p + first) = v4{x[0], x[1], x[2], x[3]};
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (col(j) < Hd) p[col(j)] = x[j];
+        }
+    };
+    const int64_t r0 = (int64_t)blockIdx.y * rows_per_band;
+    const int64_t r1 = r0 + rows_per_band < B ? r0 + rows_per_band : B;
+    float w[4], s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    load(W2, w);
+    for (int64_t r = r0; r < r1; r += kWideUnroll) {
+        float h[kWideUnroll][4];
+#pragma unroll
+        for (int u = 0; u < kWideUnroll; ++u)
+            if (r + u < r1) load(H + (r + u) * Hd, h[u]);
+#pragma unroll
+        for (int u = 0; u < kWideUnroll; ++u)
+            if (r + u < r1) {
+                const float d = d2[r + u];
+                float d1[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    s[j] += h[u][j] * d;
+                    const float g = d * w[j];
+                    d1[j] = g * h[u][j] * (1.0f - h[u][j]);
+                }
+                store(D1 + (r + u) * Hd, d1);
+            }
+    }
+    store(part + (int64_t)blockIdx.y * Hd, s);
+}
+
+constexpr int kRowsMaxHd = 4096;  // the widest row of mlp_rows_kernel
+
+// Workgroups of the row passes: one row a thread group.  Up to two a CU where each
+// writes a row of dW2 partials, up to eight where none does (29289 x 16 X W1 in the
+// forward layer: 26.6 us, with two a CU 30.9).
+int row_groups(int B, int Hd, bool partials) {
     const int lanes = Hd <= 1024 ? kThreads / 64 : 1;
-    const int64_t want = ((int64_t)B + lanes - 1) / lanes, cap = 2 * (int64_t)ch::num_cus();
+    const int64_t want = ((int64_t)B + lanes - 1) / lanes, cap = (partials ? 2 : 8) * (int64_t)ch::num_cus();
     return (int)(want < cap ? want : cap);
 }
 
+// Rows of a band of mlp_cols_kernel: about four workgroups a CU over all bands.
+int wide_rows_per_band(int B, int Hd) {
+    const int64_t across = (Hd + kWideCols - 1) / kWideCols;
+    const int64_t bands = std::max<int64_t>(1, 4 * (int64_t)ch::num_cus() / across);
+    return (int)(((int64_t)B + bands - 1) / bands);
+}
+
+// Rows of dW2 partials that the passes of a B x Hd layer write.
+int partial_rows(int B, int Hd) {
+    if (Hd <= kRowsMaxHd) return row_groups(B, Hd, true);
+    const int rows = wide_rows_per_band(B, Hd);
+    return (B + rows - 1) / rows;
+}
+
+// The hidden layer's passes over H (mlp_rows_kernel, or the two above).  d2: B floats of
+// workspace of the wide step; part has partial_rows(B, Hd) rows, sqpart row_groups(...).
 template <Rows MODE>
-int32_t run_rows(float* H, float* D1, const float* W2, const float* v, int B, int Hd, float* part, float* sqpart,
-                 float* z, hipStream_t st) {
-    const unsigned grid = (unsigned)row_groups(B, Hd);
+int32_t run_rows(float* H, float* D1, const float* W2, const float* v, int B, int Hd, float* d2, float* part,
+                 float* sqpart, float* z, hipStream_t st) {
     const bool vec = Hd % 4 == 0 && (((uintptr_t)H | (uintptr_t)D1 | (uintptr_t)W2 | (uintptr_t)part) & 15) == 0;
+    if (Hd > kRowsMaxHd) {
+        constexpr bool kIsStep = MODE == Rows::kStep;
+        if constexpr (MODE != Rows::kBwd) {
+            auto rows = [&](auto kernel) {
+                kernel<<<(unsigned)row_groups(B, Hd, false), kThreads, 0, st>>>(H, W2, v, B, Hd, kIsStep ? d2 : z,
+                                                                               sqpart);
+            };
+            vec ? rows(mlp_wide_rows_kernel<true, kIsStep>) : rows(mlp_wide_rows_kernel<false, kIsStep>);
+            CH_LAUNCHED("mlp_wide_rows_kernel");
+        }
+        if constexpr (MODE != Rows::kFwd) {
+            const dim3 grid((unsigned)((Hd + kWideCols - 1) / kWideCols), (unsigned)partial_rows(B, Hd));
+            auto cols = [&](auto kernel) {
+                kernel<<<grid, kThreads, 0, st>>>(H, kIsStep ? H : D1, W2, kIsStep ? d2 : v, B, Hd,
+                                                 wide_rows_per_band(B, Hd), part);
+            };
+            vec ? cols(mlp_cols_kernel<true>) : cols(mlp_cols_kernel<false>);
+            CH_LAUNCHED("mlp_cols_kernel");
+        }
+        return CLEAVE_HIP_OK;
+    }
+    const unsigned grid = (unsigned)row_groups(B, Hd, MODE != Rows::kFwd);
     auto go = [&](auto kernel) { kernel<<<grid, kThreads, 0, st>>>(H, D1, W2, v, B, Hd, part, sqpart, z); };
     if (Hd <= 256) vec ? go(mlp_rows_kernel<64, 4, true, MODE>) : go(mlp_rows_kernel<64, 4, false, MODE>);
     else if (Hd <= 512) vec ? go(mlp_rows_kernel<64, 8, true, MODE>) : go(mlp_rows_kernel<64, 8, false, MODE>);
     else if (Hd <= 1024) vec ? go(mlp_rows_kernel<64, 16, true, MODE>) : go(mlp_rows_kernel<64, 16, false, MODE>);
     else if (Hd <= 2048) vec ? go(mlp_rows_kernel<256, 8, true, MODE>) : go(mlp_rows_kernel<256, 8, false, MODE>);
-    else if (Hd <= 4096) vec ? go(mlp_rows_kernel<256, 16, true, MODE>) : go(mlp_rows_kernel<256, 16, false, MODE>);
-    else go(mlp_rows_wide_kernel<MODE>);
+    else vec ? go(mlp_rows_kernel<256, 16, true, MODE>) : go(mlp_rows_kernel<256, 16, false, MODE>);
     CH_LAUNCHED("mlp_rows_kernel");
     return CLEAVE_HIP_OK;
 }
@@ -283,7 +389,8 @@ struct Finish {
     const float* part2;  // groups x Hd
     int groups, Hd;
     float *dw2, *w2;
-    const float* sqpart;  // groups
+    const float* sqpart;  // errs
+    int errs;
     float* loss;
     float count, lr;
 };
@@ -310,7 +417,8 @@ __global__ __launch_bounds__(kThreads) void mlp_finish_kernel(Finish f) {
     const int c = errors ? 0 : ((int)blockIdx.x - f.blocks1) * kFoldCols + (int)threadIdx.x % cols;
     const float* p = errors ? f.sqpart : f.part2 + c;
     const int64_t pitch = errors ? 1 : f.Hd;
-    const int q0 = (int)((int64_t)f.groups * lane / lanes), q1 = (int)((int64_t)f.groups * (lane + 1) / lanes);
+    const int64_t runs = errors ? f.errs : f.groups;
+    const int q0 = (int)(runs * lane / lanes), q1 = (int)(runs * (lane + 1) / lanes);
     float acc = 0.0f;
     if (errors || c < f.Hd) {
         int q = q0;
@@ -376,8 +484,7 @@ __global__ __launch_bounds__(kThreads) void dw1_finish_kernel(const float* __res
     }
 }
 
-// loss = (sum of the n values v) / count: per-row squared errors (unfused
-// path, n = B) or per-block sums of them (fused path).
+// loss = (sum of the n values v) / count: the row blocks' sums of squared errors.
 __global__ __launch_bounds__(kThreads) void loss_kernel(const float* __restrict__ v, int n, float count,
                                                         float* __restrict__ loss) {
     __shared__ float part[kThreads / 64];
@@ -520,7 +627,7 @@ int32_t hidden_fwd(const float* x, const float* w1, const float* w2, float* h, f
     }
     int32_t rc = ch::gemm_f32_device(x, w1, h, B, Hd, D, 0, 0);
     if (rc != CLEAVE_HIP_OK) return rc;
-    return run_rows<Rows::kFwd>(h, nullptr, w2, nullptr, B, Hd, nullptr, nullptr, z, st);
+    return run_rows<Rows::kFwd>(h, nullptr, w2, nullptr, B, Hd, nullptr, nullptr, nullptr, z, st);
 }
 
 int32_t hidden_bwd(const float* x, const float* h, const float* w2, const float* g, float* dw1, float* dw2, int B,
@@ -553,12 +660,12 @@ int32_t hidden_bwd(const float* x, const float* h, const float* w2, const float*
         }
         return CLEAVE_HIP_OK;
     }
-    const int groups = row_groups(B, Hd);
+    const int groups = partial_rows(B, Hd);
     const size_t nH = (size_t)B * Hd, nPart = (size_t)groups * Hd;
     float* d1 = (float*)ch::scratch(4, sizeof(float) * (up(nH) + up(nPart)));
     if (!d1) return CLEAVE_HIP_ERR_OOM;
     float* part = d1 + up(nH);
-    int32_t rc = run_rows<Rows::kBwd>(const_cast<float*>(h), d1, w2, g, B, Hd, part, nullptr, nullptr, st);
+    int32_t rc = run_rows<Rows::kBwd>(const_cast<float*>(h), d1, w2, g, B, Hd, nullptr, part, nullptr, nullptr, st);
     if (rc != CLEAVE_HIP_OK) return rc;
     if (dw1) {
         rc = ch::gemm_f32_device(x, d1, dw1, D, Hd, B, 1, 0);
@@ -601,19 +708,21 @@ extern "C" int32_t cleave_hip_mlp_step_f32(const float* x, int64_t xlen, const f
     hipStream_t st = ch::stream();
     if (fused_fits(x, w1, B, D, Hd)) return fused_step(x, y, w1, w2, dw1, dw2, loss_dev, B, D, Hd, lr, st);
 
-    const int groups = row_groups(B, Hd);
-    // Scratch slot 4: H/d1 | dW2 partials | squared errors | dW1 if not asked for.
-    const size_t nH = (size_t)B * Hd, nPart = (size_t)groups * Hd, nG = dw1 ? 0 : (size_t)D * Hd;
+    const bool wide = Hd > kRowsMaxHd;
+    const int groups = partial_rows(B, Hd), errs = row_groups(B, Hd, !wide);
+    // Scratch slot 4: H/d1 | dW2 partials | squared errors | d2 of the wide passes | dW1 if not asked for.
+    const size_t nH = (size_t)B * Hd, nPart = (size_t)groups * Hd, nD2 = wide ? B : 0, nG = dw1 ? 0 : (size_t)D * Hd;
     auto up = [](size_t n) { return (n + 63) & ~(size_t)63; };
-    float* H = (float*)ch::scratch(4, sizeof(float) * (up(nH) + up(nPart) + up(groups) + up(nG)));
+    float* H = (float*)ch::scratch(4, sizeof(float) * (up(nH) + up(nPart) + up(errs) + up(nD2) + up(nG)));
     if (!H) return CLEAVE_HIP_ERR_OOM;
     float* part = H + up(nH);
     float* sq = part + up(nPart);
-    float* g1 = dw1 ? dw1 : sq + up(groups);
+    float* d2 = sq + up(errs);
+    float* g1 = dw1 ? dw1 : d2 + up(nD2);
 
     int32_t rc = ch::gemm_f32_device(x, w1, H, B, Hd, D, 0, 0);
     if (rc != CLEAVE_HIP_OK) return rc;
-    rc = run_rows<Rows::kStep>(H, nullptr, w2, y, B, Hd, part, sq, nullptr, st);
+    rc = run_rows<Rows::kStep>(H, nullptr, w2, y, B, Hd, d2, part, sq, nullptr, st);
     if (rc != CLEAVE_HIP_OK) return rc;
     rc = ch::gemm_f32_device(x, H, g1, D, Hd, B, 1, 0);
     if (rc != CLEAVE_HIP_OK) return rc;
@@ -621,7 +730,7 @@ extern "C" int32_t cleave_hip_mlp_step_f32(const float* x, int64_t xlen, const f
     f.g1 = g1, f.n1 = (int64_t)D * Hd, f.blocks1 = lr != 0.0f ? (int)capped_grid(f.n1) : 0;
     f.w1 = w1;
     f.part2 = part, f.groups = groups, f.Hd = Hd, f.dw2 = dw2, f.w2 = w2;
-    f.sqpart = sq, f.loss = loss_dev, f.count = (float)B, f.lr = lr;
+    f.sqpart = sq, f.errs = errs, f.loss = loss_dev, f.count = (float)B, f.lr = lr;
     mlp_finish_kernel<<<finish_grid(f), kThreads, 0, st>>>(f);
     CH_LAUNCHED("mlp_finish_kernel");
     return CLEAVE_HIP_OK;

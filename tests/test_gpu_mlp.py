@@ -238,6 +238,18 @@ def test_hidden_layer_forward_and_rule(hip, oracle, B, D, Hd):
 @pytest.mark.parametrize("Hd", [1, 3, 64, 255, 256, 257, 510, 512, 1000, 1024, 1025, 2047, 2048, 2052, 4095, 4096,
                                 4100, 5003])
 def test_row_pass_widths(hip, oracle, B, Hd):
+    _row_pass(hip, oracle, B, Hd)
+
+
+# More rows than the passes' workgroups take at once: two and eight a CU up to 4096 wide;
+# past it eight a CU for the rows and bands of 5 and 13 rows (loads of 4 and remainders)
+# for the columns.
+@pytest.mark.parametrize("B,Hd", [(9001, 30), (2301, 1100), (1001, 4100), (2500, 4097), (2600, 5003)])
+def test_row_pass_many_rows(hip, oracle, B, Hd):
+    _row_pass(hip, oracle, B, Hd)
+
+
+def _row_pass(hip, oracle, B, Hd):
     rng = np.random.default_rng(B * 10007 + Hd)
     D = 7
     X = rng.standard_normal((B, D)).astype(np.float32)
