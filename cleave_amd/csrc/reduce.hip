@@ -3,16 +3,15 @@
 // same counts as cleave's i32 type carries them).
 //
 // One launch, deterministic for a given length and device: each workgroup of a
-// fixed grid folds its run of the array's 16-byte vectors in registers, the
+// fixed grid folds its rows of the array's 16-byte vectors in registers, the
 // wave combines lanes with cross-lane shuffles, LDS carries the 4 wave results
 // to one, and the workgroup that arrives last folds the workgroups' results in
 // their order (last_block.hpp).  HBM-bound from a few MB; below that, latency.
 // The host-returning forms have the kernel write the result into pinned host
 // memory.  With a second launch for the fold and a copy of the result, a Mean of
-// 10^6 f32 took 26.7 us, now 17; Mean, Max and argmax of 10^7 together 96, now 71.
-// Queued sums: 2^20 f32 7.4 -> 5.4 us, 2^23 7.4 -> 6.4, 2^25 21.1 -> 21.8, 2^28 154 ->
-// 160 (a mean of 2^27 99 -> 94); 16 rows of loads in flight instead of 8 took the last to
-// 156-159 and cost the maximum of 2^27 4%.
+// 10^6 f32 took 26.7 us, now 17; Mean, Max and argmax of 10^7 together 96, now @TRIPLE@.
+// Queued sums of f32: 2^20 6.7 -> 4.9 us, 2^23 6.4 -> 6.1, 2^25 20.5 -> 20.4, 2^28 154 ->
+// 154-157; of u32, 2^25 21.6 -> 20.4.  max and argmax of 2^25 24.9 -> 23.4, 2^28 163 -> 160.
 //
 // Max semantics: the reference folds acc = v[0]; if v[i] > acc then acc = v[i]
 // (cmpf ogt, stdlib/num/num.cleave:303).  A NaN at i > 0 never wins; a NaN at
@@ -29,7 +28,6 @@
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kUnroll = 8;
 // Workgroups of the running reduction that have arrived, 0 between launches; the
 // allocation-free Sum has its own, as it has its own workspace.
 static __device__ uint32_t g_arrived[2][ch::kTreeWords];
@@ -38,21 +36,31 @@ static __device__ uint32_t g_arrived[2][ch::kTreeWords];
 // always).  Loads are non-temporal: the data is read once.
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 
-// The array as rows of kThreads vectors; workgroup b of G takes rows
-// [R b / G, R (b + 1) / G), so that none has more than one row over another, and up
-// to four workgroups a CU keep 128 KiB a CU in flight.  (Rows b, b + G, ... instead
-// took 207 us at 2^28 f32 against 159; eight workgroups a CU 167.)
+// The array as rows of kThreads vectors, read U rows at a time (fold_rows).
+//   Sums      U = 4, up to two workgroups a CU: workgroup b takes rows [4 b, 4 b + 4),
+//             then those a grid further on, so neighbours read neighbouring 16 KiB.
+//             2^25 / 2^28 f32 20.2 / 151 us; U = 8 with four a CU 20.6 / 156, one 20.7 /
+//             151, eight 20.7 / 153; U = 4 with four 20.5 / 154; U = 2 with four 20.0 /
+//             152, slower to 2^24; a run of rows a workgroup, U = 8, four a CU 21.6 / 156.
+//             Unaligned, a row of single elements: U = 8, four a CU (2^25 f32 22 us; 40 so).
+//   Maximum   U = 8, up to four a CU: workgroup b of G takes the run [R b / G, R (b + 1) / G)
+//             of R rows, its elements in ascending order.
 struct Rows {
-    int64_t begin, end;
+    int64_t begin, end, step;
 };
+template <int U, bool RUN>
 __device__ __forceinline__ Rows my_rows(int64_t nvec) {
     const int64_t rows = (nvec + kThreads - 1) / kThreads;
-    return {rows * blockIdx.x / gridDim.x, rows * (blockIdx.x + 1) / gridDim.x};
+    if constexpr (RUN) return {rows * blockIdx.x / gridDim.x, rows * (blockIdx.x + 1) / gridDim.x, U};
+    return {(int64_t)U * blockIdx.x, rows, (int64_t)U * gridDim.x};
 }
-unsigned row_blocks(int64_t nvec) {
-    const int64_t rows = (nvec + kThreads - 1) / kThreads, want = (rows + 3) / 4;
+constexpr int kSumUnroll = 4, kScalarUnroll = 8, kMaxUnroll = 8;
+constexpr int kMinRows = 4;                                      // a workgroup
+constexpr int kSumPerCu = 2, kScalarPerCu = 4, kMaxPerCu = 4;  // workgroups
+unsigned row_blocks(int64_t nvec, int per_cu) {
+    const int64_t rows = (nvec + kThreads - 1) / kThreads, want = (rows + kMinRows - 1) / kMinRows;
     const int64_t most = ch::kTreeArity * ch::kTreeGroups;  // of the arrival tree
-    const int64_t cap = std::min<int64_t>(4 * (int64_t)ch::num_cus(), most);
+    const int64_t cap = std::min<int64_t>(per_cu * (int64_t)ch::num_cus(), most);
     return (unsigned)(want < 1 ? 1 : want < cap ? want : cap);
 }
 
@@ -84,26 +92,31 @@ __device__ T block_sum(T v) {
     return r;  // valid in thread 0
 }
 
-// Calls fold(vector, vector index) for this workgroup's vectors in ascending order
-// per thread, kUnroll loads in flight.
-template <class VT, class Fold>
+// Calls fold(vector, slot) for this workgroup's vectors in ascending order per
+// thread, U loads (the slots) in flight.
+template <class VT, int U, bool RUN, class Fold>
 __device__ __forceinline__ void fold_rows(const void* x, int64_t nvec, Fold fold) {
     const VT* p = reinterpret_cast<const VT*>(x);
-    const Rows r = my_rows(nvec);
-    for (int64_t row = r.begin; row < r.end; row += kUnroll) {
-        VT v[kUnroll];
+    const Rows r = my_rows<U, RUN>(nvec);
+    VT v[U];
+    int64_t row = r.begin;
+    for (; row + U <= r.end && (row + U) * kThreads <= nvec; row += r.step) {
 #pragma unroll
-        for (int u = 0; u < kUnroll; ++u) {
-            const int64_t i = (row + u) * kThreads + threadIdx.x;
-            if (row + u < r.end && i < nvec) {
-                v[u] = __builtin_nontemporal_load(p + i);
-            }
-        }
+        for (int u = 0; u < U; ++u) v[u] = __builtin_nontemporal_load(p + (row + u) * kThreads + threadIdx.x);
 #pragma unroll
-        for (int u = 0; u < kUnroll; ++u) {
-            const int64_t i = (row + u) * kThreads + threadIdx.x;
-            if (row + u < r.end && i < nvec) fold(v[u], i);
-        }
+        for (int u = 0; u < U; ++u) fold(v[u], u);
+    }
+    if (row >= r.end) return;
+    // at most U rows are left, the last of which may be short
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int64_t i = (row + u) * kThreads + threadIdx.x;
+        if (row + u < r.end && i < nvec) v[u] = __builtin_nontemporal_load(p + i);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int64_t i = (row + u) * kThreads + threadIdx.x;
+        if (row + u < r.end && i < nvec) fold(v[u], u);
     }
 }
 
@@ -123,26 +136,44 @@ __device__ __forceinline__ void fold_partials(const U* partial, Fold fold) {
     }
 }
 
-// Each lane keeps one accumulator per vector element and adds them in a
-// fixed tree at the end: (a0 + a1) + (a2 + a3) for f32, a0 + a1 for f64.
+// Each lane keeps an accumulator per slot and vector element, and folds the slots'
+// into one per element, (c0 + c1) + (c2 + c3), every kChain trips, so that no chain of
+// adds grows with the array; at the end (a0 + a1) + (a2 + a3) for f32, a0 + a1 for f64.
+constexpr int kChain = 16;
 template <class T>
 __global__ __launch_bounds__(kThreads) void sum_kernel(const T* __restrict__ x, int64_t n, T* partial,
                                                        T* __restrict__ out, int aligned, int counter) {
     constexpr int V = Vec16<T>::kN;
     typedef typename Vec16<T>::type VT;
-    T acc[V];
+    static_assert(kSumUnroll == 4, "the fold of the slots");
+    T chain[kSumUnroll][V], acc[V], lane;
 #pragma unroll
-    for (int e = 0; e < V; ++e) acc[e] = T(0);
+    for (int e = 0; e < V; ++e) acc[e] = chain[0][e] = chain[1][e] = chain[2][e] = chain[3][e] = T(0);
+    int trips = 0;
+    auto fold_slots = [&]() {
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+            acc[e] += (chain[0][e] + chain[1][e]) + (chain[2][e] + chain[3][e]);
+            chain[0][e] = chain[1][e] = chain[2][e] = chain[3][e] = T(0);
+        }
+    };
+    auto next_trip = [&](bool last_slot) {
+        if (last_slot && ++trips % kChain == 0) fold_slots();
+    };
     if (aligned) {
-        fold_rows<VT>(x, n / V, [&](VT v, int64_t) {
+        fold_rows<VT, kSumUnroll, false>(x, n / V, [&](VT v, int slot) {
 #pragma unroll
-            for (int e = 0; e < V; ++e) acc[e] += v[e];
+            for (int e = 0; e < V; ++e) chain[slot][e] += v[e];
+            next_trip(slot == kSumUnroll - 1);
         });
-        if (blockIdx.x == 0 && threadIdx.x < (n % V)) acc[0] += x[n / V * V + threadIdx.x];
+        if (blockIdx.x == 0 && threadIdx.x < (n % V)) chain[0][0] += x[n / V * V + threadIdx.x];
     } else {
-        fold_rows<T>(x, n, [&](T v, int64_t) { acc[0] += v; });
+        fold_rows<T, kScalarUnroll, false>(x, n, [&](T v, int slot) {
+            chain[slot % kSumUnroll][0] += v;
+            next_trip(slot == kScalarUnroll - 1);
+        });
     }
-    T lane;
+    fold_slots();
     if constexpr (V == 4) lane = (acc[0] + acc[1]) + (acc[2] + acc[3]);
     else lane = acc[0] + acc[1];
     T r = block_sum(lane);
@@ -217,10 +248,10 @@ __global__ __launch_bounds__(kThreads) void max_kernel(const T* __restrict__ x, 
 #pragma unroll
     for (int e = 0; e < V; ++e) bv[e] = T(-INFINITY), bk[e] = kNone;
     Best<T> b{-INFINITY, INT64_MAX};
-    const int64_t first = my_rows(aligned ? n / V : n).begin * kThreads + threadIdx.x;
+    const int64_t first = my_rows<kMaxUnroll, true>(aligned ? n / V : n).begin * kThreads + threadIdx.x;
     auto index = [&](uint32_t k) { return first + (int64_t)k * kThreads; };  // of the vector
     if (aligned) {
-        fold_rows<VT>(x, n / V, [&](VT v, int64_t) {
+        fold_rows<VT, kMaxUnroll, true>(x, n / V, [&](VT v, int) {
 #pragma unroll
             for (int e = 0; e < V; ++e)
                 if (v[e] > bv[e]) bv[e] = v[e], bk[e] = met;
@@ -231,7 +262,7 @@ __global__ __launch_bounds__(kThreads) void max_kernel(const T* __restrict__ x, 
             if (bk[e] != kNone) take_better(b, bv[e], V * index(bk[e]) + e);
         if (blockIdx.x == 0 && threadIdx.x < (n % V)) take_better(b, x[n / V * V + threadIdx.x], n / V * V + threadIdx.x);
     } else {
-        fold_rows<T>(x, n, [&](T v, int64_t) {
+        fold_rows<T, kMaxUnroll, true>(x, n, [&](T v, int) {
             if (v > bv[0]) bv[0] = v, bk[0] = met;
             ++met;
         });
@@ -305,12 +336,12 @@ __global__ __launch_bounds__(kThreads) void sum_u32_kernel(const uint32_t* __res
     uint64_t acc = 0;
     if (aligned) {
         // Add in 64 bits (mod 2^64, exact for both forms).
-        fold_rows<u4>(x, n / 4, [&](u4 v, int64_t) {
+        fold_rows<u4, kSumUnroll, false>(x, n / 4, [&](u4 v, int) {
             acc += (widen<Signed>(v[0]) + widen<Signed>(v[1])) + (widen<Signed>(v[2]) + widen<Signed>(v[3]));
         });
         if (blockIdx.x == 0 && threadIdx.x < (n & 3)) acc += widen<Signed>(x[n / 4 * 4 + threadIdx.x]);
     } else {
-        fold_rows<uint32_t>(x, n, [&](uint32_t v, int64_t) { acc += widen<Signed>(v); });
+        fold_rows<uint32_t, kScalarUnroll, false>(x, n, [&](uint32_t v, int) { acc += widen<Signed>(v); });
     }
     uint64_t r = block_sum_u64(acc);
     if (gridDim.x > 1) {
@@ -331,7 +362,7 @@ template <class T>
 int32_t queue_sum(const T* x, int64_t len, T* part, T* out, int counter) {
     constexpr int V = Vec16<T>::kN;
     const int aligned = aligned16(x);
-    const unsigned blocks = row_blocks(aligned ? len / V : len);
+    const unsigned blocks = aligned ? row_blocks(len / V, kSumPerCu) : row_blocks(len, kScalarPerCu);
     sum_kernel<T><<<blocks, kThreads, 0, ch::stream()>>>(x, len, part, out, aligned, counter);
     CH_LAUNCHED("sum_kernel");
     return CLEAVE_HIP_OK;
@@ -371,7 +402,7 @@ int32_t run_max(const char* fn, const T* x, int64_t len, T* out_max, int64_t* ou
     if (!host && out_max) CH_DEVICE(fn, out_max, sizeof(T));
     if (!host && out_argmax) CH_DEVICE(fn, out_argmax, 8);
     const int aligned = aligned16(x);
-    const unsigned blocks = row_blocks(aligned ? len / V : len);
+    const unsigned blocks = row_blocks(aligned ? len / V : len, kMaxPerCu);
     char* base = partials();
     if (!base) return CLEAVE_HIP_ERR_OOM;
     int64_t* pi = (int64_t*)base;
@@ -389,7 +420,7 @@ int32_t run_sum_u32(const char* fn, const uint32_t* x, int64_t len, uint64_t* ou
     CH_DEVICE(fn, x, len * 4);
     if (!host) CH_DEVICE(fn, out, 8);
     const int aligned = aligned16(x);
-    const unsigned blocks = row_blocks(aligned ? len / 4 : len);
+    const unsigned blocks = aligned ? row_blocks(len / 4, kSumPerCu) : row_blocks(len, kScalarPerCu);
     uint64_t* part = (uint64_t*)partials();
     if (!part) return CLEAVE_HIP_ERR_OOM;
     sum_u32_kernel<Signed><<<blocks, kThreads, 0, ch::stream()>>>(x, len, part, out, aligned);
