@@ -46,6 +46,10 @@ void* scratch_try(int slot, size_t bytes);
 // Number of compute units (for grid sizing of persistent/strided kernels).
 int num_cus();
 
+// Most workgroups of 256 threads along a launch's x: the runtime takes x * 256 modulo
+// 2^32 (2^24 + 5 of them run as 5, and 2^24 are refused), without an error.
+constexpr int64_t kMaxBlocks = (int64_t(1) << 24) - 1;
+
 // a * b * c for non-negative factors, or -1 when the product exceeds int64
 // (so that no operand length matches it).
 inline int64_t count3(int64_t a, int64_t b, int64_t c) {

@@ -137,8 +137,8 @@ struct Frags {
     }
 };
 
-// `part`: tiles x slices partial tiles, unused with slices == 1.  A 1-D grid of
-// tiles_m * tiles_n * batch * slices workgroups.
+// `part`: tiles x slices partial tiles, unused with slices == 1.  A grid of at least
+// tiles_m * tiles_n * batch * slices workgroups, in rows of at most ch::kMaxBlocks.
 // (Two waves a SIMD for two k-contiguous operands on 4 x 4 fragments, which the
 // compiler gives 268 registers otherwise.)
 template <bool KCA, bool KCB, bool V2A, bool V2B, int FM, int FN, int WK, int PF, int STEP>
@@ -152,8 +152,10 @@ __global__ __launch_bounds__(kThreads, KCA && KCB && FM * FN == 16 && PF < 3 ? 2
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t block = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
+    if (block >= (int64_t)tiles_m * tiles_n * batch * slices) return;
     int b, tm, tn;  // b: batch entry and slice
-    ch::block_coords(blockIdx.x, tiles_m, tiles_n, batch * slices, b, tm, tn);
+    ch::block_coords((int)block, tiles_m, tiles_n, batch * slices, b, tm, tn);
     const int entry = b / slices, z = b - entry * slices;
     A += (int64_t)entry * sa;
     B += (int64_t)entry * sb;
@@ -325,7 +327,9 @@ int32_t launch(const Args& g, int slices) {
         part = (double*)ch::scratch_try(11, sizeof(double) * (size_t)(tiles * slices * FM * FN * 256));
         if (!part) slices = 1, kslice = g.K;  // no room: K in one piece
     }
-    gemm_f64_kernel<KCA, KCB, V2A, V2B, FM, FN, WK, PF, STEP><<<(unsigned)(tiles * slices), kThreads, 0, ch::stream()>>>(
+    const int64_t blocks = tiles * slices, across = blocks < ch::kMaxBlocks ? blocks : ch::kMaxBlocks;
+    const dim3 grid((unsigned)across, (unsigned)((blocks + across - 1) / across));
+    gemm_f64_kernel<KCA, KCB, V2A, V2B, FM, FN, WK, PF, STEP><<<grid, kThreads, 0, ch::stream()>>>(
         g.a, g.b, g.c, g.M, g.N, g.K, KCA ? g.K : g.M, KCB ? g.K : g.N, (int64_t)g.M * g.K, (int64_t)g.K * g.N,
         (int64_t)g.M * g.N, (g.M + TM - 1) / TM, (g.N + TN - 1) / TN, g.batch, slices, kslice, part);
     CH_LAUNCHED("gemm_f64_kernel");

@@ -136,3 +136,28 @@ def test_escape_counts_past_2pow31_pixels(hip, oracle):
         got = cnt.sub(r * w, (w,)).numpy()
         ref = oracle.mandelbrot(w, h, x0, y0, np.float32(dx), np.float32(dy), it, rows=(r, r + 1))[r]
         assert np.array_equal(got, ref), r
+
+
+
+# f64 products with more of their narrow tiles (32 x 16) than a launch holds, along
+# either dimension, and a batch of more entries than that: the last ones as the first.
+@pytest.mark.parametrize("wide", ["m", "n", "batch"])
+def test_f64_products_past_the_grid_limit(hip, wide):
+    n = (1 << 29) + 5 if wide != "batch" else (1 << 24) + 5
+    a = hip.zero(hip.empty((n,), "f64"))
+    where = [0, 77, n // 2, n - 2, n - 1]
+    for i, at in enumerate(where):
+        a.sub(at, (1,)).upload(np.array([i + 1.5]))
+    five = hip.from_numpy(np.array([[5.0]]))
+    if wide == "m":
+        c = hip.matmul(a.view((n, 1)), five)
+    elif wide == "n":
+        c = hip.matmul(five, a.view((1, n)))
+    else:
+        ones = hip.zero(hip.empty((n,), "f64"))
+        for at in where:
+            ones.sub(at, (1,)).upload(np.array([5.0]))
+        c = hip.matmul_batched(a.view((n, 1, 1)), ones.view((n, 1, 1)))
+    for i, at in enumerate(where):
+        assert c.view((n,)).sub(at, (1,)).numpy()[0] == 5.0 * (i + 1.5), (wide, at)
+    assert c.view((n,)).sub(1, (1,)).numpy()[0] == 0.0
