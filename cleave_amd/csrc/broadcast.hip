@@ -10,6 +10,7 @@
 // rows are not whole chunks) and walk a group of rows; the bias chunk (or the column
 // accumulator) stays in registers.  The column sums add in an order that the shape
 // alone fixes, so results are deterministic for a given shape.
+#include <algorithm>
 #include <cmath>
 
 #include "common.hpp"
@@ -251,8 +252,8 @@ int32_t run_add_row_bias(const char* fn, const T* a, int64_t alen, const T* bias
     CH_DEVICE(fn, a, alen * sizeof(T));
     CH_DEVICE(fn, bias, blen * sizeof(T));
     CH_DEVICE(fn, out, outlen * sizeof(T));
-    if (cols % V == 0 && aligned16(a) && aligned16(bias) && aligned16(out)) {
-        const Tiling t = tiling_bias(rows, cols, V);
+    const Tiling t = tiling_bias(rows, cols, V);
+    if (cols % V == 0 && aligned16(a) && aligned16(bias) && aligned16(out) && t.nseg * t.groups <= ch::kMaxBlocks) {
         const unsigned grid = (unsigned)(t.nseg * t.groups);
         if (alen * (int64_t)sizeof(T) > kStreamBytes)
             add_row_bias_kernel<T, true><<<grid, kThreads, 0, ch::stream()>>>(a, bias, out, rows, cols, t.nseg,
@@ -261,8 +262,7 @@ int32_t run_add_row_bias(const char* fn, const T* a, int64_t alen, const T* bias
             add_row_bias_kernel<T, false><<<grid, kThreads, 0, ch::stream()>>>(a, bias, out, rows, cols, t.nseg,
                                                                               t.rows_per_group);
     } else if (aligned16(a) && aligned16(out)) {
-        const unsigned grid = (unsigned)((alen / V + kThreads) / kThreads < 0x7FFFFFFF ? (alen / V + kThreads) / kThreads
-                                                                                       : 0x7FFFFFFF);
+        const unsigned grid = (unsigned)std::min<int64_t>((alen / V + kThreads) / kThreads, ch::kMaxBlocks);
         // 32 bits hold an index and the grid's stride past it (up to alen + kThreads V).
         if (2 * alen + 2 * kThreads * V <= (int64_t)UINT32_MAX)
             add_row_bias_flat<T, uint32_t><<<grid, kThreads, 0, ch::stream()>>>(a, bias, out, (uint32_t)alen, cols);

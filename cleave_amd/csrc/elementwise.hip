@@ -57,12 +57,12 @@ struct Vec16 {
 };
 
 // One 16-byte vector per thread over a grid that covers the whole array (a
-// grid-stride loop only past 2^31 blocks), with non-temporal loads, and stores
+// grid-stride loop only past the most workgroups a launch takes), with non-temporal loads, and stores
 // past kCachedBytes: streamed data is not kept in L2, which lifts a read+write
 // stream from ~5.5 to ~6.4 TB/s on MI355X.
 unsigned grid_for(int64_t nvec) {
     int64_t want = (nvec + kThreads - 1) / kThreads;
-    if (want > 0x7FFFFFFF) want = 0x7FFFFFFF;
+    if (want > ch::kMaxBlocks) want = ch::kMaxBlocks;
     return (unsigned)(want < 1 ? 1 : want);
 }
 

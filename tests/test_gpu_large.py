@@ -5,7 +5,7 @@ integers; the fast GEMM kernels address a tile with 32-bit per-lane offsets
 from a 64-bit per-tile base, so an operand spanning 4 GiB or more stays on
 them.  Each case checks sampled entries against the oracle (or exact closed
 forms) without copying the arrays back whole.
-One MI355X holds 288 GB; the largest case here allocates 24 GiB.
+One MI355X holds 288 GB; the largest case here allocates 64 GiB.
 """
 from __future__ import annotations
 
@@ -137,6 +137,43 @@ def test_escape_counts_past_2pow31_pixels(hip, oracle):
         ref = oracle.mandelbrot(w, h, x0, y0, np.float32(dx), np.float32(dy), it, rows=(r, r + 1))[r]
         assert np.array_equal(got, ref), r
 
+
+
+# One 16-byte vector a thread would take 2^24 workgroups of 256, which the runtime
+# refuses, or a few more, of which it runs only the few (in place: 64 GiB).
+@pytest.mark.parametrize("dtype,vectors", [("f32", 1 << 32), ("f64", 1 << 32), ("f64", (1 << 32) + 5000)])
+def test_row_bias_and_maps_past_the_grid_limit(hip, dtype, vectors):
+    np_t, per = (np.float32, 4) if dtype == "f32" else (np.float64, 2)
+    cols = 1001  # rows that are not whole vectors
+    rows = vectors * per // cols
+    print(f"row bias of {rows} x {cols} {dtype}", flush=True)
+    t = hip.empty((rows, cols), dtype)
+    n = rows * cols
+    for at in range(0, n, 1 << 31):
+        hip.zero(t.view((n,)).sub(at, (min(1 << 31, n - at),)))
+    pick = [0, 1, rows // 2, rows - 6, rows - 2, rows - 1]
+    rng = np.random.default_rng(3)
+    want = {r: rng.standard_normal(cols).astype(np_t) for r in pick}
+    for r in pick:
+        t.sub(r * cols, (cols,)).upload(want[r])
+    b = rng.standard_normal(cols).astype(np_t)
+    hip.add_row_bias(t, hip.from_numpy(b), out=t)
+    for r in pick:
+        assert np.array_equal(t.sub(r * cols, (cols,)).numpy(), want[r] + b), r
+    hip.neg(t, out=t)
+    for r in pick:
+        assert np.array_equal(t.sub(r * cols, (cols,)).numpy(), -(want[r] + b)), r
+    hip.zero(t)
+    assert not t.sub((rows - 1) * cols, (cols,)).numpy().any()
+
+
+def test_row_bias_of_more_narrow_rows_than_a_grid_holds(hip):
+    rows, cols = 8 * ((1 << 24) + 5) + 3, 4  # a workgroup per eight rows
+    t = hip.zero((rows, cols))
+    b = np.array([1, -2, 3, 0.5], np.float32)
+    hip.add_row_bias(t, hip.from_numpy(b), out=t)
+    for r in (0, 41, rows // 2, rows - 1):
+        assert np.array_equal(t.sub(r * cols, (cols,)).numpy(), b), r
 
 
 # f64 products with more of their narrow tiles (32 x 16) than a launch holds, along
