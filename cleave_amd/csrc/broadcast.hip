@@ -12,6 +12,7 @@
 // alone fixes, so results are deterministic for a given shape.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "common.hpp"
 #include "last_block.hpp"
@@ -23,8 +24,17 @@ constexpr int kRowUnroll = 4;
 
 // Past the 256 MiB MALL a matrix read once streams with non-temporal loads, and one
 // written streams out; a smaller one is often still there from the kernel that wrote
-// it, and is left there for the one that reads it.
-constexpr int64_t kStreamBytes = 256LL << 20;
+// it, and is left there for the one that reads it.  Maps of up to kResidentBytes of
+// result read through the caches too, as the same-shape maps do (elementwise.hip).
+constexpr int64_t kStreamBytes = 256LL << 20, kResidentBytes = 72LL << 20;
+enum class Reuse { kBoth, kResult, kNone };
+// go(std::integral_constant<Reuse, ...>) for a result of `bytes`.
+template <class Go>
+void by_reuse(int64_t bytes, Go go) {
+    if (bytes <= kResidentBytes) go(std::integral_constant<Reuse, Reuse::kBoth>{});
+    else if (bytes <= kStreamBytes) go(std::integral_constant<Reuse, Reuse::kResult>{});
+    else go(std::integral_constant<Reuse, Reuse::kNone>{});
+}
 
 // A 16-byte column chunk: 4 floats or 2 doubles.
 template <class T>
@@ -36,9 +46,14 @@ template <class T>
 __device__ __forceinline__ typename Chunk<T>::type ldnt(const T* p) {
     return __builtin_nontemporal_load(reinterpret_cast<const typename Chunk<T>::type*>(p));
 }
-template <class T, bool NT>
+template <class T, Reuse R>
+__device__ __forceinline__ typename Chunk<T>::type ld(const T* p) {
+    if constexpr (R == Reuse::kBoth) return *reinterpret_cast<const typename Chunk<T>::type*>(p);
+    else return ldnt(p);
+}
+template <class T, Reuse R>
 __device__ __forceinline__ void st(T* p, typename Chunk<T>::type v) {
-    if constexpr (NT) __builtin_nontemporal_store(v, reinterpret_cast<typename Chunk<T>::type*>(p));
+    if constexpr (R == Reuse::kNone) __builtin_nontemporal_store(v, reinterpret_cast<typename Chunk<T>::type*>(p));
     else *reinterpret_cast<typename Chunk<T>::type*>(p) = v;
 }
 
@@ -63,7 +78,7 @@ Tiling tiling_rows(int64_t rows, int64_t cols, int64_t rows_per_group, int per_c
 // one-shot map) keep the most bytes in flight: 8 rows per block measured
 // 6.6 TB/s at 65536 x 4096 against 4.8 TB/s for 128.
 Tiling tiling_bias(int64_t rows, int64_t cols, int per_chunk) { return tiling_rows(rows, cols, 8, per_chunk); }
-template <class T, bool NT>
+template <class T, Reuse R>
 __global__ __launch_bounds__(kThreads) void add_row_bias_kernel(const T* __restrict__ a, const T* __restrict__ bias,
                                                                 T* __restrict__ out, int64_t rows, int64_t cols,
                                                                 int64_t nseg, int64_t rpg) {
@@ -78,11 +93,11 @@ __global__ __launch_bounds__(kThreads) void add_row_bias_kernel(const T* __restr
     for (; r + kRowUnroll <= r1; r += kRowUnroll) {
         V v[kRowUnroll];
 #pragma unroll
-        for (int u = 0; u < kRowUnroll; ++u) v[u] = ldnt(a + (r + u) * cols + c);
+        for (int u = 0; u < kRowUnroll; ++u) v[u] = ld<T, R>(a + (r + u) * cols + c);
 #pragma unroll
-        for (int u = 0; u < kRowUnroll; ++u) st<T, NT>(out + (r + u) * cols + c, v[u] + b);
+        for (int u = 0; u < kRowUnroll; ++u) st<T, R>(out + (r + u) * cols + c, v[u] + b);
     }
-    for (; r < r1; ++r) st<T, NT>(out + r * cols + c, ldnt(a + r * cols + c) + b);
+    for (; r < r1; ++r) st<T, R>(out + r * cols + c, ld<T, R>(a + r * cols + c) + b);
 }
 
 // Column sums, out[j] = sum_i g[i][j], in one launch for any width.
@@ -199,7 +214,7 @@ __global__ __launch_bounds__(kThreads) void col_sums_kernel(const U* __restrict_
 // on.  One division a chunk, in 32 bits up to about 2^31 elements, where a thread an element
 // took a 64-bit one each (a layer's bias, tanh, its backward and column sums over 20000
 // x 1001 f32: 137 us, now 115, of which the cached stores give about 12).
-template <class T, class I>
+template <class T, class I, Reuse R>
 __global__ __launch_bounds__(kThreads) void add_row_bias_flat(const T* __restrict__ a, const T* __restrict__ bias,
                                                               T* __restrict__ out, I n, uint32_t cols) {
     constexpr int V = Chunk<T>::kN;
@@ -207,13 +222,13 @@ __global__ __launch_bounds__(kThreads) void add_row_bias_flat(const T* __restric
     for (I i = ((I)blockIdx.x * kThreads + threadIdx.x) * V; i < n; i += (I)gridDim.x * kThreads * V) {
         uint32_t c = (uint32_t)(i % cols);
         if (n - i >= V) {
-            vec v = ldnt(a + i);
+            vec v = ld<T, R>(a + i);
 #pragma unroll
             for (int e = 0; e < V; ++e) {
                 v[e] = v[e] + bias[c];
                 if (++c == cols) c = 0;
             }
-            st<T, false>(out + i, v);
+            st<T, R>(out + i, v);
         } else {
             for (I e = i; e < n; ++e) {
                 out[e] = a[e] + bias[c];
@@ -253,21 +268,24 @@ int32_t run_add_row_bias(const char* fn, const T* a, int64_t alen, const T* bias
     CH_DEVICE(fn, bias, blen * sizeof(T));
     CH_DEVICE(fn, out, outlen * sizeof(T));
     const Tiling t = tiling_bias(rows, cols, V);
+    const int64_t bytes = alen * (int64_t)sizeof(T);
     if (cols % V == 0 && aligned16(a) && aligned16(bias) && aligned16(out) && t.nseg * t.groups <= ch::kMaxBlocks) {
         const unsigned grid = (unsigned)(t.nseg * t.groups);
-        if (alen * (int64_t)sizeof(T) > kStreamBytes)
-            add_row_bias_kernel<T, true><<<grid, kThreads, 0, ch::stream()>>>(a, bias, out, rows, cols, t.nseg,
-                                                                             t.rows_per_group);
-        else
-            add_row_bias_kernel<T, false><<<grid, kThreads, 0, ch::stream()>>>(a, bias, out, rows, cols, t.nseg,
-                                                                              t.rows_per_group);
+        by_reuse(bytes, [&](auto r) {
+            add_row_bias_kernel<T, r.value><<<grid, kThreads, 0, ch::stream()>>>(a, bias, out, rows, cols, t.nseg,
+                                                                                t.rows_per_group);
+        });
     } else if (aligned16(a) && aligned16(out)) {
         const unsigned grid = (unsigned)std::min<int64_t>((alen / V + kThreads) / kThreads, ch::kMaxBlocks);
-        // 32 bits hold an index and the grid's stride past it (up to alen + kThreads V).
-        if (2 * alen + 2 * kThreads * V <= (int64_t)UINT32_MAX)
-            add_row_bias_flat<T, uint32_t><<<grid, kThreads, 0, ch::stream()>>>(a, bias, out, (uint32_t)alen, cols);
-        else
-            add_row_bias_flat<T, uint64_t><<<grid, kThreads, 0, ch::stream()>>>(a, bias, out, (uint64_t)alen, cols);
+        by_reuse(bytes, [&](auto r) {
+            // 32 bits hold an index and the grid's stride past it (up to alen + kThreads V).
+            if (2 * alen + 2 * kThreads * V <= (int64_t)UINT32_MAX)
+                add_row_bias_flat<T, uint32_t, r.value><<<grid, kThreads, 0, ch::stream()>>>(a, bias, out,
+                                                                                            (uint32_t)alen, cols);
+            else
+                add_row_bias_flat<T, uint64_t, r.value><<<grid, kThreads, 0, ch::stream()>>>(a, bias, out,
+                                                                                            (uint64_t)alen, cols);
+        });
     } else {
         add_row_bias_scalar<T><<<blocks_for(alen), kThreads, 0, ch::stream()>>>(a, bias, out, rows, cols);
     }
@@ -376,7 +394,7 @@ __device__ __forceinline__ void bcast_row_offsets(const BDims& d, I row, I& oa, 
 // the row and the output stream through non-temporal loads and stores, as in
 // the same-shape maps.  Requires the VEC conditions.
 constexpr int kRowChunks = 64;
-template <class Op, class T, class I, bool NT>
+template <class Op, class T, class I, Reuse R>
 __global__ __launch_bounds__(kThreads) void bcast_rows_kernel(const T* __restrict__ a, const T* __restrict__ b,
                                                               T* __restrict__ out, BDims d, I rows, I chunks) {
     constexpr int V = Chunk<T>::kN;
@@ -399,8 +417,8 @@ __global__ __launch_bounds__(kThreads) void bcast_rows_kernel(const T* __restric
                 const I c = c0 + u * kThreads;
                 va[u] = sa, vb[u] = sb;
                 if (c < chunks) {
-                    if (ia) va[u] = ldnt(pa + c * V);
-                    if (ib) vb[u] = ldnt(pb + c * V);
+                    if (ia) va[u] = ld<T, R>(pa + c * V);
+                    if (ib) vb[u] = ld<T, R>(pb + c * V);
                 }
             }
 #pragma unroll
@@ -410,7 +428,7 @@ __global__ __launch_bounds__(kThreads) void bcast_rows_kernel(const T* __restric
                     vec r;
 #pragma unroll
                     for (int t = 0; t < V; ++t) r[t] = op(va[u][t], vb[u][t]);
-                    st<T, NT>(o + c * V, r);
+                    st<T, R>(o + c * V, r);
                 }
             }
         }
@@ -559,14 +577,14 @@ int32_t run_bcast(const char* fn, const T* a, int64_t alen, const int32_t* ash, 
     const bool narrow = outlen < (int64_t)1 << 31 && alen < (int64_t)1 << 31 && blen < (int64_t)1 << 31;
     if (vec && chunks >= kRowChunks) {
         const unsigned grid = (unsigned)(rows < 65536 * 8 ? rows : 65536 * 8);
-        if (outlen * (int64_t)sizeof(T) <= kStreamBytes && narrow)
-            bcast_rows_kernel<Op, T, uint32_t, false><<<grid, kThreads, 0, ch::stream()>>>(a, b, out, d, (uint32_t)rows,
-                                                                                          (uint32_t)chunks);
-        else if (narrow)
-            bcast_rows_kernel<Op, T, uint32_t, true><<<grid, kThreads, 0, ch::stream()>>>(a, b, out, d, (uint32_t)rows,
-                                                                                         (uint32_t)chunks);
-        else
-            bcast_rows_kernel<Op, T, int64_t, true><<<grid, kThreads, 0, ch::stream()>>>(a, b, out, d, rows, chunks);
+        by_reuse(outlen * (int64_t)sizeof(T), [&](auto r) {
+            if (narrow)
+                bcast_rows_kernel<Op, T, uint32_t, r.value><<<grid, kThreads, 0, ch::stream()>>>(
+                    a, b, out, d, (uint32_t)rows, (uint32_t)chunks);
+            else
+                bcast_rows_kernel<Op, T, int64_t, Reuse::kNone><<<grid, kThreads, 0, ch::stream()>>>(a, b, out, d, rows,
+                                                                                                   chunks);
+        });
         CH_LAUNCHED(fn);
         return CLEAVE_HIP_OK;
     }

@@ -7,6 +7,8 @@
 // The library is compiled with -ffp-contract=off, so every op below rounds
 // exactly where the reference's scalar loop does (add/sub/mul/div/neg/relu
 // are bit-exact; exp/tanh come from the device math library).
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace {
@@ -57,47 +59,62 @@ struct Vec16 {
 };
 
 // One 16-byte vector per thread over a grid that covers the whole array (a
-// grid-stride loop only past the most workgroups a launch takes), with non-temporal loads, and stores
-// past kCachedBytes: streamed data is not kept in L2, which lifts a read+write
-// stream from ~5.5 to ~6.4 TB/s on MI355X.
+// grid-stride loop only past the most workgroups a launch takes).
 unsigned grid_for(int64_t nvec) {
     int64_t want = (nvec + kThreads - 1) / kThreads;
     if (want > ch::kMaxBlocks) want = ch::kMaxBlocks;
     return (unsigned)(want < 1 ? 1 : want);
 }
 
-template <class T>
+// How a map meets the caches, by the bytes of its result.  us for a map of f32 repeated
+// on its buffers | over buffers not touched lately | bias, tanh, its backward and column
+// sums over n x 1024 (a map's result is the next one's input):
+//                        neg 24 MiB | 64 MiB        add 24 | 64   bias.. 24 | 64 | 128 MiB
+//   streamed both ways    7.1 | 10.1   20.1 | 22.9   10.5 | 30.0     49 | 101 | 183
+//   loads streamed        8.9 | 10.5   22.7 | 23.8   12.8 | 31.5     42 |  92 | 165
+//   through the caches    8.2 | 11.2   19.5 | 24.4   11.9 | 27.7     39 |  90 | 196
+//   ... stores streamed   4.8 | 10.5   19.8 | 23.3   11.5 | 28.0     45 |  97 | 186
+// Up to kResidentBytes loads go through the caches, which may hold the operand from the
+// kernel that wrote it or an earlier pass, and two-operand maps store through them too;
+// one-operand maps stream their result past the operand (the chain 40 and 90 us so).  Up
+// to the MALL's 256 MiB only results stay, for the map that follows; past it nothing does
+// (2^28 f32 sigmoid 327 us streamed, results kept 346).  What streaming both ways would
+// still win: neg of 32-40 MiB 9%, of 80-96 MiB 5-9%, add of 16-24 MiB 11-20%, buffers not
+// touched lately up to 5%, against 10-20% of the chain at all these sizes.
+enum class Reuse { kBoth, kResult, kNone };
+constexpr int64_t kResidentBytes = 72LL << 20, kResultBytes = 256LL << 20;
+
+template <class T, Reuse R>
 __device__ __forceinline__ typename Vec16<T>::type ldv(const T* p) {
-    return __builtin_nontemporal_load(reinterpret_cast<const typename Vec16<T>::type*>(p));
+    const typename Vec16<T>::type* q = reinterpret_cast<const typename Vec16<T>::type*>(p);
+    if constexpr (R == Reuse::kBoth) return *q;
+    else return __builtin_nontemporal_load(q);
 }
-// Results of up to the MALL's 256 MiB are stored through the caches, as the map
-// that follows reads them there: bias, tanh, its backward and column sums over
-// n x 1024 f32 take 52.8 us instead of 60.4 at 32 MiB, 91 instead of 100 at 64,
-// 165 instead of 183 at 128, and with streaming stores between 20 and 48 MiB
-// 57.1 at 32.  A map whose result nobody reads next pays 4-6% (32 MiB 13.5 us
-// against 12.8), and one repeated on the same buffers up to a third around the
-// L2s' 32 MiB (24 MiB 9.7 against 7.1, 64 MiB 22.7 against 20.1, 192 MiB 58.7
-// against 60.7).  Larger ones stream past them (2^28 f32 sigmoid 327 us, through
-// the caches 346).
-constexpr int64_t kCachedBytes = 256LL << 20;
-template <class T, bool NT>
+template <class T, bool STREAM>
 __device__ __forceinline__ void stv(T* p, typename Vec16<T>::type v) {
-    if constexpr (NT) __builtin_nontemporal_store(v, reinterpret_cast<typename Vec16<T>::type*>(p));
+    if constexpr (STREAM) __builtin_nontemporal_store(v, reinterpret_cast<typename Vec16<T>::type*>(p));
     else *reinterpret_cast<typename Vec16<T>::type*>(p) = v;
 }
+// go(std::integral_constant<Reuse, ...>) for a result of `bytes`.
+template <class Go>
+void by_reuse(int64_t bytes, Go go) {
+    if (bytes <= kResidentBytes) go(std::integral_constant<Reuse, Reuse::kBoth>{});
+    else if (bytes <= kResultBytes) go(std::integral_constant<Reuse, Reuse::kResult>{});
+    else go(std::integral_constant<Reuse, Reuse::kNone>{});
+}
 
-template <class Op, class T, bool NT>
+template <class Op, class T, Reuse R>
 __global__ __launch_bounds__(kThreads) void map1_kernel(const T* __restrict__ a, T* __restrict__ out, int64_t n) {
     constexpr int V = Vec16<T>::kN;
     Op op;
     const int64_t nv = n / V;
     const int64_t step = (int64_t)gridDim.x * kThreads;
     for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < nv; i += step) {
-        const typename Vec16<T>::type x = ldv(a + V * i);
+        const typename Vec16<T>::type x = ldv<T, R>(a + V * i);
         typename Vec16<T>::type y;
 #pragma unroll
         for (int e = 0; e < V; ++e) y[e] = op(x[e]);
-        stv<T, NT>(out + V * i, y);
+        stv<T, R != Reuse::kResult>(out + V * i, y);
     }
     if (blockIdx.x == 0 && threadIdx.x < (n % V)) {
         int64_t i = nv * V + threadIdx.x;
@@ -105,7 +122,7 @@ __global__ __launch_bounds__(kThreads) void map1_kernel(const T* __restrict__ a,
     }
 }
 
-template <class Op, class T, bool NT>
+template <class Op, class T, Reuse R>
 __global__ __launch_bounds__(kThreads) void map2_kernel(const T* __restrict__ a, const T* __restrict__ b,
                                                         T* __restrict__ out, int64_t n) {
     constexpr int V = Vec16<T>::kN;
@@ -113,11 +130,11 @@ __global__ __launch_bounds__(kThreads) void map2_kernel(const T* __restrict__ a,
     const int64_t nv = n / V;
     const int64_t step = (int64_t)gridDim.x * kThreads;
     for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < nv; i += step) {
-        const typename Vec16<T>::type x = ldv(a + V * i), y = ldv(b + V * i);
+        const typename Vec16<T>::type x = ldv<T, R>(a + V * i), y = ldv<T, R>(b + V * i);
         typename Vec16<T>::type z;
 #pragma unroll
         for (int e = 0; e < V; ++e) z[e] = op(x[e], y[e]);
-        stv<T, NT>(out + V * i, z);
+        stv<T, R == Reuse::kNone>(out + V * i, z);
     }
     if (blockIdx.x == 0 && threadIdx.x < (n % V)) {
         int64_t i = nv * V + threadIdx.x;
@@ -153,10 +170,10 @@ int32_t run1(const char* name, const T* a, int64_t alen, T* out, int64_t outlen)
     CH_DEVICE(name, out, outlen * sizeof(T));
     if (!aligned16(a) || !aligned16(out))
         map1_scalar_kernel<Op, T><<<grid_for(alen / V + 1), kThreads, 0, ch::stream()>>>(a, out, alen);
-    else if (alen * (int64_t)sizeof(T) > kCachedBytes)
-        map1_kernel<Op, T, true><<<grid_for(alen / V), kThreads, 0, ch::stream()>>>(a, out, alen);
     else
-        map1_kernel<Op, T, false><<<grid_for(alen / V), kThreads, 0, ch::stream()>>>(a, out, alen);
+        by_reuse(alen * (int64_t)sizeof(T), [&](auto r) {
+            map1_kernel<Op, T, r.value><<<grid_for(alen / V), kThreads, 0, ch::stream()>>>(a, out, alen);
+        });
     CH_LAUNCHED(name);
     return CLEAVE_HIP_OK;
 }
@@ -175,10 +192,10 @@ int32_t run2(const char* name, const T* a, int64_t alen, const T* b, int64_t ble
     CH_DEVICE(name, out, outlen * sizeof(T));
     if (!aligned16(a) || !aligned16(b) || !aligned16(out))
         map2_scalar_kernel<Op, T><<<grid_for(alen / V + 1), kThreads, 0, ch::stream()>>>(a, b, out, alen);
-    else if (alen * (int64_t)sizeof(T) > kCachedBytes)
-        map2_kernel<Op, T, true><<<grid_for(alen / V), kThreads, 0, ch::stream()>>>(a, b, out, alen);
     else
-        map2_kernel<Op, T, false><<<grid_for(alen / V), kThreads, 0, ch::stream()>>>(a, b, out, alen);
+        by_reuse(alen * (int64_t)sizeof(T), [&](auto r) {
+            map2_kernel<Op, T, r.value><<<grid_for(alen / V), kThreads, 0, ch::stream()>>>(a, b, out, alen);
+        });
     CH_LAUNCHED(name);
     return CLEAVE_HIP_OK;
 }

@@ -216,3 +216,27 @@ def test_add_row_bias_ragged_widths(hip, rows, cols, dtype):
     hip.add_row_bias(hip.from_numpy(A), hip.from_numpy(b), out=out.sub(0, (rows, cols)))
     got = out.numpy()
     assert np.array_equal(got[:rows * cols].reshape(rows, cols), A + b) and np.all(got[rows * cols:] == 7.0)
+
+
+# Each way that maps meet the caches, on both sides of its bounds: results of 72 MiB and of
+# 256 MiB, and a row more.
+@pytest.mark.parametrize("mib", [72, 256])
+@pytest.mark.parametrize("more", [0, 1])
+def test_maps_around_the_cache_bounds(hip, mib, more):
+    rows, cols = mib * 256 + more, 1024
+    rng = np.random.default_rng(mib + more)
+    A = rng.standard_normal(rows * cols).astype(np.float32)
+    b = rng.standard_normal(cols).astype(np.float32)
+    a, out = hip.from_numpy(A), hip.from_numpy(np.full(rows * cols, np.nan, np.float32))
+    assert np.array_equal(hip.neg(a, out=out).numpy(), -A)
+    assert np.array_equal(hip.sub(a, out, out=out).numpy(), A + A)
+    A2 = A.reshape(rows, cols)
+    a, out = a.view((rows, cols)), out.view((rows, cols))
+    assert np.array_equal(hip.add_row_bias(a, hip.from_numpy(b), out=out).numpy(), A2 + b)
+    assert np.array_equal(hip.mul(a, hip.from_numpy(b), out=out).numpy(), A2 * b)
+    # rows that are not whole vectors
+    n = rows * cols // 1001
+    b = rng.standard_normal(1001).astype(np.float32)
+    odd, to = (v.view((rows * cols,)).sub(0, (n, 1001)) for v in (a, out))
+    got = hip.add_row_bias(odd, hip.from_numpy(b), out=to).numpy()
+    assert np.array_equal(got, A[:n * 1001].reshape(n, 1001) + b)
