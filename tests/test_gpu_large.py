@@ -198,3 +198,21 @@ def test_f64_products_past_the_grid_limit(hip, wide):
     for i, at in enumerate(where):
         assert c.view((n,)).sub(at, (1,)).numpy()[0] == 5.0 * (i + 1.5), (wide, at)
     assert c.view((n,)).sub(1, (1,)).numpy()[0] == 0.0
+
+
+# Row bias of odd widths around the switch from 32-bit to 64-bit indexes: below 2^31
+# elements by the grid's stride past the end, and above it.
+@pytest.mark.parametrize("rows", [((1 << 31) - 2048) // 1001, ((1 << 31) - 2048) // 1001 + 1, (1 << 31) // 1001 + 9])
+def test_row_bias_around_the_index_switch(hip, rows):
+    cols = 1001
+    t = hip.zero((rows, cols))
+    rng = np.random.default_rng(rows)
+    pick = [0, 1, rows // 3, rows - 2, rows - 1]
+    want = {r: rng.standard_normal(cols).astype(np.float32) for r in pick}
+    for r in pick:
+        t.sub(r * cols, (cols,)).upload(want[r])
+    b = rng.standard_normal(cols).astype(np.float32)
+    hip.add_row_bias(t, hip.from_numpy(b), out=t)
+    for r in pick:
+        assert np.array_equal(t.sub(r * cols, (cols,)).numpy(), want[r] + b), r
+    assert np.array_equal(t.sub((rows - 3) * cols, (cols,)).numpy(), b)
