@@ -296,18 +296,24 @@ int32_t run_add_row_bias(const char* fn, const T* a, int64_t alen, const T* bias
 template <class T, class U>
 int32_t launch_col_sums(const char* fn, const T* g, T* out, int64_t rows, int64_t units) {
     const ColSums p = col_sums_plan(rows, units, sizeof(U) > sizeof(T));
+    const size_t row = sizeof(U) * (size_t)units;
+    // A result that lies inside g (over one of its rows, say) may be written while other
+    // segments still read there, unless its columns are g's: it is put aside until then.
+    const bool aside = ch::overlaps(g, row * (size_t)rows, out, row) && ((intptr_t)out - (intptr_t)g) % (intptr_t)row != 0;
     U* part = nullptr;
-    if (p.groups > 1) {
-        part = (U*)ch::scratch(5, sizeof(U) * (size_t)(p.groups * units));
+    if (p.groups > 1 || aside) {
+        part = (U*)ch::scratch(5, row * (size_t)(p.groups + aside));
         if (!part)
-            return ch::fail(CLEAVE_HIP_ERR_OOM, "%s: scratch of %lld elements", fn, (long long)(p.groups * units));
+            return ch::fail(CLEAVE_HIP_ERR_OOM, "%s: scratch of %lld elements", fn, (long long)((p.groups + aside) * units));
     }
+    U* to = aside ? part + p.groups * units : (U*)out;
     const unsigned grid = (unsigned)(p.nseg * p.groups);
     if (rows * units * (int64_t)sizeof(U) > kStreamBytes)
-        col_sums_kernel<U, Read::kStream><<<grid, kThreads, 0, ch::stream()>>>((const U*)g, part, (U*)out, rows, p);
+        col_sums_kernel<U, Read::kStream><<<grid, kThreads, 0, ch::stream()>>>((const U*)g, part, to, rows, p);
     else
-        col_sums_kernel<U, Read::kCached><<<grid, kThreads, 0, ch::stream()>>>((const U*)g, part, (U*)out, rows, p);
+        col_sums_kernel<U, Read::kCached><<<grid, kThreads, 0, ch::stream()>>>((const U*)g, part, to, rows, p);
     CH_LAUNCHED(fn);
+    if (aside) CH_HIP(hipMemcpyAsync(out, to, row, hipMemcpyDeviceToDevice, ch::stream()));
     return CLEAVE_HIP_OK;
 }
 

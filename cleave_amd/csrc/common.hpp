@@ -59,6 +59,12 @@ inline int64_t count3(int64_t a, int64_t b, int64_t c) {
     return ab > INT64_MAX / c ? -1 : ab * c;
 }
 
+// True when the bytes [a, a + na) and [b, b + nb) share any.
+inline bool overlaps(const void* a, size_t na, const void* b, size_t nb) {
+    const uintptr_t p = (uintptr_t)a, q = (uintptr_t)b;
+    return p < q + nb && q < p + na;
+}
+
 // Workspace of the allocation-free entry point (cleave_hip_reduce_sum_f32_noalloc):
 // a static device array of kNoAllocFloats floats, its device address resolved
 // once at init with the library's device current.  nullptr when that failed.

@@ -240,3 +240,20 @@ def test_maps_around_the_cache_bounds(hip, mib, more):
     odd, to = (v.view((rows * cols,)).sub(0, (n, 1001)) for v in (a, out))
     got = hip.add_row_bias(odd, hip.from_numpy(b), out=to).numpy()
     assert np.array_equal(got, A[:n * 1001].reshape(n, 1001) + b)
+
+
+# The result inside g: over one of its rows, and across two of them (several segments, with
+# one group of rows and with many), in whole vectors and in single elements.
+@pytest.mark.parametrize("rows", [9, 4099])
+@pytest.mark.parametrize("cols", [1000, 1001])
+@pytest.mark.parametrize("at", [0, 3000, 8, 1004, 4502])
+def test_sum_rows_into_its_operand(hip, rows, cols, at):
+    G = np.random.default_rng(rows + cols + at).integers(-8, 9, (rows, cols)).astype(np.float32)
+    g = hip.from_numpy(G)
+    flat = g.view((rows * cols,))
+    got = hip.sum_rows(g, out=flat.sub(at, (cols,))).numpy()
+    want = G.sum(axis=0)
+    assert np.array_equal(got, want)
+    kept = G.reshape(-1).copy()
+    kept[at:at + cols] = want
+    assert np.array_equal(flat.numpy(), kept)
