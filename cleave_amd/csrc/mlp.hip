@@ -598,6 +598,11 @@ int32_t fused_step(const float* x, const float* y, float* w1, float* w2, float* 
 // g = dL/dz and writes dW1 = X^T d1, dW2 = H^T g with d1 = (g w2^T) H(1-H).
 bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
+// The product that forms dW1 reads x: a dW1 that shares memory with x is formed aside.
+bool dw1_aside(const float* dw1, const float* x, int B, int D, int Hd) {
+    return dw1 && ch::overlaps(dw1, sizeof(float) * (size_t)D * Hd, x, sizeof(float) * (size_t)B * D);
+}
+
 bool layer_fwd_fits(const float* x, const float* w1, const float* h, int B, int D, int Hd) {
     return B % 256 == 0 && D % 256 == 0 && Hd % 256 == 0 && aligned16(x) && aligned16(w1) && aligned16(h) &&
            FusedTile1::fits(B, Hd, D, D, Hd);
@@ -661,15 +666,18 @@ int32_t hidden_bwd(const float* x, const float* h, const float* w2, const float*
         return CLEAVE_HIP_OK;
     }
     const int groups = partial_rows(B, Hd);
-    const size_t nH = (size_t)B * Hd, nPart = (size_t)groups * Hd;
-    float* d1 = (float*)ch::scratch(4, sizeof(float) * (up(nH) + up(nPart)));
+    const bool aside = dw1_aside(dw1, x, B, D, Hd);
+    const size_t nH = (size_t)B * Hd, nPart = (size_t)groups * Hd, nG = aside ? (size_t)D * Hd : 0;
+    float* d1 = (float*)ch::scratch(4, sizeof(float) * (up(nH) + up(nPart) + up(nG)));
     if (!d1) return CLEAVE_HIP_ERR_OOM;
     float* part = d1 + up(nH);
+    float* g1 = aside ? part + up(nPart) : dw1;
     int32_t rc = run_rows<Rows::kBwd>(const_cast<float*>(h), d1, w2, g, B, Hd, nullptr, part, nullptr, nullptr, st);
     if (rc != CLEAVE_HIP_OK) return rc;
     if (dw1) {
-        rc = ch::gemm_f32_device(x, d1, dw1, D, Hd, B, 1, 0);
+        rc = ch::gemm_f32_device(x, d1, g1, D, Hd, B, 1, 0);
         if (rc != CLEAVE_HIP_OK) return rc;
+        if (aside) CH_HIP(hipMemcpyAsync(dw1, g1, sizeof(float) * nG, hipMemcpyDeviceToDevice, st));
     }
     Finish f{};
     if (dw2) f.part2 = part, f.groups = groups, f.Hd = Hd, f.dw2 = dw2;
@@ -710,15 +718,17 @@ extern "C" int32_t cleave_hip_mlp_step_f32(const float* x, int64_t xlen, const f
 
     const bool wide = Hd > kRowsMaxHd;
     const int groups = partial_rows(B, Hd), errs = row_groups(B, Hd, !wide);
-    // Scratch slot 4: H/d1 | dW2 partials | squared errors | d2 of the wide passes | dW1 if not asked for.
-    const size_t nH = (size_t)B * Hd, nPart = (size_t)groups * Hd, nD2 = wide ? B : 0, nG = dw1 ? 0 : (size_t)D * Hd;
+    const bool aside = dw1_aside(dw1, x, B, D, Hd);
+    // Scratch slot 4: H/d1 | dW2 partials | squared errors | d2 of the wide passes | dW1 if not asked for, or aside.
+    const size_t nH = (size_t)B * Hd, nPart = (size_t)groups * Hd, nD2 = wide ? B : 0;
+    const size_t nG = dw1 && !aside ? 0 : (size_t)D * Hd;
     auto up = [](size_t n) { return (n + 63) & ~(size_t)63; };
     float* H = (float*)ch::scratch(4, sizeof(float) * (up(nH) + up(nPart) + up(errs) + up(nD2) + up(nG)));
     if (!H) return CLEAVE_HIP_ERR_OOM;
     float* part = H + up(nH);
     float* sq = part + up(nPart);
     float* d2 = sq + up(errs);
-    float* g1 = dw1 ? dw1 : d2 + up(nD2);
+    float* g1 = nG == 0 ? dw1 : d2 + up(nD2);
 
     int32_t rc = ch::gemm_f32_device(x, w1, H, B, Hd, D, 0, 0);
     if (rc != CLEAVE_HIP_OK) return rc;
@@ -733,6 +743,7 @@ extern "C" int32_t cleave_hip_mlp_step_f32(const float* x, int64_t xlen, const f
     f.sqpart = sq, f.errs = errs, f.loss = loss_dev, f.count = (float)B, f.lr = lr;
     mlp_finish_kernel<<<finish_grid(f), kThreads, 0, st>>>(f);
     CH_LAUNCHED("mlp_finish_kernel");
+    if (aside) CH_HIP(hipMemcpyAsync(dw1, g1, sizeof(float) * nG, hipMemcpyDeviceToDevice, st));
     return CLEAVE_HIP_OK;
 }
 

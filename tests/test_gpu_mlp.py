@@ -283,3 +283,32 @@ def _row_pass(hip, oracle, B, Hd):
             assert np.all(np.abs(a.numpy() - X.T @ d1) <= tol * (np.abs(X).T @ np.abs(d1)) + 1e-30)
         if which != "dw1":
             assert np.all(np.abs(b.numpy() - Hn.T @ G) <= tol * (Hn.T @ np.abs(G)) + 1e-30)
+
+
+# A gradient that takes the place of the batch it came from, whose rows it needs to the
+# last: the step off the fused shapes and the layer's rule.
+@pytest.mark.parametrize("B,D,Hd", [(400, 70, 130), (512, 128, 256), (5000, 16, 4100)])
+def test_dw1_over_the_batch(hip, B, D, Hd):
+    rng = np.random.default_rng(B + D + Hd)
+    n = max(B * D, D * Hd)
+    X = rng.standard_normal((B, D)).astype(np.float32)
+    y = hip.from_numpy((rng.random(B) < 0.5).astype(np.float32))
+    W1, W2 = _xavier(rng, D, Hd, (D, Hd)), _xavier(rng, Hd, 1, Hd)
+
+    def batch():  # x and dW1 over one buffer
+        buf = hip.empty((n,))
+        return buf.sub(0, (B, D)).upload(X), buf.sub(0, (D, Hd))
+
+    want, want1 = hip.empty((D, Hd)), hip.from_numpy(W1)
+    hip.mlp_step(hip.from_numpy(X), y, want1, hip.from_numpy(W2), 0.01, dw1=want)
+    (x, dw1), w1 = batch(), hip.from_numpy(W1)
+    hip.mlp_step(x, y, w1, hip.from_numpy(W2), 0.01, dw1=dw1)
+    assert np.array_equal(dw1.numpy(), want.numpy()) and np.array_equal(w1.numpy(), want1.numpy())
+
+    x, dw1 = batch()
+    w2 = hip.from_numpy(W2.reshape(Hd, 1))
+    h, _ = hip.sigmoid_hidden_fwd(x, hip.from_numpy(W1), w2)
+    g = hip.from_numpy(rng.standard_normal((B, 1)).astype(np.float32))
+    hip.sigmoid_hidden_bwd(hip.from_numpy(X), h, w2, g, want, None)
+    hip.sigmoid_hidden_bwd(x, h, w2, g, dw1, None)
+    assert np.array_equal(dw1.numpy(), want.numpy())
