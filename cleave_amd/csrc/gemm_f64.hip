@@ -38,6 +38,8 @@
 // product are read from its last row and feed only entries that are not
 // stored; k past K enters as zero on both sides.  Any M, N, K takes the same path (K = 0
 // included: C = 0, the zero-filled accumulator of matrix.cleave:59).
+#include <algorithm>
+
 #include "common.hpp"
 #include "gemm_common.hpp"
 #include "last_block.hpp"
@@ -137,8 +139,8 @@ struct Frags {
     }
 };
 
-// `part`: tiles x slices partial tiles, unused with slices == 1.  A grid of at least
-// tiles_m * tiles_n * batch * slices workgroups, in rows of at most ch::kMaxBlocks.
+// `part`: tiles x slices partial tiles, unused with slices == 1.  A 1-D grid of
+// tiles_m * tiles_n * batch * slices workgroups.
 // (Two waves a SIMD for two k-contiguous operands on 4 x 4 fragments, which the
 // compiler gives 268 registers otherwise.)
 template <bool KCA, bool KCB, bool V2A, bool V2B, int FM, int FN, int WK, int PF, int STEP>
@@ -152,10 +154,8 @@ __global__ __launch_bounds__(kThreads, KCA && KCB && FM * FN == 16 && PF < 3 ? 2
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t block = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
-    if (block >= (int64_t)tiles_m * tiles_n * batch * slices) return;
     int b, tm, tn;  // b: batch entry and slice
-    ch::block_coords((int)block, tiles_m, tiles_n, batch * slices, b, tm, tn);
+    ch::block_coords(blockIdx.x, tiles_m, tiles_n, batch * slices, b, tm, tn);
     const int entry = b / slices, z = b - entry * slices;
     A += (int64_t)entry * sa;
     B += (int64_t)entry * sb;
@@ -309,6 +309,7 @@ struct Args {
     const double *a, *b;
     double* c;
     int M, N, K, batch;
+    int64_t lda, ldb;  // row pitches of a and b as stored
 };
 
 int64_t tile_count(const Args& g, int tm, int tn) {
@@ -327,11 +328,9 @@ int32_t launch(const Args& g, int slices) {
         part = (double*)ch::scratch_try(11, sizeof(double) * (size_t)(tiles * slices * FM * FN * 256));
         if (!part) slices = 1, kslice = g.K;  // no room: K in one piece
     }
-    const int64_t blocks = tiles * slices, across = blocks < ch::kMaxBlocks ? blocks : ch::kMaxBlocks;
-    const dim3 grid((unsigned)across, (unsigned)((blocks + across - 1) / across));
-    gemm_f64_kernel<KCA, KCB, V2A, V2B, FM, FN, WK, PF, STEP><<<grid, kThreads, 0, ch::stream()>>>(
-        g.a, g.b, g.c, g.M, g.N, g.K, KCA ? g.K : g.M, KCB ? g.K : g.N, (int64_t)g.M * g.K, (int64_t)g.K * g.N,
-        (int64_t)g.M * g.N, (g.M + TM - 1) / TM, (g.N + TN - 1) / TN, g.batch, slices, kslice, part);
+    gemm_f64_kernel<KCA, KCB, V2A, V2B, FM, FN, WK, PF, STEP><<<(unsigned)(tiles * slices), kThreads, 0, ch::stream()>>>(
+        g.a, g.b, g.c, g.M, g.N, g.K, g.lda, g.ldb, (int64_t)g.M * g.K, (int64_t)g.K * g.N, (int64_t)g.M * g.N,
+        (g.M + TM - 1) / TM, (g.N + TN - 1) / TN, g.batch, slices, kslice, part);
     CH_LAUNCHED("gemm_f64_kernel");
     return CLEAVE_HIP_OK;
 }
@@ -339,11 +338,12 @@ int32_t launch(const Args& g, int slices) {
 // The wave tiles, and the time of a product on each as fitted to sweeps on
 // MI355X (48 shapes and layouts from 33 x 77 x 1000 to 4096^3, and 26 outputs
 // with K of 128 and 256; within 19% of the best of all measured):
-//   base + max(busiest CU's (MFMA time / eff + end), one wave's steps x (MFMA + lat) + end) + fold
+//   base + max(busiest CU's MFMA time / eff + ends, one wave's steps x (MFMA + lat)) + fold
 // A step, 16 of K here, is FM FN x 256 cycles of MFMA, 0.107 us a fragment pair.
 // lat is what a wave's load latency adds where nothing else runs on its SIMD;
-// end is a workgroup's add of the partial tiles in LDS, by one wave: without it
-// 20000 x 500 x 128 took 85 us on the 64 x 32 tiles, 62 on the 128 x 128 ones.
+// ends, where K is up to 256, is the add of the partial tiles in LDS, by one wave, of
+// each workgroup on a CU after the first: without it 20000 x 500 x 128 took 85 us on
+// the 64 x 32 tiles, 62 on the 128 x 128 ones.
 // eff_k applies where both operands are k-contiguous (A.B^T), whose 64-byte
 // row pieces use the L1 less well.  Past one slice, each partial tile is
 // written and read past the L2: about 3 TB/s for the two, and 3 us.
@@ -352,9 +352,9 @@ struct TileCost {
     double base, eff, eff_k, lat, end;  // us, share of the MFMA rate, us a step, us a tile
 };
 constexpr TileCost kTiles[] = {
-    {1, 1, 4, 3.3, 0.32, 0.27, 0.3, 0.2},
-    {2, 2, 4, 3.55, 0.65, 0.53, 0.6, 0.45},
-    {4, 2, 4, 5.0, 0.77, 0.70, 0.6, 0.8},
+    {1, 1, 4, 3.5, 0.32, 0.27, 0.3, 0.2},
+    {2, 2, 4, 4.0, 0.65, 0.53, 0.6, 0.4},
+    {4, 2, 4, 6.0, 0.77, 0.70, 0.6, 0.8},
     {4, 4, 1, 9.0, 0.86, 0.80, 0.6, 0.0},
 };
 constexpr int kSlices[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
@@ -373,16 +373,17 @@ Plan choose_tile(const Args& g, bool kca, bool kcb) {
         const int tm = 16 * t.fm * (t.wk == 1 ? 2 : 1), tn = 16 * t.fn * (t.wk == 1 ? 2 : 1);
         const int64_t tiles = tile_count(g, tm, tn);
         if ((!kca && g.M < t.fm) || (!kcb && g.N < t.fn)) continue;  // a lane's group of rows must exist
-        if (tiles > 0x7FFFFFFF) continue;  // the 128 x 128 tiles' count is checked by the caller
+        if (tiles > ch::kMaxBlocks) continue;  // run_matmul_f64 sees to it that some tile fits
         double last = 1e300;
         for (const int s : kSlices) {
             // slices of at least 128, at most 16 workgroups a CU, a counter per tile
             if (s > 1 && (t.wk == 1 || g.K / s < 128 || tiles * s > 16 * (int64_t)cus || tiles > kCounters)) break;
             const double steps = (double)((((int64_t)g.K + s - 1) / s + 16 * t.wk - 1) / (16 * t.wk));
             const double mfma = 0.107 * t.fm * t.fn;
-            const double busy =
-                (double)((tiles * s + cus - 1) / cus) * (steps * mfma / (both_k ? t.eff_k : t.eff) + t.end);
-            const double chain = steps * (mfma + t.lat) + t.end;
+            const double busiest = (double)((tiles * s + cus - 1) / cus);
+            const double ends = g.K <= 256 ? (busiest - 1) * t.end : 0.0;
+            const double busy = busiest * steps * mfma / (both_k ? t.eff_k : t.eff) + ends;
+            const double chain = steps * (mfma + t.lat);
             const double us = t.base + (busy > chain ? busy : chain) +
                               (s > 1 ? 3.0 + (double)(tiles * s) * tm * tn * 16.0 / 3e6 : 0.0);
             if (us < best_us) best_us = us, best.tile = i, best.slices = s;
@@ -422,16 +423,16 @@ int narrow_slices(const Args& g, int64_t tiles) {
 // 4096^2 x 64 53 there, 67 here.
 bool shallow(const Args& g, bool both_k) {
     const int64_t t64 = tile_count(g, 64, 64), t128 = tile_count(g, 128, 128);
-    if (g.K > 64 || 2 * t64 <= 5 * (int64_t)ch::num_cus() || t64 > 0x7FFFFFFF) return false;
+    if (g.K > 64 || 2 * t64 <= 5 * (int64_t)ch::num_cus() || t64 > ch::kMaxBlocks) return false;
     if (2.0 * 64 * 64 * t64 > 3.0 * g.M * g.N * g.batch || (g.K > 8 && g.N % 2)) return false;
     return !both_k || g.K <= 8 || t128 < ch::num_cus() || t64 < 3 * t128;
 }
 
 template <bool KCA, bool KCB, bool V2A, bool V2B>
 int32_t run_shape(const Args& g) {
-    if (g.N <= 16 && (KCA || g.M >= 2) && tile_count(g, 32, 16) <= 0x7FFFFFFF)
+    if (g.N <= 16 && (KCA || g.M >= 2))
         return launch<KCA, KCB, V2A, V2B, 2, 1, 4, 2, 16>(g, narrow_slices(g, tile_count(g, 32, 16)));
-    if (g.M <= 16 && (KCB || g.N >= 2) && tile_count(g, 16, 32) <= 0x7FFFFFFF)
+    if (g.M <= 16 && (KCB || g.N >= 2))
         return launch<KCA, KCB, V2A, V2B, 1, 2, 4, 2, 16>(g, narrow_slices(g, tile_count(g, 16, 32)));
     if ((KCA || g.M >= 2) && (KCB || g.N >= 2) && shallow(g, KCA && KCB))
         return launch<KCA, KCB, V2A, V2B, 2, 2, 1, 2, 8>(g, 1);
@@ -481,13 +482,35 @@ int32_t run_matmul_f64(const char* fn, const double* a, int64_t alen, const doub
         CH_DEVICE(fn, b, blen * 8);
     }
     CH_DEVICE(fn, c, clen * 8);
-    const Args g{a, b, c, M, N, K, batch};
-    CH_REQUIRE(tile_count(g, 128, 128) <= 0x7FFFFFFF, "%s: %lld workgroups exceed the grid limit", fn,
-               (long long)tile_count(g, 128, 128));
-    if (!trans_a && !trans_b) return run_layout<true, false>(g);
-    if (!trans_a) return run_layout<true, true>(g);
-    if (!trans_b) return run_layout<false, false>(g);
-    return run_layout<false, true>(g);
+    // What fits a launch on the smallest tiles (16 x 16): `entries` of the batch, or, of one
+    // narrow product (the others have larger tiles), a run of rows or of one row's columns.
+    Args g{a, b, c, M, N, K, batch, trans_a ? M : K, trans_b ? K : N};
+    auto run = [&]() {
+        if (!trans_a && !trans_b) return run_layout<true, false>(g);
+        if (!trans_a) return run_layout<true, true>(g);
+        if (!trans_b) return run_layout<false, false>(g);
+        return run_layout<false, true>(g);
+    };
+    if (tile_count(g, 16, 16) <= ch::kMaxBlocks) return run();
+    g.batch = 1;
+    const int64_t per = tile_count(g, 16, 16), entries = std::max<int64_t>(1, ch::kMaxBlocks / per);
+    const int64_t most = ch::kMaxBlocks * 16;
+    int64_t rows = M, cols = N;
+    if (per > ch::kMaxBlocks && N <= 16) rows = most;
+    else if (per > ch::kMaxBlocks && M <= 16) rows = 1, cols = most;
+    for (int64_t e = 0; e < batch; e += entries)
+        for (int64_t m = 0; m < M; m += rows)
+            for (int64_t n = 0; n < N; n += cols) {
+                g.batch = (int)std::min<int64_t>(entries, batch - e);
+                g.M = (int)std::min<int64_t>(rows, M - m);
+                g.N = (int)std::min<int64_t>(cols, N - n);
+                g.a = a + e * M * K + (trans_a ? m : m * K);
+                g.b = b + e * K * N + (trans_b ? n * K : n);
+                g.c = c + e * M * N + m * N + n;
+                const int32_t st = run();
+                if (st != CLEAVE_HIP_OK) return st;
+            }
+    return CLEAVE_HIP_OK;
 }
 
 }  // namespace
