@@ -645,23 +645,23 @@ int slice_depth(int K, int S) { return (int)(((int64_t)K + S - 1) / S + 15) / 16
 
 // One ragged product (an M or N off the 64 grid) with a long K as S K
 // slices on the 64 x 64 kernel's guarded-edge form, its batch running over
-// the slices, added in order (deterministic); each slice at least 512 deep
-// and whole 16-byte chunks (K % 4S == 0).  At most a round of tiles: the
-// most slices, up to kEdgeTilesPerCu tiles per CU over all of them (2048 x
-// 200 x 2000: 40.2 us in one launch of 128 tiles).  Up to kEdgeTilesPerCu
-// tiles per CU and K from 4096: the count (up to 16) that evens out the
-// tiles per CU, priced as the busiest CU's tiles times the slice depth
-// (kEdgeTileKUs) plus the slices written and read back at 5 TB/s, when that
-// saves 5%: 2500 x 640 x 16384 (400 tiles, 2 on most CUs) 8 slices, 535 ->
-// 437-446 us; 1500^2 x 16384 A^T.B 4, 792 -> 603; 1200 x 1100 x 12000 A.B^T
-// 5, 377 -> 278; 1536 x 1100 x 8192 4, 269 -> 239.  From K = 4096 the
-// slices run on 128 x 128 tiles instead (up to 4 per CU) where the same
-// pricing (kEdge128TileKUs) puts them 3% under the 64 x 64 choice, at
-// least three per CU: 1000^2 x 65536 16 slices, 1082 -> 988 us; 1000^2 x
-// 32768 A.B^T 532 -> 503; 1001 x 1003 x 32768 (aligned copies) 586 -> 554;
-// 2000^2 x 8192 4 slices (unsplit before) 530 -> 506.  It priced 700 x 900 x 30000
-// and 512 x 2000 x 20000 within 3% of their times on 128 x 128 tiles (373
-// and 372 us, against 335 and 330 on 64 x 64), which it therefore keeps.
+// the slices, added in order (deterministic).  S, up to 64 with K / S at least
+// 512 and 8 tiles per CU over all slices, is the cheapest by price: the busiest
+// CU's tiles times the slice depth (kEdgeTileKUs), 4 us for the launch of the
+// sum, and the slices written and read back at 5 TB/s.  Slices are whole
+// 16-deep k-tiles deep (slice_depth), the last one as deep as what is left.
+// With more than a round of tiles (up to kEdgeTilesPerCu per CU, K from 4096)
+// the price has to be 5% under one launch's: 2500 x 640 x 16384 (400 tiles, 2
+// on most CUs) 8 slices, 535 -> 437-446 us; 1500^2 x 16384 A^T.B 4, 792 ->
+// 603; 1200 x 1100 x 12000 A.B^T 5, 377 -> 278; 1536 x 1100 x 8192 4, 269 ->
+// 239.  From K = 4096 the slices run on 128 x 128 tiles instead (up to 4 per
+// CU) where the same pricing (kEdge128TileKUs) puts them 3% under the 64 x 64
+// choice, at least three per CU: 1000^2 x 65536 16 slices, 1082 -> 988 us;
+// 1000^2 x 32768 A.B^T 532 -> 503; 1001 x 1003 x 32768 (aligned copies) 586 ->
+// 554; 2000^2 x 8192 4 slices (unsplit before) 530 -> 506.  It priced 700 x 900
+// x 30000 and 512 x 2000 x 20000 within 3% of their times on 128 x 128 tiles
+// (373 and 372 us, against 335 and 330 on 64 x 64), which it therefore keeps.
+// A k-contiguous operand's K is whole 16-byte chunks (K % 4 == 0).
 // `padded`: the operands are aligned copies (ch::edge_chunks).  False when
 // not split.
 template <bool TA, bool TB>
