@@ -53,9 +53,11 @@ def test_config3_full_grid(hip, oracle):
 
 
 # Windows whose orbits settle on cycles of period 1, 2, 3 and many, around the
-# iteration counts at which the compared state is taken (16, 24, 36, ...), with
-# max_iter on both sides of a block of 8; and windows that hold NaN and infinity.
-@pytest.mark.parametrize("it", [0, 1, 7, 8, 15, 16, 17, 24, 31, 41, 1000, 3001])
+# iteration counts at which the compared state is taken (48, 72, then 112: the
+# first block's end past 108), with max_iter on both sides of each and of a block
+# of 8; and windows that hold NaN and infinity.
+@pytest.mark.parametrize("it", [0, 1, 7, 8, 15, 16, 17, 41, 47, 48, 49, 55, 56, 57, 71, 72, 73, 79, 80, 81, 104, 107,
+                                108, 111, 112, 113, 120, 1000, 3001])
 @pytest.mark.parametrize("x0,y0,span", [(-0.3, -0.2, 0.4), (-1.1, -0.1, 0.2), (-0.16, 0.70, 0.1),
                                         (-0.9, -0.05, 0.3), (-1.41, -0.01, 0.02), (-1e20, 0.0, 2e20)])
 def test_cycling_orbits_bit_exact(hip, oracle, x0, y0, span, it):

@@ -191,7 +191,10 @@ def test_sum_rows_edges(hip, rows, cols, dtype):
     assert np.array_equal(hip.sum_rows(flat.sub(1, (rows, cols))).numpy(), G.sum(axis=0))
 
 
-@pytest.mark.parametrize("cols", [2048 * 128, 2048 * 256])  # one group takes all rows: no fold
+# Wide rows, on both sides of the 2048 segments from which one group takes all rows and
+# nothing is folded: in whole vectors (64 a segment) and in single elements (128).
+@pytest.mark.parametrize("cols", [2048 * 128, 2047 * 256, 2047 * 256 + 4, 2048 * 256, 2047 * 128 - 1, 2047 * 128 + 1,
+                                  2048 * 128 + 1])
 def test_sum_rows_wide(hip, cols):
     G = np.random.default_rng(cols).integers(-8, 9, (300, cols)).astype(np.float32)
     assert np.array_equal(hip.sum_rows(hip.from_numpy(G)).numpy(), G.sum(axis=0))
