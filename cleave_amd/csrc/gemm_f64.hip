@@ -15,8 +15,9 @@
 // a (16 FM) x (16 FN) tile of C from register fragments that it loads from the
 // caches, STEP of K at a time (FM FN x 16 STEP cycles of MFMA a step), PF steps
 // ahead, and the other waves of its SIMD cover the rest of the loads' latency.
-// The register-staged LDS tiles of 128 x 128 that this replaced were slower at
-// every size: 4096^3 A.B 2206 -> 1906 us, A.B^T 2428 -> 2235, 4095^3 A.B^T (rows
+// The register-staged LDS tiles of 128 x 128 that this replaced were slower but
+// for A.B^T with K of 16 to 128 (43 of 4031 x 267 x 64 194 against 212 us, 4096^2 x
+// 64 53.5 against 53): 4096^3 A.B 2206 -> 1906 us, A.B^T 2428 -> 2235, 4095^3 A.B^T (rows
 // not 16-byte aligned) 3412 -> 2230, and with few tiles 1000^3 167 -> 40, 256^3
 // 45 -> 5, 64^2 x 10000 1586 -> 10, 8192 x 10 x 4096 660 -> 45.  The same LDS
 // scheme on 64 x 64 tiles took 69-73 us at 1000^3.
@@ -440,7 +441,13 @@ int32_t run_shape(const Args& g) {
     switch (p.tile) {
         case 0: return launch<KCA, KCB, V2A, V2B, 1, 1, 4, 4, 16>(g, p.slices);
         case 1: return launch<KCA, KCB, V2A, V2B, 2, 2, 4, 1, 16>(g, p.slices);
-        case 2: return launch<KCA, KCB, V2A, V2B, 4, 2, 4, 3, 8>(g, p.slices);
+        // Two k-contiguous operands whose rows are not 16-byte aligned load 8 bytes at a time,
+        // and do better a whole step of 16 ahead: 1001^3 41 us against 45.5, 3001^3 973 against
+        // 1164, 784 x 500 x 9999 177 against 211; aligned, 1000^3 40.5 against 41, 1200^3 108
+        // against 83, and A.B 1000^3 44 against 39.
+        case 2:
+            if constexpr (KCA && KCB && !(V2A && V2B)) return launch<KCA, KCB, V2A, V2B, 4, 2, 4, 1, 16>(g, p.slices);
+            else return launch<KCA, KCB, V2A, V2B, 4, 2, 4, 3, 8>(g, p.slices);
     }
     // A step ahead of 16 leaves the loads to the CU's other wave: 4096^3 A.B
     // 1906 us against 2190 with three of 8, 2000^3 274 against 268.
