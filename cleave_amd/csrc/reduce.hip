@@ -9,9 +9,10 @@
 // their order (last_block.hpp).  HBM-bound from a few MB; below that, latency.
 // The host-returning forms have the kernel write the result into pinned host
 // memory.  With a second launch for the fold and a copy of the result, a Mean of
-// 10^6 f32 took 26.7 us, now 17; Mean, Max and argmax of 10^7 together 96, now @TRIPLE@.
-// Queued sums of f32: 2^20 6.7 -> 4.9 us, 2^23 6.4 -> 6.1, 2^25 20.5 -> 20.4, 2^28 154 ->
-// 154-157; of u32, 2^25 21.6 -> 20.4.  max and argmax of 2^25 24.9 -> 23.4, 2^28 163 -> 160.
+// 10^6 f32 took 26.7 us, now 17; Mean, Max and argmax of 10^7 together 96, now 71.
+// Queued sums of f32: 2^20 6.9 -> 4.9 us, 2^23 6.8 -> 6.1, 2^25 20.7 -> 20.1, 2^28 154 ->
+// 151; of u32, 2^25 21.6 -> 20.2; of f64, 2^27 156 -> 152.  max and argmax of 2^23 10.5 ->
+// 9.1, 2^25 24.7 -> 24.0, 2^28 163 -> 154, unaligned 330 -> 174.
 //
 // Max semantics: the reference folds acc = v[0]; if v[i] > acc then acc = v[i]
 // (cmpf ogt, stdlib/num/num.cleave:303).  A NaN at i > 0 never wins; a NaN at
@@ -43,8 +44,12 @@ typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 //             151, eight 20.7 / 153; U = 4 with four 20.5 / 154; U = 2 with four 20.0 /
 //             152, slower to 2^24; a run of rows a workgroup, U = 8, four a CU 21.6 / 156.
 //             Unaligned, a row of single elements: U = 8, four a CU (2^25 f32 22 us; 40 so).
-//   Maximum   U = 8, up to four a CU: workgroup b of G takes the run [R b / G, R (b + 1) / G)
-//             of R rows, its elements in ascending order.
+//   Maximum   Grids and U alike, but workgroup b of G takes the run [R b / G, R (b + 1) / G)
+//             of R rows, its elements in ascending order.  2^18 / 2^23 / 2^25 / 2^28 f32
+//             6.9 / 9.1 / 24.0 / 154 us; U = 8 with four a CU 7.2 / 9.2 / 23.7 / 161, with two
+//             7.3 / 8.7 / 23.3 / 157, eight 7.3 / 11.1 / 24.7 / 161; U = 4 with four 6.9 / 9.1 /
+//             24.9 / 159; U = 16 with two 7.7 / 8.6 / 22.8 / 156.  Unaligned 6.9 / 10.2 / 24.8 /
+//             174; U = 4 with two 6.7 / 14.7 / 43 / 304, U = 16 with four 7.2 / 10.3 / 24.8 / 171.
 struct Rows {
     int64_t begin, end, step;
 };
@@ -54,14 +59,17 @@ __device__ __forceinline__ Rows my_rows(int64_t nvec) {
     if constexpr (RUN) return {rows * blockIdx.x / gridDim.x, rows * (blockIdx.x + 1) / gridDim.x, U};
     return {(int64_t)U * blockIdx.x, rows, (int64_t)U * gridDim.x};
 }
-constexpr int kSumUnroll = 4, kScalarUnroll = 8, kMaxUnroll = 8;
+constexpr int kVectorUnroll = 4, kScalarUnroll = 8;
 constexpr int kMinRows = 4;                                      // a workgroup
-constexpr int kSumPerCu = 2, kScalarPerCu = 4, kMaxPerCu = 4;  // workgroups
+constexpr int kVectorPerCu = 2, kScalarPerCu = 4;  // workgroups
 unsigned row_blocks(int64_t nvec, int per_cu) {
     const int64_t rows = (nvec + kThreads - 1) / kThreads, want = (rows + kMinRows - 1) / kMinRows;
     const int64_t most = ch::kTreeArity * ch::kTreeGroups;  // of the arrival tree
     const int64_t cap = std::min<int64_t>(per_cu * (int64_t)ch::num_cus(), most);
     return (unsigned)(want < 1 ? 1 : want < cap ? want : cap);
+}
+unsigned grid_for(int64_t len, int per_vector, bool aligned) {
+    return aligned ? row_blocks(len / per_vector, kVectorPerCu) : row_blocks(len, kScalarPerCu);
 }
 
 // ---- sum f32 / f64 ------------------------------------------------------------
@@ -145,8 +153,8 @@ __global__ __launch_bounds__(kThreads) void sum_kernel(const T* __restrict__ x, 
                                                        T* __restrict__ out, int aligned, int counter) {
     constexpr int V = Vec16<T>::kN;
     typedef typename Vec16<T>::type VT;
-    static_assert(kSumUnroll == 4, "the fold of the slots");
-    T chain[kSumUnroll][V], acc[V], lane;
+    static_assert(kVectorUnroll == 4, "the fold of the slots");
+    T chain[kVectorUnroll][V], acc[V], lane;
 #pragma unroll
     for (int e = 0; e < V; ++e) acc[e] = chain[0][e] = chain[1][e] = chain[2][e] = chain[3][e] = T(0);
     int trips = 0;
@@ -161,15 +169,15 @@ __global__ __launch_bounds__(kThreads) void sum_kernel(const T* __restrict__ x, 
         if (last_slot && ++trips % kChain == 0) fold_slots();
     };
     if (aligned) {
-        fold_rows<VT, kSumUnroll, false>(x, n / V, [&](VT v, int slot) {
+        fold_rows<VT, kVectorUnroll, false>(x, n / V, [&](VT v, int slot) {
 #pragma unroll
             for (int e = 0; e < V; ++e) chain[slot][e] += v[e];
-            next_trip(slot == kSumUnroll - 1);
+            next_trip(slot == kVectorUnroll - 1);
         });
         if (blockIdx.x == 0 && threadIdx.x < (n % V)) chain[0][0] += x[n / V * V + threadIdx.x];
     } else {
         fold_rows<T, kScalarUnroll, false>(x, n, [&](T v, int slot) {
-            chain[slot % kSumUnroll][0] += v;
+            chain[slot % kVectorUnroll][0] += v;
             next_trip(slot == kScalarUnroll - 1);
         });
     }
@@ -248,10 +256,10 @@ __global__ __launch_bounds__(kThreads) void max_kernel(const T* __restrict__ x, 
 #pragma unroll
     for (int e = 0; e < V; ++e) bv[e] = T(-INFINITY), bk[e] = kNone;
     Best<T> b{-INFINITY, INT64_MAX};
-    const int64_t first = my_rows<kMaxUnroll, true>(aligned ? n / V : n).begin * kThreads + threadIdx.x;
+    const int64_t first = my_rows<kVectorUnroll, true>(aligned ? n / V : n).begin * kThreads + threadIdx.x;
     auto index = [&](uint32_t k) { return first + (int64_t)k * kThreads; };  // of the vector
     if (aligned) {
-        fold_rows<VT, kMaxUnroll, true>(x, n / V, [&](VT v, int) {
+        fold_rows<VT, kVectorUnroll, true>(x, n / V, [&](VT v, int) {
 #pragma unroll
             for (int e = 0; e < V; ++e)
                 if (v[e] > bv[e]) bv[e] = v[e], bk[e] = met;
@@ -262,7 +270,7 @@ __global__ __launch_bounds__(kThreads) void max_kernel(const T* __restrict__ x, 
             if (bk[e] != kNone) take_better(b, bv[e], V * index(bk[e]) + e);
         if (blockIdx.x == 0 && threadIdx.x < (n % V)) take_better(b, x[n / V * V + threadIdx.x], n / V * V + threadIdx.x);
     } else {
-        fold_rows<T, kMaxUnroll, true>(x, n, [&](T v, int) {
+        fold_rows<T, kScalarUnroll, true>(x, n, [&](T v, int) {
             if (v > bv[0]) bv[0] = v, bk[0] = met;
             ++met;
         });
@@ -336,7 +344,7 @@ __global__ __launch_bounds__(kThreads) void sum_u32_kernel(const uint32_t* __res
     uint64_t acc = 0;
     if (aligned) {
         // Add in 64 bits (mod 2^64, exact for both forms).
-        fold_rows<u4, kSumUnroll, false>(x, n / 4, [&](u4 v, int) {
+        fold_rows<u4, kVectorUnroll, false>(x, n / 4, [&](u4 v, int) {
             acc += (widen<Signed>(v[0]) + widen<Signed>(v[1])) + (widen<Signed>(v[2]) + widen<Signed>(v[3]));
         });
         if (blockIdx.x == 0 && threadIdx.x < (n & 3)) acc += widen<Signed>(x[n / 4 * 4 + threadIdx.x]);
@@ -362,7 +370,7 @@ template <class T>
 int32_t queue_sum(const T* x, int64_t len, T* part, T* out, int counter) {
     constexpr int V = Vec16<T>::kN;
     const int aligned = aligned16(x);
-    const unsigned blocks = aligned ? row_blocks(len / V, kSumPerCu) : row_blocks(len, kScalarPerCu);
+    const unsigned blocks = grid_for(len, V, aligned);
     sum_kernel<T><<<blocks, kThreads, 0, ch::stream()>>>(x, len, part, out, aligned, counter);
     CH_LAUNCHED("sum_kernel");
     return CLEAVE_HIP_OK;
@@ -402,7 +410,7 @@ int32_t run_max(const char* fn, const T* x, int64_t len, T* out_max, int64_t* ou
     if (!host && out_max) CH_DEVICE(fn, out_max, sizeof(T));
     if (!host && out_argmax) CH_DEVICE(fn, out_argmax, 8);
     const int aligned = aligned16(x);
-    const unsigned blocks = row_blocks(aligned ? len / V : len, kMaxPerCu);
+    const unsigned blocks = grid_for(len, V, aligned);
     char* base = partials();
     if (!base) return CLEAVE_HIP_ERR_OOM;
     int64_t* pi = (int64_t*)base;
@@ -420,7 +428,7 @@ int32_t run_sum_u32(const char* fn, const uint32_t* x, int64_t len, uint64_t* ou
     CH_DEVICE(fn, x, len * 4);
     if (!host) CH_DEVICE(fn, out, 8);
     const int aligned = aligned16(x);
-    const unsigned blocks = aligned ? row_blocks(len / 4, kSumPerCu) : row_blocks(len, kScalarPerCu);
+    const unsigned blocks = grid_for(len, 4, aligned);
     uint64_t* part = (uint64_t*)partials();
     if (!part) return CLEAVE_HIP_ERR_OOM;
     sum_u32_kernel<Signed><<<blocks, kThreads, 0, ch::stream()>>>(x, len, part, out, aligned);
