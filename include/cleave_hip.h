@@ -278,7 +278,9 @@ CLEAVE_HIP_API int32_t cleave_hip_reduce_sum_i32_i64(const int32_t* x, int64_t l
  * one per workgroup; a call needing more is CLEAVE_HIP_ERR_ARG) whose
  * address the library's init resolves, so call cleave_hip_init() first if
  * the first call must not initialise.  Every call on a device shares that
- * workspace: calls that overlap on one device race. */
+ * workspace, and a count of arrived workgroups that each call leaves at zero:
+ * calls that overlapped on one device would spoil each other and every later
+ * one.  Through this header they cannot, as all run on the library's one stream. */
 CLEAVE_HIP_API int32_t cleave_hip_reduce_sum_f32_noalloc(const float* x, int64_t len, float* out_dev);
 /* Host-returning forms, like the stdlib functions (synchronise). */
 CLEAVE_HIP_API float cleave_hip_sum_f32(const float* x, int64_t len);
